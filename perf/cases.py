@@ -221,6 +221,16 @@ def _subspace_matrix(case, seed):
     return a + a.conj().T + np.diag(d)
 
 
+def _probe(m):
+    rng = np.random.Generator(np.random.PCG64(m))
+    return rng.standard_normal(m) + 1j * rng.standard_normal(m)
+
+
+def _fix_phase(z, probe):
+    """Rows of z, each times the phase that makes its product with probe real and positive."""
+    return z * torch.sgn(z @ probe).conj()[:, None]
+
+
 def _density(case, seed):
     """A positive, smooth random density of about 0.03 electrons per cubic bohr on a cell with
     0.255 bohr between grid points, as the Al cell has."""
@@ -244,7 +254,8 @@ def prepare(case, seed):
         m, nev = case["m"], case["nev"]
         a = torch.from_numpy(np.ascontiguousarray(_subspace_matrix(case, seed).T)).cuda()
         return {"kind": kind, "ctx": ctx, "m": m, "nev": nev, "a": a, "w": torch.empty(nev, dtype=torch.float64, device="cuda"),
-                "z": torch.empty((nev, m), dtype=torch.complex128, device="cuda"), "stream": _stream().cuda_stream}
+                "z": torch.empty((nev, m), dtype=torch.complex128, device="cuda"),
+                "probe": torch.from_numpy(_probe(m)).cuda(), "stream": _stream()}
     if kind == "xc":
         cell = _xc_cell(case)
         grid = dzhip.ScfGrid(ctx, (case["nx"], case["ny"], case["nz"]), tables.reciprocal(cell), float(np.prod(np.diag(cell))))
@@ -289,8 +300,11 @@ def run(state):
         return state["y"]
     if kind == "heev":
         state["ctx"].heev_dev(state["a"].data_ptr(), state["m"], state["m"], state["nev"], state["w"].data_ptr(),
-                              state["z"].data_ptr(), state["m"], state["stream"])
-        return {"values": state["w"], "vectors": state["z"]}
+                              state["z"].data_ptr(), state["m"], state["stream"].cuda_stream)
+        # An eigenvector has no phase of its own: each is given a real positive overlap with a
+        # fixed vector, the convention that makes bands of different calls comparable.
+        with torch.cuda.stream(state["stream"]):
+            return {"values": state["w"], "vectors": _fix_phase(state["z"], state["probe"])}
     if kind == "xc":
         state["grid"].init_rho(state["rho"])
         return state["grid"].read(dzhip.GRID_VIN)
@@ -429,8 +443,9 @@ def _exact_xc(case, rho):
 def exact(case, seed):
     kind = case["kind"]
     if kind == "heev":
-        # An eigenvector has no phase of its own.
-        return {"values": np.linalg.eigvalsh(_subspace_matrix(case, seed))[:case["nev"]], "vectors": None}
+        w, z = np.linalg.eigh(_subspace_matrix(case, seed))
+        z = torch.from_numpy(np.ascontiguousarray(z[:, :case["nev"]].T))
+        return {"values": w[:case["nev"]], "vectors": _fix_phase(z, torch.from_numpy(_probe(case["m"])))}
     if kind == "xc":
         return _exact_xc(case, _density(case, seed))
     s = _system(case, seed)
