@@ -3,8 +3,9 @@
 // all on the device in a handful of launches.
 //
 //   1. Householder tridiagonalisation (zhetd2's reflectors, A = Q T Q^H with T real tridiagonal)
-//      in one grid-synchronised launch: the trailing matrix is distributed over the workgroups'
-//      LDS by columns and each reflector costs one grid barrier.  The enqueue-only entry points
+//      in one launch of co-resident workgroups: the trailing matrix is distributed over the
+//      wavefronts' registers by columns and each reflector costs one exchange of two vectors
+//      through memory.  The enqueue-only entry points
 //      launch it cooperatively; the solvers' Rayleigh-Ritz step launches it as an ordinary
 //      dispatch admitted by the device's tridiagonalisation gate (TrdAdmission), so that the
 //      grids of concurrent solves on different streams run side by side.
@@ -24,27 +25,25 @@ namespace dzhip {
 constexpr int kHeevMaxM = 1024;
 
 struct HeevWork {
-    DevBuf vh, tau, d, e, pbuf, nbuf, sync, z, zt, gram;
-    int err_offset = 0;  // int index of the error flag in sync
+    DevBuf vh, tau, d, e, pub, err, z, zt, gram;
     void release();
 };
 
 // Largest matrix of the allocation-free variant (its buffers live in a 6 MiB device array).
 constexpr int kHeevNoAllocMaxM = 256;
 
-// Share of the device's tridiagonalisation gate held by one eigensolver call.  A grid barrier
-// needs all of its workgroups resident at once.  Workgroups are dealt to the XCDs round robin, so
+// Share of the device's tridiagonalisation gate held by one eigensolver call.  Its exchange needs
+// all of the grid's workgroups resident at once.  Workgroups are dealt to the XCDs round robin, so
 // a grid of G groups needs at most ceil(G / XCDs) CUs on any XCD (one workgroup per CU at worst).
 // The gate admits grids only while their sum stays within the CUs of one XCD; every other kernel
 // the library launches runs to completion without waiting on another workgroup, so an admitted
 // grid's missing workgroups are placed as those retire.  That can take long: with many streams
-// issuing kernels, smaller workgroups keep refilling the CUs a tridiagonalisation workgroup (80-100
-// KB of LDS) waits for (one barrier ran out of its spin limit in a concurrent-k SCF of some
-// thousands of calls).  An admitted grid's barrier therefore gives up after 2^19 polls (an eighth
+// issuing kernels, smaller workgroups keep refilling the CUs a tridiagonalisation workgroup (one
+// wavefront per SIMD at the larger sizes) waits for.  An admitted grid therefore gives up after 2^19 polls (an eighth
 // of the cooperative launch's limit) and heev_lowest_shared repeats the call cooperatively.  The holder synchronises its stream
 // (the grid has finished) and returns its share when it goes out of scope.  Cooperative launches (the enqueue-only entry
 // points) are not counted: one that runs while concurrent solves hold the gate may find the
-// device short of CUs, and its barrier's spin limit then reports an error instead of waiting.
+// device short of CUs, and its spin limit then reports an error instead of waiting.
 struct TrdAdmission {
     int device = -1, units = 0;
     hipStream_t stream = nullptr;
@@ -67,11 +66,11 @@ void heev_lowest(HeevWork& w, const double2* A, int lda, int m, int nev, double*
 // The tridiagonal stage only (for tests): d[0:m], e[0:m-1] of T on the device.
 void heev_tridiag_only(HeevWork& w, const double2* A, int lda, int m, hipStream_t s);
 
-// Error flag of the last tridiagonalisation (a grid barrier that did not complete); synchronises s.
+// Error flag of the last tridiagonalisation (an exchange that did not complete); synchronises s.
 int heev_error_flag(HeevWork& w, hipStream_t s);
 
 // heev_lowest through the gate, synchronised: the tridiagonalisation runs as an admitted ordinary
-// dispatch whose barrier gives up after 2^19 polls without all its workgroups (other streams'
+// dispatch that gives up after 2^19 polls without all its workgroups (other streams'
 // kernels can keep the CUs it waits for), and is then repeated as a cooperative launch.  Throws if
 // that fails too.  heev_shared_retries counts the repeats in the process.
 void heev_lowest_shared(HeevWork& w, const double2* A, int lda, int m, int nev, double* w_dev, double2* Y, int ldy,

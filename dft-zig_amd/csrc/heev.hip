@@ -14,12 +14,9 @@ namespace dzhip {
 
 namespace {
 
-constexpr int kTrdThreads = 256;
-constexpr int kTrdColsPerGroup = 6;   // trailing-matrix columns held in each workgroup's LDS
-constexpr int kTrdMaxCols = 16;
-constexpr int kTrdRowsPerThread = (1024 + 255) / 256;  // rows per thread at m <= kHeevMaxM
-constexpr unsigned kSpinLimit = 1u << 22;  // barrier polls (each after s_sleep) before giving up
-// Barrier polls of a tridiagonalisation admitted by the gate: its grid may find the device short
+constexpr int kTrdWaves = 4;  // wavefronts per workgroup of the tridiagonalisation, one per SIMD
+constexpr unsigned kSpinLimit = 1u << 22;  // polls of one exchange (under a microsecond each) before giving up
+// The same for a tridiagonalisation admitted by the gate: its grid may find the device short
 // of CUs for a long time while other streams' kernels keep taking them, and it is then repeated as
 // a cooperative launch (heev_lowest_shared).  Si-64 concurrent-k SCF, mixed arm to 1e-6 Ha: 9.16 s
 // at 2^16 polls (frequent repeats), 8.60 s at 2^19, 10.21 s with cooperative launches only.
@@ -33,114 +30,66 @@ __device__ __forceinline__ double dpp_rot(double v) {
     return __hiloint2double(hi, lo);
 }
 
-__device__ __forceinline__ double read_lane(double v, int lane) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+// Exchange between the lane rows (16 lanes) of a wavefront and add: ROWS = 1 pairs rows 0-1 and 2-3,
+// ROWS = 2 the halves.  Both lanes of a pair add the same two values in the same order.
+template <int ROWS>
+__device__ __forceinline__ double swap_add(double v) {
+    const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+    if constexpr (ROWS == 1) {
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+    } else {
+        const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+    }
 }
 
 // Sum over the 64 lanes of a wavefront (all lanes active), the same value in every lane: rotations
 // by 8, 4, 2, 1 within each 16-lane row leave every lane of the row holding the row's sum (the same
-// pairs added in every lane, so bitwise equal), then the four row sums are read from lanes 0, 16,
-// 32 and 48.  No LDS traffic (a __shfl_xor butterfly is six ds_bpermute round trips).
+// pairs added in every lane, so bitwise equal), then the rows are swapped and added pairwise.  No
+// LDS traffic (a __shfl_xor butterfly is six ds_bpermute round trips) and no scalar registers.
 __device__ __forceinline__ double wave_sum(double v) {
     v += dpp_rot<0x128>(v);  // row_ror:8
     v += dpp_rot<0x124>(v);  // row_ror:4
     v += dpp_rot<0x122>(v);  // row_ror:2
     v += dpp_rot<0x121>(v);  // row_ror:1
-    return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
+    return swap_add<2>(swap_add<1>(v));
 }
 
-// Sum of n values over the workgroup (NT threads); every thread gets the n sums in out[].
-// red holds (NT / 64) * n doubles.
-template <int NT, int N>
-__device__ __forceinline__ void block_sums(double (&vals)[N], double* red, double (&out)[N]) {
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-#pragma unroll
-    for (int k = 0; k < N; ++k) vals[k] = wave_sum(vals[k]);
-    __syncthreads();
-    if (lane == 0) {
-#pragma unroll
-        for (int k = 0; k < N; ++k) red[wv * N + k] = vals[k];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        double s = 0.0;
-#pragma unroll
-        for (int i = 0; i < NT / 64; ++i) s += red[i * N + k];
-        out[k] = s;
-    }
+// 1 / sqrt(s) and 1 / s from the hardware's estimates (relative error e about 1e-8) by one
+// third-order Newton step, 1 - e expanded to e^2: a few dependent operations on the chain of every
+// reflector, where the IEEE square root and divisions are some sixty.
+__device__ __forceinline__ double rsqrt3(double s) {
+    const double r = __builtin_amdgcn_rsq(s);
+    const double e = fma(-(s * r), r, 1.0);
+    return fma(r * e, fma(0.375, e, 0.5), r);
+}
+__device__ __forceinline__ double recip3(double s) {
+    const double r = __builtin_amdgcn_rcp(s);
+    const double e = fma(-s, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 }
 
-// Data that one workgroup writes and others read inside the tridiagonalisation (the published
-// p_j and column j+1) goes through relaxed agent-scope atomics: such stores write through the
-// XCD's L2 and such loads do not hit a stale L2 copy, so the barrier below needs no L2 writeback
-// or invalidate (an agent-scope fence costs several microseconds per workgroup), only that every
-// store has completed before the flag goes out.
-__device__ __forceinline__ void xstore(double2* p, double2 v) {
-    double* q = reinterpret_cast<double*>(p);
-    __hip_atomic_store(q, v.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(q + 1, v.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ double2 xload(const double2* p) {
-    const double* q = reinterpret_cast<const double*>(p);
-    return make_double2(__hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                        __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
+// The workgroups of the tridiagonalisation exchange two vectors per reflector (p_j and column j+1)
+// through a buffer that is written once per call: every entry starts as kUnset, a signalling NaN
+// that no arithmetic result can be (published values are canonicalised, which quiets NaNs), and a
+// reader polls the entry itself until it is set.  One trip through memory per reflector, where a
+// barrier costs three (wait for the stores, flag, then the values): 2.3 us against about 1 us.
+// Stores and polls are relaxed agent-scope atomics, which write through the XCD's L2 and do not hit
+// a stale copy there; each 8-byte entry carries its own arrival, so no ordering between entries is
+// assumed.
+constexpr unsigned long long kUnset = 0x7FF4DEADBEEF5A5Aull;
 
-// Barrier over the whole (co-resident) grid.  Each workgroup owns a flag on its own 64-byte line
-// and stores the barrier's epoch there (no read-modify-write on a shared counter, whose atomics
-// serialise: about 70 ns per arriving workgroup); wavefront 0 of every workgroup then polls all
-// flags (64 per load instruction) until each has reached the epoch.  Every thread first waits for
-// its own memory operations to complete (s_waitcnt 0), so the exchanged data written with xstore
-// is in place before the flag is.  With part != nullptr, wavefront 0 then also sums part[0:G]
-// (one complex value per workgroup, written with xstore before the barrier) into sum[0:2].
-// A wait longer than spin_limit polls (or an error raised elsewhere) sets *err; every thread
-// returns false then and the kernel winds down.
-__device__ bool grid_sync(unsigned* flags, unsigned epoch, int* err, int* s_ok, unsigned spin_limit,
-                          const double2* part = nullptr, double* sum = nullptr) {
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __syncthreads();
-    if (threadIdx.x < 64) {
-        const int lane = (int)threadIdx.x;
-        const int G = (int)gridDim.x;
-        if (lane == 0)
-            __hip_atomic_store(flags + (size_t)blockIdx.x * 16, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        unsigned spins = 0;
-        int ok = 1;
-        while (true) {
-            int arrived = 1;
-            for (int q = lane; q < G; q += 64)
-                arrived &= __hip_atomic_load(flags + (size_t)q * 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= epoch;
-            if (__all(arrived)) break;
-            const int bad = lane == 0 ? __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-            if (__any(bad) || ++spins > spin_limit) {
-                if (lane == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                ok = 0;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        if (part && ok) {
-            double sx = 0.0, sy = 0.0;
-            for (int q = lane; q < G; q += 64) {
-                const double2 v = xload(part + q);
-                sx += v.x;
-                sy += v.y;
-            }
-            sx = wave_sum(sx);
-            sy = wave_sum(sy);
-            if (lane == 0) {
-                sum[0] = sx;
-                sum[1] = sy;
-            }
-        }
-        if (lane == 0) *s_ok = ok;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    __syncthreads();
-    return *s_ok != 0;
+__device__ __forceinline__ void publish(double* p, double v) {
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(p),
+                       (unsigned long long)__double_as_longlong(__builtin_canonicalize(v)), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long peek(const double* p) {
+    return __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __device__ __forceinline__ double2 cm(double2 a, double2 b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
@@ -151,237 +100,315 @@ __device__ __forceinline__ double2 cjm(double2 a, double2 b) {
 
 struct TrdArgs {
     const double2* A;
-    int lda, m, ncl;
+    int lda, m;
     double2* vh;   // m x m: column j holds reflector v_j in rows j+1..m-1 (v_j[j+1] = 1)
     double2* tau;  // m
     double* d;     // m
     double* e;     // m - 1
-    double2* pbuf; // 2 x m: tau_j A v_j, then 2 x G: per-workgroup parts of p_j^H v_j; by step parity
-    double2* nbuf; // 2 x m: the next column after the previous rank-2 update
-    unsigned* flags;  // one per workgroup, 16 apart
+    double* pub;   // m rows of 2 m doubles (several workgroups only): see trd_p, trd_n
     int* err;
-    unsigned spin_limit;  // barrier polls before giving up
+    unsigned spin_limit;  // polls of one exchange before giving up
 };
 
+// Where step j's vectors lie in pub, real parts then (m doubles on) imaginary parts: p_j[r], r > j,
+// in the upper part of row j and column j+1's rows r > j in the part of row m-1-j that p_{m-1-j}
+// leaves free (0 <= r-j-1 <= m-2-j, and p_{m-1-j} starts at m-j).
+__device__ __forceinline__ double* trd_p(double* pub, int m, int j, int r) { return pub + (size_t)j * 2 * m + r; }
+__device__ __forceinline__ double* trd_n(double* pub, int m, int j, int r) {
+    return pub + (size_t)(m - 1 - j) * 2 * m + (r - j - 1);
+}
+
 // Householder tridiagonalisation A = Q T Q^H, Q = H_0 ... H_{m-2}, H_j = I - tau_j v_j v_j^H, with
-// zhetd2's reflectors (zlarfg: H_j^H x = beta e_1, beta real).  Workgroup g holds the trailing
-// columns i = g + c G (c < NCL) in LDS for the whole reduction, and every workgroup keeps its own
-// copy of the current column.  Step j (thread t works on rows r = j+1+t (mod 256) throughout, so
-// that its phases need no workgroup barrier between them):
-//   A. every workgroup forms v_j, tau_j from the current column j (norm of rows j+2.. summed at
-//      the end of the previous step);
-//   B. fused pass over its own columns i > j: the rank-2 update of step j-1
-//      a_i -= v_{j-1} conj(w_{j-1}[i]) + w_{j-1} conj(v_{j-1}[i]), then p_j[i] = tau_j a_i^H v_j
-//      (A is Hermitian, so (A v)_i = a_i^H v); the owner of column j+1 publishes it (updated), and
-//      every workgroup publishes its part of p_j^H v_j;
-//   C. grid barrier, which also sums those parts;
-//   D. w_j = p_j - (tau_j / 2) (p_j^H v_j) v_j, from the published p_j;
-//   E. column j+1 = published column - v_j conj(w_j[j+1]) - w_j conj(v_j[j+1]), and the norm of
-//      its rows j+3.. for the next step.
-// The owner never updates column j+1 in place at step j, so the published copy stays valid while
-// the others read it; the published buffers alternate by step parity.
-template <int NCL>
-__global__ __launch_bounds__(kTrdThreads) void k_hetrd(TrdArgs a) {
-    extern __shared__ double2 lds[];
-    __shared__ double red[(kTrdThreads / 64) * 2 * kTrdMaxCols];
-    __shared__ double s_dot[2];
-    __shared__ int s_ok;
-    constexpr int ncl = NCL;
-    constexpr int NT = kTrdThreads;
-    const int m = a.m, G = (int)gridDim.x, g = (int)blockIdx.x, t = (int)threadIdx.x;
-    const int wv = t >> 6, lane = t & 63;
-    double2* cols = lds;
-    // Roles, rotated every step: vc = current column (becomes v_j in place), wn = w_j,
-    // vp / wp = v_{j-1}, w_{j-1}.
-    double2* vc_b = cols + (size_t)ncl * m;
-    double2* wn_b = cols + (size_t)(ncl + 1) * m;
-    double2* vp_b = cols + (size_t)(ncl + 2) * m;
-    double2* wp_b = cols + (size_t)(ncl + 3) * m;
-    // Only the lower triangle of A is read (the upper one is its mirror; the diagonal is real), as
-    // LAPACK's zheev with uplo = 'L'.
-    for (int c = 0; c < ncl; ++c) {
-        const int i = g + c * G;
-        if (i >= m) break;
-        for (int r = t; r < m; r += NT) {
-            double2 x;
-            if (r > i) x = a.A[(size_t)i * a.lda + r];
-            else if (r == i) x = make_double2(a.A[(size_t)i * a.lda + r].x, 0.0);
-            else {
-                const double2 y = a.A[(size_t)r * a.lda + i];
-                x = make_double2(y.x, -y.y);
-            }
-            cols[(size_t)c * m + r] = x;
-        }
+// zhetd2's reflectors (zlarfg: H_j^H x = beta e_1, beta real).  Every wavefront owns CW trailing
+// columns for the whole reduction, in registers: lane l holds rows l + 64 q (q < NQ) of them and of
+// every vector, so all products are lane-local and every sum is one wavefront's, and the wavefronts
+// form v_j and w_j redundantly instead of exchanging them.  Step j:
+//   A. receive p_{j-1} and column j (each wavefront polls a share of the rows into LDS; one
+//      workgroup barrier);
+//   B. w_{j-1} = p_{j-1} - (tau_{j-1} / 2) (p_{j-1}^H v_{j-1}) v_{j-1}; column j minus
+//      v_{j-1} conj(w_{j-1}[j]) + w_{j-1} gives d_j and y; own columns i > j minus
+//      v_{j-1} conj(w_{j-1}[i]) + w_{j-1} conj(v_{j-1}[i]) (the owner of column j+1 publishes it);
+//   C. one reduction of |y|^2 and of the own columns' products with y gives tau_j, beta_j and
+//      p_j[i] = tau_j a_i^H v_j (A Hermitian; v_j is y scaled below row j+1, where it is one), published;
+//   D. while that travels: v_j, and the rows of v_j and of the own columns that step j+1 needs as
+//      scalars (through LDS, like every other scalar row).
+// The chain of a step is one memory trip, two wavefront sums and a square root with two divisions.
+// The steps of one 64-row chunk are a loop of their own with the chunks above it left out at
+// compile time: skipping them by branches kept every chunk's LDS reads from overlapping (0.36 us a
+// chunk and step).  A workgroup whose columns are all reduced leaves.
+template <int NQ, int CW>
+struct Trd {
+    static constexpr int NW = kTrdWaves, NT = 64 * NW, M64 = 64 * NQ, KR = NQ * 64 / NT + (NQ * 64 % NT != 0);
+    const TrdArgs& a;
+    double2* lds;  // two steps' [p | column j], M64 rows each
+    double2* s_x;  // two steps' [NW * CW own columns' next row | v's next row]
+    int* s_bad;
+    int m, t, lane, wv, last_col;
+    bool scribe;  // the wavefront that owns the last column writes T and the reflectors
+    int ic[CW];
+    double2 x[CW][NQ], y[NQ], v[NQ], w[NQ];
+    double2 alpha, tau, vn;                // column j's row j+1, tau_j, v_{j-1}[j+1]
+    double2 vi[CW], wi[CW], yi[CW], xo[CW];  // rows i of v, w and y; own columns' row j+1
+
+    __device__ __forceinline__ double2 elem(int r, int i) const {
+        // Only the lower triangle of A is read (the upper one is its mirror; the diagonal is real),
+        // as LAPACK's zheev with uplo = 'L'.  Zero outside the matrix.
+        if (r >= m || i >= m) return make_double2(0.0, 0.0);
+        const double2 u = r >= i ? a.A[(size_t)i * a.lda + r] : a.A[(size_t)r * a.lda + i];
+        return make_double2(u.x, r == i ? 0.0 : (r > i ? u.y : -u.y));
     }
-    for (int r = t; r < m; r += NT) vc_b[r] = r == 0 ? make_double2(a.A[0].x, 0.0) : a.A[r];
-    __syncthreads();
-    double xs = 0.0;  // this thread's part of |column j, rows j+2..|^2
-    for (int r = 1 + t; r < m; r += NT)
-        if (r >= 2) xs += vc_b[r].x * vc_b[r].x + vc_b[r].y * vc_b[r].y;
-    for (int j = 0; j + 1 < m; ++j) {
-        double2* vc = vc_b;
-        // A. reflector of column j (rows j+1..m-1).  Every thread reads alpha between the two
-        // barriers; thread 0 overwrites its row only after the second.
-        xs = wave_sum(xs);
-        __syncthreads();
-        const double2 alpha = vc[j + 1];
-        const double dj = vc[j].x;
-        if (lane == 0) red[wv] = xs;
-        __syncthreads();
-        double xn2 = 0.0;
+
+    // C and D of step j, whose rows j+1.. lie in chunks QB and up.
+    template <int QB>
+    __device__ __forceinline__ void reflect(int j) {
 #pragma unroll
-        for (int q = 0; q < NT / 64; ++q) xn2 += red[q];
+        for (int c = 0; c < CW; ++c)
+            if (ic[c] == j + 1) {
+#pragma unroll
+                for (int q = QB; q < NQ; ++q) {
+                    const int r = lane + 64 * q;
+                    if (r <= j || r >= m) continue;
+                    double* pn = trd_n(a.pub, m, j, r);
+                    publish(pn, x[c][q].x);
+                    publish(pn + m, x[c][q].y);
+                }
+            }
+        double sums[1 + 2 * CW];
+#pragma unroll
+        for (int c = 0; c < 1 + 2 * CW; ++c) sums[c] = 0.0;
+#pragma unroll
+        for (int q = QB; q < NQ; ++q) {
+            sums[0] += y[q].x * y[q].x + y[q].y * y[q].y;
+#pragma unroll
+            for (int c = 0; c < CW; ++c) {
+                const double2 u = cjm(x[c][q], y[q]);
+                sums[1 + 2 * c] += u.x;
+                sums[2 + 2 * c] += u.y;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 1 + 2 * CW; ++c) sums[c] = wave_sum(sums[c]);
+        const double xn2 = sums[0];
         double beta;
-        double2 tau, scale;
+        double2 scale;
         if (xn2 == 0.0 && alpha.y == 0.0) {
             tau = make_double2(0.0, 0.0);
             beta = alpha.x;
             scale = make_double2(0.0, 0.0);
         } else {
-            const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + xn2);
+            const double n2 = alpha.x * alpha.x + alpha.y * alpha.y + xn2;
+            const double ir = rsqrt3(n2), nrm = n2 * ir;
+            const double ib = alpha.x >= 0.0 ? -ir : ir;
             beta = alpha.x >= 0.0 ? -nrm : nrm;
-            tau = make_double2((beta - alpha.x) / beta, -alpha.y / beta);
+            tau = make_double2((beta - alpha.x) * ib, -alpha.y * ib);
             const double2 den = make_double2(alpha.x - beta, alpha.y);
-            const double dd = den.x * den.x + den.y * den.y;
-            scale = make_double2(den.x / dd, -den.y / dd);
+            const double id = recip3(den.x * den.x + den.y * den.y);
+            scale = make_double2(den.x * id, -den.y * id);
         }
-        if (g == 0 && t == 0) {
-            a.d[j] = dj;
-            a.e[j] = beta;
-            a.tau[j] = tau;
-        }
-        for (int r = j + 1 + t; r < m; r += NT) {
-            const double2 v = r == j + 1 ? make_double2(1.0, 0.0) : cm(vc[r], scale);
-            vc[r] = v;
-            if (g == 0) a.vh[(size_t)j * m + r] = v;
-        }
-        // B. fused update (step j-1) and product (step j) over the own columns i >= j+1.
-        const double2* vp = vp_b;
-        const double2* wp = wp_b;
-        double part[2 * ncl];
-        double2 wi[ncl], vi[ncl];
 #pragma unroll
-        for (int c = 0; c < ncl; ++c) {
-            const int i = g + c * G;
-            const bool live = j > 0 && i > j && i < m;
-            wi[c] = live ? wp[i] : make_double2(0.0, 0.0);
-            vi[c] = live ? vp[i] : make_double2(0.0, 0.0);
-            part[2 * c] = 0.0;
-            part[2 * c + 1] = 0.0;
-        }
-        double2* nb_out = a.nbuf + (size_t)((j + 1) & 1) * m;
-        for (int r = j + 1 + t; r < m; r += NT) {
-            const double2 vr = vc[r];
-            const double2 vpr = j > 0 ? vp[r] : make_double2(0.0, 0.0);
-            const double2 wpr = j > 0 ? wp[r] : make_double2(0.0, 0.0);
-#pragma unroll
-            for (int c = 0; c < ncl; ++c) {
-                const int i = g + c * G;
-                if (i <= j || i >= m) continue;
-                double2* col = cols + (size_t)c * m;
-                double2 x = col[r];
-                if (j > 0) {
-                    // x -= vp[r] conj(wi) + wp[r] conj(vi)
-                    const double2 u1 = cjm(wi[c], vpr);
-                    const double2 u2 = cjm(vi[c], wpr);
-                    x.x -= u1.x + u2.x;
-                    x.y -= u1.y + u2.y;
-                    col[r] = x;
-                }
-                const double2 pr = cjm(x, vr);
-                part[2 * c] += pr.x;
-                part[2 * c + 1] += pr.y;
-                if (i == j + 1) xstore(nb_out + r, x);
-            }
-        }
-        double sums[2 * ncl];
-        block_sums<NT>(part, red, sums);
-        double2* pb = a.pbuf + (size_t)(j & 1) * m;
-        double2* dpart = a.pbuf + (size_t)2 * m + (size_t)(j & 1) * G;
-        double2 pdot = make_double2(0.0, 0.0);
-#pragma unroll
-        for (int c = 0; c < ncl; ++c) {
-            const int i = g + c * G;
-            if (i > j && i < m) {
-                const double2 p = cm(tau, make_double2(sums[2 * c], sums[2 * c + 1]));
-                if (t == c) xstore(pb + i, p);
-                const double2 u = cjm(p, vc[i]);
-                pdot.x += u.x;
-                pdot.y += u.y;
-            }
-        }
-        if (t == 0) xstore(dpart + g, pdot);
-        // C.
-        if (!grid_sync(a.flags, (unsigned)(j + 1), a.err, &s_ok, a.spin_limit)) return;
-        // Every published value this thread needs, loaded together: p_j and column j+1 on its own
-        // rows, p_j[j+1], and (wavefront 0) the parts of p_j^H v_j.
-        const double2* nb_in = a.nbuf + (size_t)((j + 1) & 1) * m;
-        double2 pr_in[kTrdRowsPerThread], nr_in[kTrdRowsPerThread];
-#pragma unroll
-        for (int q = 0; q < kTrdRowsPerThread; ++q) {
-            const int r = j + 1 + t + q * NT;
-            if (r < m) {
-                pr_in[q] = xload(pb + r);
-                nr_in[q] = xload(nb_in + r);
-            }
-        }
-        const double2 pj1 = xload(pb + j + 1);
-        if (wv == 0) {
-            double sx = 0.0, sy = 0.0;
-            for (int q = lane; q < G; q += 64) {
-                const double2 v = xload(dpart + q);
-                sx += v.x;
-                sy += v.y;
-            }
-            sx = wave_sum(sx);
-            sy = wave_sum(sy);
+        for (int c = 0; c < CW; ++c) {
+            if (ic[c] <= j || ic[c] >= m) continue;
+            const double2 s = cm(scale, make_double2(sums[1 + 2 * c], sums[2 + 2 * c]));
+            const double2 p = cm(tau, make_double2(xo[c].x + s.x, s.y - xo[c].y));
             if (lane == 0) {
-                s_dot[0] = sx;
-                s_dot[1] = sy;
+                double* pp = trd_p(a.pub, m, j, ic[c]);
+                publish(pp, p.x);
+                publish(pp + m, p.y);
+            }
+        }
+        double2* sx = s_x + (j & 1) * (NW * CW + 1);
+#pragma unroll
+        for (int q = QB; q < NQ; ++q) {
+            v[q] = cm(y[q], scale);
+            if (q <= QB + 1) {
+                const int r = lane + 64 * q;
+                if (r == j + 1) v[q] = make_double2(1.0, 0.0);
+                if (r == j + 2) {
+                    if (wv == 0) sx[NW * CW] = v[q];
+#pragma unroll
+                    for (int c = 0; c < CW; ++c) sx[wv * CW + c] = x[c][q];
+                }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < CW; ++c) vi[c] = ic[c] == j + 1 ? make_double2(1.0, 0.0) : cm(yi[c], scale);
+        if (scribe) {
+#pragma unroll
+            for (int q = QB; q < NQ; ++q) {
+                const int r = lane + 64 * q;
+                if (r > j && r < m) a.vh[(size_t)j * m + r] = v[q];
+            }
+            if (lane == 0) {
+                a.e[j] = beta;
+                a.tau[j] = tau;
+            }
+        }
+    }
+
+    // A and B of step j (rows j.. in chunks QB and up); false when the exchange gave up.
+    template <int QB>
+    __device__ __forceinline__ bool advance(int j) {
+        double2* sp = lds + (j & 1) * 2 * M64;
+        double2* sn = sp + M64;
+        unsigned long long in[KR][4];
+        unsigned spins = 0;
+        while (true) {
+            bool set = true;
+#pragma unroll
+            for (int k = 0; k < KR; ++k) {
+                const int r = t + k * NT;
+                if (r >= j && r < m) {
+                    const double* pp = trd_p(a.pub, m, j - 1, r);
+                    const double* pn = trd_n(a.pub, m, j - 1, r);
+                    in[k][0] = peek(pp);
+                    in[k][1] = peek(pp + m);
+                    in[k][2] = peek(pn);
+                    in[k][3] = peek(pn + m);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < KR; ++k) {
+                const int r = t + k * NT;
+                if (r >= j && r < m)
+                    set = set && in[k][0] != kUnset && in[k][1] != kUnset && in[k][2] != kUnset && in[k][3] != kUnset;
+            }
+            if (__all(set)) break;
+            ++spins;
+            const bool stop = (spins & 255u) == 0 &&
+                              __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+            if (spins > a.spin_limit || __any(stop)) {
+                if (lane == 0) {
+                    __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    *s_bad = 1;
+                }
+                break;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < KR; ++k) {
+            const int r = t + k * NT;
+            if (r >= j && r < m) {
+                sp[r] = make_double2(__longlong_as_double((long long)in[k][0]), __longlong_as_double((long long)in[k][1]));
+                sn[r] = make_double2(__longlong_as_double((long long)in[k][2]), __longlong_as_double((long long)in[k][3]));
             }
         }
         __syncthreads();
-        // D. w_j = p_j - (tau_j / 2) (p_j^H v_j) v_j on the own rows; row j+1 by every thread.
-        double2* wn = wn_b;
-        const double2 al = cm(make_double2(-0.5 * tau.x, -0.5 * tau.y), make_double2(s_dot[0], s_dot[1]));
+        if (*s_bad) return false;
+        // Rows below j of sp and sn are an earlier step's (finite) and meet v = 0 there; rows from m
+        // on are zero.
+        const double2* sx = s_x + ((j - 1) & 1) * (NW * CW + 1);
 #pragma unroll
-        for (int q = 0; q < kTrdRowsPerThread; ++q) {
-            const int r = j + 1 + t + q * NT;
-            if (r < m) {
-                const double2 u = cm(al, vc[r]);
-                wn[r] = make_double2(pr_in[q].x + u.x, pr_in[q].y + u.y);
+        for (int q = QB; q < NQ; ++q) w[q] = sp[lane + 64 * q];
+        const int j1 = min(j + 1, M64 - 1);
+        const double2 pj = sp[j], pj1 = sp[j1];
+        vn = sx[NW * CW];
+        double2 pi[CW];
+#pragma unroll
+        for (int c = 0; c < CW; ++c) {
+            pi[c] = sp[min(ic[c], M64 - 1)];
+            yi[c] = sn[min(ic[c], M64 - 1)];
+            xo[c] = sx[wv * CW + c];
+        }
+        const double2 nj = sn[j], nj1 = sn[j1];
+#pragma unroll
+        for (int q = QB; q < NQ; ++q) y[q] = sn[lane + 64 * q];
+        double2 dot = make_double2(0.0, 0.0);
+#pragma unroll
+        for (int q = QB; q < NQ; ++q) {
+            const double2 u = cjm(w[q], v[q]);
+            dot.x += u.x;
+            dot.y += u.y;
+        }
+        dot.x = wave_sum(dot.x);
+        dot.y = wave_sum(dot.y);
+        const double2 al = cm(make_double2(-0.5 * tau.x, -0.5 * tau.y), dot);
+        const double2 wj = make_double2(pj.x + al.x, pj.y + al.y);  // v_{j-1}[j] = 1
+        const double2 aln = cm(al, vn), wn = make_double2(pj1.x + aln.x, pj1.y + aln.y);
+        const double2 ua = cjm(wj, vn);
+        alpha = make_double2(nj1.x - ua.x - wn.x, nj1.y - ua.y - wn.y);
+        if (scribe && lane == 0) a.d[j] = nj.x - 2.0 * wj.x;
+#pragma unroll
+        for (int c = 0; c < CW; ++c) {
+            const double2 u = cm(al, vi[c]);
+            wi[c] = make_double2(pi[c].x + u.x, pi[c].y + u.y);
+            const double2 uy = cjm(wj, vi[c]);
+            yi[c] = make_double2(yi[c].x - uy.x - wi[c].x, yi[c].y - uy.y - wi[c].y);
+            const double2 u1 = cjm(wi[c], vn), u2 = cjm(vi[c], wn);
+            xo[c] = make_double2(xo[c].x - u1.x - u2.x, xo[c].y - u1.y - u2.y);
+        }
+#pragma unroll
+        for (int q = QB; q < NQ; ++q) {
+            const double2 u = cm(al, v[q]);
+            w[q] = make_double2(w[q].x + u.x, w[q].y + u.y);
+            const double2 u0 = cjm(wj, v[q]);
+            y[q] = make_double2(y[q].x - u0.x - w[q].x, y[q].y - u0.y - w[q].y);
+            if (q <= QB + 1 && lane + 64 * q < j + 2) y[q] = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int c = 0; c < CW; ++c) {
+                const double2 u1 = cjm(wi[c], v[q]), u2 = cjm(vi[c], w[q]);
+                x[c][q].x -= u1.x + u2.x;
+                x[c][q].y -= u1.y + u2.y;
             }
         }
-        const double2 wj1 = make_double2(pj1.x + al.x, pj1.y + al.y);  // v_j[j+1] = 1
-        // E. column j+1 after the step-j update, into the buffer of v_{j-1} (no longer needed).
-        double2* vnext = vp_b;
-        xs = 0.0;
-#pragma unroll
-        for (int q = 0; q < kTrdRowsPerThread; ++q) {
-            const int r = j + 1 + t + q * NT;
-            if (r >= m) continue;
-            const double2 x = nr_in[q];
-            const double2 u1 = cjm(wj1, vc[r]);
-            const double2 w = wn[r];  // conj(v_j[j+1]) w_j[r] with v_j[j+1] = 1
-            const double2 y = make_double2(x.x - u1.x - w.x, x.y - u1.y - w.y);
-            vnext[r] = y;
-            if (r >= j + 3) xs += y.x * y.x + y.y * y.y;
-        }
-        if (j + 2 == m && g == 0 && t == 0) a.d[m - 1] = vnext[m - 1].x;
-        // Rotate: v_{j-1} <- v_j, w_{j-1} <- w_j, current column <- column j+1.
-        double2* const old_vp = vp_b;
-        double2* const old_wp = wp_b;
-        vp_b = vc_b;
-        wp_b = wn_b;
-        vc_b = old_vp;
-        wn_b = old_wp;
+        return true;
     }
-    if (m == 1 && g == 0 && t == 0) a.d[0] = a.A[0].x;
+
+    // Steps whose reflector starts in chunk QB, then the next chunks'.
+    template <int QB>
+    __device__ __forceinline__ void run() {
+        if constexpr (QB < NQ) {
+            const int end = min(64 * (QB + 1), m - 1);
+            for (int j = 64 * QB; j < end; ++j) {
+                reflect<QB>(j);
+                if (last_col <= j + 1 && last_col != m - 1) return;
+                if (!advance<QB>(j + 1)) return;
+            }
+            run<QB + 1>();
+        }
+    }
+};
+
+template <int NQ, int CW>
+__global__ __launch_bounds__(64 * kTrdWaves, 1) void k_hetrd(TrdArgs a) {
+    extern __shared__ double2 lds[];
+    __shared__ double2 s_x[2 * (kTrdWaves * CW + 1)];
+    __shared__ int s_bad;
+    using K = Trd<NQ, CW>;
+    const int t = (int)threadIdx.x, g = (int)blockIdx.x, m = a.m;
+    K k{a, lds, s_x, &s_bad, m, t, t & 63, __builtin_amdgcn_readfirstlane(t >> 6)};
+    k.last_col = min(m, (g + 1) * K::NW * CW) - 1;
+    k.scribe = false;
+    for (int i = t; i < 4 * K::M64; i += K::NT) lds[i] = make_double2(0.0, 0.0);
+    if (t < 2 * (K::NW * CW + 1)) s_x[t] = make_double2(0.0, 0.0);
+    if (t == 0) s_bad = 0;
+#pragma unroll
+    for (int c = 0; c < CW; ++c) {
+        const int i = k.ic[c] = (g * K::NW + k.wv) * CW + c;
+        k.scribe = k.scribe || i == m - 1;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) k.x[c][q] = k.elem(k.lane + 64 * q, i);
+        k.xo[c] = k.elem(1, i);
+        k.yi[c] = k.elem(i, 0);
+        k.vi[c] = make_double2(0.0, 0.0);
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int r = k.lane + 64 * q;
+        k.y[q] = r >= 2 ? k.elem(r, 0) : make_double2(0.0, 0.0);
+        k.v[q] = make_double2(0.0, 0.0);
+    }
+    k.alpha = k.elem(1, 0);
+    k.tau = k.vn = make_double2(0.0, 0.0);
+    if (k.scribe && k.lane == 0) a.d[0] = a.A[0].x;
+    __syncthreads();
+    k.template run<0>();
 }
 
-__global__ void k_zero_u32(unsigned* p, int n) {
-    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i < n) p[i] = 0u;
+// The exchange buffer's entries unset, the error flag cleared.
+__global__ __launch_bounds__(256) void k_trd_init(ulonglong2* pub, size_t n, int* err) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i == 0) *err = 0;
+    if (i < n) pub[i] = make_ulonglong2(kUnset, kUnset);
 }
 
 // Sturm counts: numbers of eigenvalues of T(d, e) below x[0..NP) (e2 = e^2), with tiny pivots
@@ -458,7 +485,7 @@ __global__ __launch_bounds__(256) void k_stebz(const double* __restrict__ d_in, 
     const int lane = t & 63;
     const int idx = (int)blockIdx.x * 4 + (t >> 6);
     if (idx >= nev) return;
-    // A tridiagonalisation whose grid barrier did not complete leaves NaN eigenvalues (the signal
+    // A tridiagonalisation whose exchange did not complete leaves NaN eigenvalues (the signal
     // a caller without a synchronising check sees).
     if (*err != 0) {
         if (lane == 0) w[idx] = __builtin_nan("");
@@ -815,18 +842,18 @@ const void* unmtr_kernel(int m) {
     return (const void*)k_unmtr<16>;
 }
 
-size_t trd_lds_bytes(int m, int ncl) { return (size_t)(ncl + 4) * (size_t)m * sizeof(double2); }
 size_t stein_lds_bytes(int m) { return (size_t)7 * m * sizeof(double) + (size_t)m; }
 
-// The tridiagonalisation kernel for ncl columns per workgroup (1..kTrdMaxCols).
-const void* trd_kernel(int ncl) {
-    static const void* const table[kTrdMaxCols] = {
-        (const void*)k_hetrd<1>,  (const void*)k_hetrd<2>,  (const void*)k_hetrd<3>,  (const void*)k_hetrd<4>,
-        (const void*)k_hetrd<5>,  (const void*)k_hetrd<6>,  (const void*)k_hetrd<7>,  (const void*)k_hetrd<8>,
-        (const void*)k_hetrd<9>,  (const void*)k_hetrd<10>, (const void*)k_hetrd<11>, (const void*)k_hetrd<12>,
-        (const void*)k_hetrd<13>, (const void*)k_hetrd<14>, (const void*)k_hetrd<15>, (const void*)k_hetrd<16>};
-    return table[std::max(1, std::min(ncl, kTrdMaxCols)) - 1];
-}
+// One instance of the tridiagonalisation: m <= 64 nq rows, cw columns per wavefront.
+struct TrdKernel {
+    int nq, cw;
+    const void* fn;
+    size_t lds() const { return (size_t)4 * 64 * nq * sizeof(double2); }
+};
+#define DZ_TRD(NQ) {NQ, 1, (const void*)k_hetrd<NQ, 1>}, {NQ, 2, (const void*)k_hetrd<NQ, 2>}
+const TrdKernel kTrdKernels[] = {DZ_TRD(1), DZ_TRD(2), DZ_TRD(3), DZ_TRD(4), DZ_TRD(6),
+                                 DZ_TRD(8), DZ_TRD(11), DZ_TRD(13), DZ_TRD(16)};
+#undef DZ_TRD
 
 // Co-resident workgroups per device for the tridiagonalisation (one per CU at its LDS size),
 // queried once per device.
@@ -846,46 +873,49 @@ CoopInfo coop_info(int dev) {
         DZ_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
         DZ_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
         DZ_REQUIRE(coop != 0, DZHIP_ERR_HIP, "device does not support cooperative launches");
-        for (int c = 1; c <= kTrdMaxCols; ++c) set_max_dynamic_lds(trd_kernel(c), kMaxLdsBytes - 2048);
+        for (const TrdKernel& k : kTrdKernels) set_max_dynamic_lds(k.fn, k.lds());
         set_max_dynamic_lds((const void*)k_stein, stein_lds_bytes(kHeevMaxM));
         for (int mm : {256, 512, 768, kHeevMaxM}) set_max_dynamic_lds(unmtr_kernel(mm), unmtr_lds_bytes(kHeevMaxM));
-        // Launch-shape override for sweeps: trailing columns per workgroup.
+        // Launch-shape override for sweeps: trailing columns per workgroup (4 or 8).
         if (const char* env = std::getenv("DZHIP_HEEV_COLS")) c.cols_per_group = std::max(0, std::atoi(env));
         c.groups = cus;
     }
     return c;
 }
 
-// Launch shape of the tridiagonalisation: G workgroups holding ncl columns each.
-void trd_shape(int m, int* G_out, int* ncl_out) {
+// Launch shape of the tridiagonalisation: the instance and its G workgroups.  One column per
+// wavefront while the workgroups fit the device (m <= 1024 on 256 CUs): a step's chain is latency
+// and the redundant vector work of each wavefront, so a second column only lengthens it (m = 164 /
+// 328 / 648, whole eigensolver call, us: 821 / 1786 / 4013 with one, 856 / 1891 / 4560 with two).
+// This kernel alone: 1,024 -> 400 us at m = 164 and 4,887 -> 2,150 us at m = 648 (6.2 -> 2.4 and
+// 7.5 -> 3.3 us a reflector) against columns in LDS shared by four wavefronts with block sums and a
+// grid barrier.
+TrdKernel trd_shape(int m, int* G_out) {
     int dev = 0;
     DZ_HIP(hipGetDevice(&dev));
     const CoopInfo ci = coop_info(dev);
-    const int per = ci.cols_per_group > 0 ? ci.cols_per_group : kTrdColsPerGroup;
-    int G = std::max(1, std::min((m + per - 1) / per, ci.groups));
-    int ncl = (m + G - 1) / G;
-    while (trd_lds_bytes(m, ncl) > kMaxLdsBytes - 2048 && G < ci.groups) {
-        ++G;
-        ncl = (m + G - 1) / G;
-    }
-    DZ_REQUIRE(ncl <= kTrdMaxCols && trd_lds_bytes(m, ncl) <= kMaxLdsBytes - 2048, DZHIP_ERR_ARG,
-               "Hermitian eigensolver: matrix too large for the tridiagonalisation's LDS");
-    // Every workgroup must be co-resident (one per CU at this LDS size).
+    const TrdKernel* k = nullptr;
+    int cw = ci.cols_per_group >= 2 * kTrdWaves ? 2 : 1;
+    if ((m + kTrdWaves * cw - 1) / (kTrdWaves * cw) > ci.groups) cw = 2;
+    for (const TrdKernel& c : kTrdKernels)
+        if (!k && c.cw == cw && m <= 64 * c.nq) k = &c;
+    const int G = (m + kTrdWaves * cw - 1) / (kTrdWaves * cw);
+    DZ_REQUIRE(k, DZHIP_ERR_ARG, "Hermitian eigensolver: matrix too large for the tridiagonalisation");
+    // Every workgroup must be co-resident.
     int per_cu = 0;
-    DZ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, trd_kernel(ncl), kTrdThreads,
-                                                        trd_lds_bytes(m, ncl)));
+    DZ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k->fn, 64 * kTrdWaves, k->lds()));
     DZ_REQUIRE(per_cu >= 1 && G <= per_cu * ci.groups, DZHIP_ERR_HIP,
                "Hermitian eigensolver: grid does not fit on the device");
     *G_out = G;
-    *ncl_out = ncl;
+    return *k;
 }
 
 // Device buffers of one eigensolver call (from a HeevWork, or carved from the static scratch array).
 struct HeevBufs {
-    double2 *vh, *tau, *pbuf, *nbuf;
+    double2 *vh, *tau;
+    double *pub;  // 2 m^2: the tridiagonalisation's exchange
     double *d, *e, *z, *zt, *gram;
-    unsigned* sync;  // (G + 1) * 16 words: barrier flags, then the error flag
-    int err_offset;
+    int* err;
 };
 
 // The tridiagonalisation gate of each device (see TrdAdmission): CUs per XCD taken by admitted
@@ -933,7 +963,7 @@ bool trd_gated_enabled() {
 }
 
 // Spin limit of admitted launches; DZHIP_HEEV_SHARED_SPIN overrides it (a test sets 1 so that the
-// barrier gives up at once and the cooperative repeat runs).
+// exchange gives up at once and the cooperative repeat runs).
 unsigned shared_spin_limit() {
     static const unsigned v = [] {
         const char* env = std::getenv("DZHIP_HEEV_SHARED_SPIN");
@@ -942,29 +972,27 @@ unsigned shared_spin_limit() {
     return v;
 }
 
-void run_tridiag(const HeevBufs& b, int G, int ncl, const double2* A, int lda, int m, hipStream_t s,
+void run_tridiag(const HeevBufs& b, const TrdKernel& k, int G, const double2* A, int lda, int m, hipStream_t s,
                  bool cooperative = true) {
-    // Barrier flags (one 64-byte line per workgroup) and the error flag after them, cleared by a
-    // kernel (not a memset node) on the same stream.
-    const int nsync = (G + 1) * 16;
-    hipLaunchKernelGGL(k_zero_u32, dim3((unsigned)((nsync + 255) / 256)), dim3(256), 0, s, b.sync, nsync);
+    // The exchange's entries unset and the error flag cleared by a kernel (not a memset node) on the
+    // same stream.
+    const size_t npub = (size_t)m * m;
+    hipLaunchKernelGGL(k_trd_init, dim3((unsigned)((npub + 255) / 256)), dim3(256), 0, s,
+                       reinterpret_cast<ulonglong2*>(b.pub), npub, b.err);
     DZ_HIP(hipGetLastError());
-    TrdArgs args{A, lda, m, ncl, b.vh, b.tau, b.d, b.e, b.pbuf, b.nbuf, b.sync,
-                 reinterpret_cast<int*>(b.sync) + b.err_offset, cooperative ? kSpinLimit : shared_spin_limit()};
+    TrdArgs args{A, lda, m, b.vh, b.tau, b.d, b.e, b.pub, b.err, cooperative ? kSpinLimit : shared_spin_limit()};
     void* kargs[] = {&args};
-    if (cooperative) {
-        DZ_HIP(hipLaunchCooperativeKernel(trd_kernel(ncl), dim3((unsigned)G), dim3(kTrdThreads), kargs,
-                                          (unsigned)trd_lds_bytes(m, ncl), s));
+    if (cooperative && G > 1) {
+        DZ_HIP(hipLaunchCooperativeKernel(k.fn, dim3((unsigned)G), dim3(64u * kTrdWaves), kargs, (unsigned)k.lds(), s));
     } else {
-        DZ_HIP(hipLaunchKernel(trd_kernel(ncl), dim3((unsigned)G), dim3(kTrdThreads), kargs,
-                               (unsigned)trd_lds_bytes(m, ncl), s));
+        DZ_HIP(hipLaunchKernel(k.fn, dim3((unsigned)G), dim3(64u * kTrdWaves), kargs, k.lds(), s));
     }
 }
 
 void run_eig(const HeevBufs& b, int m, int nev, double* w_dev, double2* Y, int ldy, hipStream_t s) {
     double* scal = b.gram + (size_t)nev * nev;
     hipLaunchKernelGGL(k_stebz, dim3((unsigned)((nev + 3) / 4)), dim3(256), 2 * m * sizeof(double), s, b.d, b.e, m,
-                       nev, w_dev, scal, reinterpret_cast<const int*>(b.sync) + b.err_offset);
+                       nev, w_dev, scal, b.err);
     DZ_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_stein, dim3((unsigned)nev), dim3(64), stein_lds_bytes(m), s, b.d, b.e, m, nev, w_dev, scal,
                        b.z, m);
@@ -994,23 +1022,20 @@ void run_eig(const HeevBufs& b, int m, int nev, double* w_dev, double2* Y, int l
     DZ_HIP(hipGetLastError());
 }
 
-HeevBufs work_bufs(HeevWork& w, int m, int nev, int G) {
+HeevBufs work_bufs(HeevWork& w, int m, int nev) {
     w.vh.ensure((size_t)m * m * sizeof(double2));
     w.tau.ensure((size_t)m * sizeof(double2));
     w.d.ensure((size_t)m * sizeof(double));
     w.e.ensure((size_t)m * sizeof(double));
-    w.pbuf.ensure((size_t)2 * (m + G) * sizeof(double2));
-    w.nbuf.ensure((size_t)2 * m * sizeof(double2));
-    w.sync.ensure((size_t)(G + 1) * 16 * sizeof(unsigned));
+    w.pub.ensure((size_t)m * m * sizeof(double2));
+    w.err.ensure(64);
     if (nev > 0) {
         w.z.ensure((size_t)m * nev * sizeof(double));
         w.zt.ensure((size_t)m * nev * sizeof(double));
         w.gram.ensure((size_t)nev * nev * sizeof(double) + 64);
     }
-    w.err_offset = G * 16;
-    return HeevBufs{w.vh.as<double2>(), w.tau.as<double2>(), w.pbuf.as<double2>(), w.nbuf.as<double2>(),
-                    w.d.as<double>(),   w.e.as<double>(),     w.z.as<double>(),     w.zt.as<double>(),
-                    w.gram.as<double>(), w.sync.as<unsigned>(), G * 16};
+    return HeevBufs{w.vh.as<double2>(), w.tau.as<double2>(), w.pub.as<double>(), w.d.as<double>(),   w.e.as<double>(),
+                    w.z.as<double>(),   w.zt.as<double>(),   w.gram.as<double>(), w.err.as<int>()};
 }
 
 // ----------------------------------------------------------------- allocation-free variant
@@ -1029,19 +1054,18 @@ size_t carve(size_t& off, size_t bytes) {
     return at;
 }
 
-// Offsets of the buffers in the scratch for (m, nev, G); returns the bytes needed.
-size_t scratch_layout(int m, int nev, int G, size_t out[10]) {
+// Offsets of the buffers in the scratch for (m, nev); returns the bytes needed.
+size_t scratch_layout(int m, int nev, size_t out[9]) {
     size_t off = 0;
     out[0] = carve(off, (size_t)m * m * sizeof(double2));       // vh
     out[1] = carve(off, (size_t)m * sizeof(double2));           // tau
-    out[2] = carve(off, (size_t)2 * (m + G) * sizeof(double2)); // pbuf
-    out[3] = carve(off, (size_t)2 * m * sizeof(double2));       // nbuf
-    out[4] = carve(off, (size_t)m * sizeof(double));            // d
-    out[5] = carve(off, (size_t)m * sizeof(double));            // e
-    out[6] = carve(off, (size_t)m * nev * sizeof(double));      // z
-    out[7] = carve(off, (size_t)m * nev * sizeof(double));      // zt
-    out[8] = carve(off, (size_t)nev * nev * sizeof(double) + 64);  // gram + scale
-    out[9] = carve(off, (size_t)(G + 1) * 16 * sizeof(unsigned));  // sync
+    out[2] = carve(off, (size_t)m * m * sizeof(double2));       // pub
+    out[3] = carve(off, (size_t)m * sizeof(double));            // d
+    out[4] = carve(off, (size_t)m * sizeof(double));            // e
+    out[5] = carve(off, (size_t)m * nev * sizeof(double));      // z
+    out[6] = carve(off, (size_t)m * nev * sizeof(double));      // zt
+    out[7] = carve(off, (size_t)nev * nev * sizeof(double) + 64);  // gram + scale
+    out[8] = carve(off, 64);                                    // error flag
     return off;
 }
 
@@ -1068,31 +1092,31 @@ void heev_lowest_noalloc(int device, const double2* A, int lda, int m, int nev, 
         base = device >= 0 && device < 64 ? g_scratch_ptr[device] : nullptr;
     }
     DZ_REQUIRE(base, DZHIP_ERR_STATE, "eigensolver scratch not set up on this device (dzhip_ctx_create)");
-    int G = 1, ncl = 1;
-    trd_shape(m, &G, &ncl);
-    size_t off[10];
-    const size_t need = scratch_layout(m, nev, G, off);
+    int G = 1;
+    const TrdKernel k = trd_shape(m, &G);
+    size_t off[9];
+    const size_t need = scratch_layout(m, nev, off);
     DZ_REQUIRE(need <= kHeevNoAllocBytes, DZHIP_ERR_ARG, "allocation-free Hermitian eigensolver: scratch too small");
     unsigned char* p = static_cast<unsigned char*>(base);
     const HeevBufs b{reinterpret_cast<double2*>(p + off[0]), reinterpret_cast<double2*>(p + off[1]),
-                     reinterpret_cast<double2*>(p + off[2]), reinterpret_cast<double2*>(p + off[3]),
+                     reinterpret_cast<double*>(p + off[2]),  reinterpret_cast<double*>(p + off[3]),
                      reinterpret_cast<double*>(p + off[4]),  reinterpret_cast<double*>(p + off[5]),
                      reinterpret_cast<double*>(p + off[6]),  reinterpret_cast<double*>(p + off[7]),
-                     reinterpret_cast<double*>(p + off[8]),  reinterpret_cast<unsigned*>(p + off[9]), G * 16};
-    run_tridiag(b, G, ncl, A, lda, m, s);
+                     reinterpret_cast<int*>(p + off[8])};
+    run_tridiag(b, k, G, A, lda, m, s);
     run_eig(b, m, nev, w_dev, Y, ldy, s);
 }
 
 void HeevWork::release() {
-    DevBuf* bufs[] = {&vh, &tau, &d, &e, &pbuf, &nbuf, &sync, &z, &zt, &gram};
+    DevBuf* bufs[] = {&vh, &tau, &d, &e, &pub, &err, &z, &zt, &gram};
     for (DevBuf* b : bufs) b->release();
 }
 
 void heev_tridiag_only(HeevWork& w, const double2* A, int lda, int m, hipStream_t s) {
     DZ_REQUIRE(m >= 1 && m <= kHeevMaxM && lda >= m, DZHIP_ERR_ARG, "Hermitian eigensolver: bad size");
-    int G = 1, ncl = 1;
-    trd_shape(m, &G, &ncl);
-    run_tridiag(work_bufs(w, m, 0, G), G, ncl, A, lda, m, s);
+    int G = 1;
+    const TrdKernel k = trd_shape(m, &G);
+    run_tridiag(work_bufs(w, m, 0), k, G, A, lda, m, s);
 }
 
 TrdAdmission::~TrdAdmission() {
@@ -1105,9 +1129,9 @@ void heev_lowest(HeevWork& w, const double2* A, int lda, int m, int nev, double*
                  hipStream_t s, TrdAdmission* adm) {
     DZ_REQUIRE(m >= 1 && m <= kHeevMaxM && nev >= 1 && nev <= m && lda >= m && ldy >= m, DZHIP_ERR_ARG,
                "Hermitian eigensolver: need 1 <= nev <= m <= 1024 and leading dimensions >= m");
-    int G = 1, ncl = 1;
-    trd_shape(m, &G, &ncl);
-    const HeevBufs b = work_bufs(w, m, nev, G);
+    int G = 1;
+    const TrdKernel k = trd_shape(m, &G);
+    const HeevBufs b = work_bufs(w, m, nev);
     if (adm && trd_gated_enabled()) {
         DZ_REQUIRE(adm->units == 0, DZHIP_ERR_STATE, "Hermitian eigensolver: admission already held");
         int dev = 0;
@@ -1118,9 +1142,9 @@ void heev_lowest(HeevWork& w, const double2* A, int lda, int m, int nev, double*
         adm->device = dev;
         adm->units = units;
         adm->stream = s;
-        run_tridiag(b, G, ncl, A, lda, m, s, false);
+        run_tridiag(b, k, G, A, lda, m, s, false);
     } else {
-        run_tridiag(b, G, ncl, A, lda, m, s);
+        run_tridiag(b, k, G, A, lda, m, s);
     }
     run_eig(b, m, nev, w_dev, Y, ldy, s);
 }
@@ -1145,8 +1169,8 @@ unsigned long long heev_shared_retries() { return g_trd_retries.load(std::memory
 
 int heev_error_flag(HeevWork& w, hipStream_t s) {
     int flag = 0;
-    if (!w.sync.ptr) return 0;
-    DZ_HIP(hipMemcpyAsync(&flag, w.sync.as<int>() + w.err_offset, sizeof(int), hipMemcpyDeviceToHost, s));
+    if (!w.err.ptr) return 0;
+    DZ_HIP(hipMemcpyAsync(&flag, w.err.ptr, sizeof(int), hipMemcpyDeviceToHost, s));
     DZ_HIP(hipStreamSynchronize(s));
     return flag;
 }

@@ -41,6 +41,15 @@ def test_heev_random(ctx, m, nev):
     check(ctx, a, nev)
 
 
+@pytest.mark.parametrize("m", [3, 4, 5, 63, 64, 65, 66, 127, 129, 193, 257, 385, 513, 705, 833, 1023, 1024])
+def test_heev_register_chunks(ctx, m):
+    """Sizes at the edges of the tridiagonalisation's 64-row register chunks and of its four columns
+    per workgroup, one more row than each instance holds, and the largest; bars as above."""
+    rng = np.random.default_rng(2000 + m)
+    g = rng.standard_normal((m, m)) + 1j * rng.standard_normal((m, m))
+    check(ctx, 0.5 * (g + g.conj().T) + np.diag(np.linspace(0.0, 20.0, m)), min(m, 24))
+
+
 def test_heev_degenerate_and_clustered(ctx):
     """Exactly degenerate triplets and pairs (symmetry-degenerate bands), a cluster split by
     1e-13, and a zero off-diagonal block (a reducible tridiagonal)."""
