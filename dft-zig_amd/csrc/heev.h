@@ -15,7 +15,7 @@
 //      wavefront per eigenvalue); the members of a cluster of eigenvalues closer than a threshold
 //      are then orthonormalised together (two classical Gram-Schmidt passes), and two
 //      Newton-Schulz steps Z <- Z (3 I - Z^T Z) / 2 orthonormalise all nev vectors.
-//   4. Back-transformation Y = Q Z (one wavefront per eigenvector).
+//   4. Back-transformation Y = Q Z with the reflectors in blocks (one workgroup per eigenvector).
 #pragma once
 
 #include "dzhip_internal.h"

@@ -30,6 +30,11 @@ __device__ __forceinline__ double dpp_rot(double v) {
     return __hiloint2double(hi, lo);
 }
 
+__device__ __forceinline__ double read_lane(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
 // Exchange between the lane rows (16 lanes) of a wavefront and add: ROWS = 1 pairs rows 0-1 and 2-3,
 // ROWS = 2 the halves.  Both lanes of a pair add the same two values in the same order.
 template <int ROWS>
@@ -101,7 +106,7 @@ __device__ __forceinline__ double2 cjm(double2 a, double2 b) {
 struct TrdArgs {
     const double2* A;
     int lda, m;
-    double2* vh;   // m x m: column j holds reflector v_j in rows j+1..m-1 (v_j[j+1] = 1)
+    double2* vh;   // m x m: column j holds reflector v_j in rows j+1..m-1 (v_j[j+1] = 1), zeros above
     double2* tau;  // m
     double* d;     // m
     double* e;     // m - 1
@@ -404,11 +409,15 @@ __global__ __launch_bounds__(64 * kTrdWaves, 1) void k_hetrd(TrdArgs a) {
     k.template run<0>();
 }
 
-// The exchange buffer's entries unset, the error flag cleared.
-__global__ __launch_bounds__(256) void k_trd_init(ulonglong2* pub, size_t n, int* err) {
+// The exchange buffer's entries unset, the reflectors' rows (of which the tridiagonalisation writes
+// those from v_j[j+1] on) zero, the error flag cleared.
+__global__ __launch_bounds__(256) void k_trd_init(ulonglong2* pub, double2* vh, size_t n, int* err) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i == 0) *err = 0;
-    if (i < n) pub[i] = make_ulonglong2(kUnset, kUnset);
+    if (i < n) {
+        pub[i] = make_ulonglong2(kUnset, kUnset);
+        vh[i] = make_double2(0.0, 0.0);
+    }
 }
 
 // Sturm counts: numbers of eigenvalues of T(d, e) below x[0..NP) (e2 = e^2), with tiny pivots
@@ -721,125 +730,247 @@ __global__ __launch_bounds__(256) void k_ns_update(const double* __restrict__ Z,
     out[(size_t)j * ldz + r] = acc;
 }
 
-// Y[:, cols] = Q Z[:, cols] = H_0 (H_1 (... H_{m-2} Z)).  One workgroup per kUnmtrWgCols columns,
-// each wavefront holding kUnmtrWaveCols of them in registers (lane l: rows l + 64 q).  The
-// reflectors are staged through LDS in blocks of unmtr_block(NQ) (rows <= k zero, row k+1 one), and the
-// next block's global loads are issued into registers before the current block is applied.
-// NQ: rows per lane (m <= 64 NQ).  One eigenvector per wavefront (40 workgroups for 160 of them):
-// the reflector sequence is latency-bound, and halving each wavefront's dot products, sums and
-// updates per reflector beat two per wavefront by 3 % at m = 164..1000.
-constexpr int kUnmtrWaveCols = 1;
-constexpr int kUnmtrWgCols = 4 * kUnmtrWaveCols;
-// Reflectors per LDS stage (fewer for the larger register sets).
-constexpr int unmtr_block(int nq) { return nq <= 8 ? 8 : 4; }
-
-template <int NQ>
-__global__ __launch_bounds__(256) void k_unmtr(const double2* __restrict__ vh, const double2* __restrict__ tau, int m,
-                                               int nev, const double* __restrict__ Z, int ldz, double2* __restrict__ Y,
-                                               int ldy) {
-    extern __shared__ double2 vs[];  // kUnmtrBlk x m
-    __shared__ double2 ts[8];
-    static_assert(unmtr_block(NQ) <= 8, "ts holds one block's tau values");
-    const int t = (int)threadIdx.x, wv = t >> 6, lane = t & 63;
-    constexpr int kUnmtrRegs = NQ;
-    constexpr int kUnmtrBlk = unmtr_block(NQ);
-    constexpr int kUnmtrPre = kUnmtrBlk * 64 * NQ / 256;  // staged values per thread
-    const int col0 = (int)blockIdx.x * kUnmtrWgCols + wv * kUnmtrWaveCols;
-    double2 y[kUnmtrWaveCols][kUnmtrRegs];
+// The reflectors of A = Q T Q^H in compact form, blocks of kWyNb of them: H_k0 ... H_k1 = I - V T V^H
+// with T upper triangular (T[j][j] = tau_j, T[0:j, j] = -tau_j T[0:j, 0:j] V[:, 0:j]^H v_j), and
+// W = V T, so that a block acts on a vector as y - W (V^H y).  One workgroup per two blocks: the
+// Gram products V^H V on the matrix cores (FP64 16x16x4; both operands are the same registers, lane
+// l holding row l / 16 of a group of four of reflector l % 16), the two triangles by one lane per
+// row, W by one thread per row.  w: column k0 + j holds W_j, its rows up to
+// k0 zero like V's.
+constexpr int kWyNb = 8;
+typedef double wy_v4d __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(256) void k_wy(const double2* __restrict__ vh, const double2* __restrict__ tau, int m,
+                                            double2* __restrict__ w) {
+    __shared__ double2 gs[4][16][17];  // each wavefront's share of V^H V, then their sum in gs[0]
+    __shared__ double2 ts[2][kWyNb][kWyNb];
+    const int t = (int)threadIdx.x, wv = t >> 6, lane = t & 63, l16 = lane & 15, l4 = lane >> 4;
+    const int k0 = (int)blockIdx.x * 2 * kWyNb, nref = m - 1;
+    // Row 0 of every reflector and the column past the last one are zero.
+    const double2* vcol = vh + (size_t)min(k0 + l16, nref) * m;
+    wy_v4d re = {0, 0, 0, 0}, im = {0, 0, 0, 0};
+#pragma unroll 8
+    for (int r0 = k0 + 1 + 4 * wv; r0 < m; r0 += 16) {
+        const double2 v = vcol[r0 + l4 < m ? r0 + l4 : 0];
+        re = __builtin_amdgcn_mfma_f64_16x16x4f64(v.x, v.x, re, 0, 0, 0);
+        im = __builtin_amdgcn_mfma_f64_16x16x4f64(v.x, v.y, im, 0, 0, 0);
+        re = __builtin_amdgcn_mfma_f64_16x16x4f64(v.y, v.y, re, 0, 0, 0);
+        im = __builtin_amdgcn_mfma_f64_16x16x4f64(-v.y, v.x, im, 0, 0, 0);
+    }
+    // D slot r: row l / 16 + 4 r, column l % 16.
 #pragma unroll
-    for (int c = 0; c < kUnmtrWaveCols; ++c)
+    for (int r = 0; r < 4; ++r) gs[wv][l4 + 4 * r][l16] = make_double2(re[r], im[r]);
+    __syncthreads();
+    {
+        const int i = t >> 4, j = t & 15;
+        double2 g = gs[0][i][j];
 #pragma unroll
-        for (int q = 0; q < kUnmtrRegs; ++q) {
-            const int r = lane + 64 * q;
-            y[c][q] = make_double2(r < m && col0 + c < nev ? Z[(size_t)(col0 + c) * ldz + r] : 0.0, 0.0);
+        for (int q = 1; q < 4; ++q) {
+            g.x += gs[q][i][j].x;
+            g.y += gs[q][i][j].y;
         }
-    // Block b holds reflectors klo(b) .. khi(b), applied from khi down; blocks from the bottom up.
-    double2 pre[kUnmtrPre];
-    auto fetch = [&](int khi) {
-        const int klo = khi - kUnmtrBlk + 1 < 0 ? 0 : khi - kUnmtrBlk + 1;
-        const int cnt = (khi - klo + 1) * m;
-#pragma unroll
-        for (int q = 0; q < kUnmtrPre; ++q) {
-            const int idx = t + 256 * q;
-            double2 v = make_double2(0.0, 0.0);
-            if (idx < cnt) {
-                const int sft = idx / m, r = idx - sft * m, k = klo + sft;
-                if (r == k + 1) v = make_double2(1.0, 0.0);
-                else if (r > k + 1) v = vh[(size_t)k * m + r];
-            }
-            pre[q] = v;
-        }
-    };
-    if (m >= 2) fetch(m - 2);
-    for (int khi = m - 2; khi >= 0; khi -= kUnmtrBlk) {
-        const int klo = khi - kUnmtrBlk + 1 < 0 ? 0 : khi - kUnmtrBlk + 1;
-        const int nk = khi - klo + 1;
-        __syncthreads();  // the previous block is consumed
-#pragma unroll
-        for (int q = 0; q < kUnmtrPre; ++q) {
-            const int idx = t + 256 * q;
-            if (idx < nk * m) vs[idx] = pre[q];
-        }
-        if (t < nk) ts[t] = tau[klo + t];
         __syncthreads();
-        if (klo > 0) fetch(klo - 1);
-        for (int sft = nk - 1; sft >= 0; --sft) {
-            const int k = klo + sft;
-            const double2 tk = ts[sft];
-            if (tk.x == 0.0 && tk.y == 0.0) continue;
-            const double2* v = vs + (size_t)sft * m;
-            double acc[2 * kUnmtrWaveCols];
+        gs[0][i][j] = g;
+    }
+    __syncthreads();
+    if (t < 2 * kWyNb) {
+        const int h = t / kWyNb, a = t % kWyNb;  // row a of block h
+        double2 row[kWyNb];
 #pragma unroll
-            for (int c = 0; c < 2 * kUnmtrWaveCols; ++c) acc[c] = 0.0;
+        for (int j = 0; j < kWyNb; ++j) {
+            const int kj = k0 + h * kWyNb + j;
+            const double2 tj = kj < nref ? tau[kj] : make_double2(0.0, 0.0);
+            double2 s = make_double2(0.0, 0.0);
 #pragma unroll
-            for (int q = 0; q < kUnmtrRegs; ++q) {
-                const int r = lane + 64 * q;
-                if (r < m && r > k) {
-                    const double2 vr = v[r];
-#pragma unroll
-                    for (int c = 0; c < kUnmtrWaveCols; ++c) {
-                        const double2 p = cjm(vr, y[c][q]);
-                        acc[2 * c] += p.x;
-                        acc[2 * c + 1] += p.y;
-                    }
-                }
+            for (int b = 0; b < j; ++b) {
+                const double2 u = cm(row[b], gs[0][h * kWyNb + b][h * kWyNb + j]);
+                s.x += u.x;
+                s.y += u.y;
             }
-#pragma unroll
-            for (int c = 0; c < 2 * kUnmtrWaveCols; ++c) acc[c] = wave_sum(acc[c]);
-            double2 tsc[kUnmtrWaveCols];
-#pragma unroll
-            for (int c = 0; c < kUnmtrWaveCols; ++c) tsc[c] = cm(tk, make_double2(acc[2 * c], acc[2 * c + 1]));
-#pragma unroll
-            for (int q = 0; q < kUnmtrRegs; ++q) {
-                const int r = lane + 64 * q;
-                if (r < m && r > k) {
-                    const double2 vr = v[r];
-#pragma unroll
-                    for (int c = 0; c < kUnmtrWaveCols; ++c) {
-                        const double2 u = cm(vr, tsc[c]);
-                        y[c][q].x -= u.x;
-                        y[c][q].y -= u.y;
-                    }
-                }
-            }
+            const double2 u = cm(tj, s);
+            row[j] = a == j ? tj : (a < j ? make_double2(-u.x, -u.y) : make_double2(0.0, 0.0));
+            ts[h][a][j] = row[j];
         }
     }
+    __syncthreads();
+    for (int r = t; r < m; r += 256) {
+        double2 v[2 * kWyNb];
 #pragma unroll
-    for (int c = 0; c < kUnmtrWaveCols; ++c)
+        for (int i = 0; i < 2 * kWyNb; ++i) v[i] = vh[(size_t)min(k0 + i, nref) * m + r];
 #pragma unroll
-        for (int q = 0; q < kUnmtrRegs; ++q) {
-            const int r = lane + 64 * q;
-            if (r < m && col0 + c < nev) Y[(size_t)(col0 + c) * ldy + r] = y[c][q];
-        }
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < kWyNb; ++j) {
+                double2 s = make_double2(0.0, 0.0);
+#pragma unroll
+                for (int i = 0; i <= j; ++i) {
+                    const double2 u = cm(v[h * kWyNb + i], ts[h][i][j]);
+                    s.x += u.x;
+                    s.y += u.y;
+                }
+                const int k = k0 + h * kWyNb + j;
+                if (k < m) w[(size_t)k * m + r] = s;
+            }
+    }
 }
 
-size_t unmtr_lds_bytes(int m) { return (size_t)unmtr_block((m + 63) / 64) * m * sizeof(double2); }
+// Two values' lane exchange and sum (see swap_add): the first value's pairs land in the even lane
+// rows (the lower half), the second's in the odd ones (the upper half).
+template <int ROWS>
+__device__ __forceinline__ double swap_add2(double a, double b) {
+    const unsigned al = (unsigned)__double2loint(a), ah = (unsigned)__double2hiint(a);
+    const unsigned bl = (unsigned)__double2loint(b), bh = (unsigned)__double2hiint(b);
+    if constexpr (ROWS == 1) {
+        const auto l = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
+        return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+    } else {
+        const auto l = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
+        return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+    }
+}
 
-const void* unmtr_kernel(int m) {
-    if (m <= 256) return (const void*)k_unmtr<4>;
-    if (m <= 512) return (const void*)k_unmtr<8>;
-    if (m <= 768) return (const void*)k_unmtr<12>;
-    return (const void*)k_unmtr<16>;
+// Y[:, col] = Q Z[:, col] = H_0 (H_1 (... H_{m-2} Z[:, col])), one workgroup per column, one block of
+// reflectors after another from the last: u = V^H y, y -= W u.  Thread t holds one row of each row
+// group of y; V and W of the next two blocks are in flight while one is applied (all workgroups read
+// a block at about the same time, so its first reader on an XCD waits for memory).  The chain is one workgroup sum per kWyNb reflectors, where one reflector at a time (a
+// wavefront per column) took a wavefront sum each; V and W (16 m^2 bytes between them) stream through
+// every CU from L2, which sets the floor (m = 648: 45 us).  nev = 160, m = 164 / 648:
+// 109 -> 37 us and 918 -> 187 us, k_wy (11 and 30 us) included.
+template <int NQ, int NW>
+struct ApplyQ {
+    static constexpr int GR = 64 * NW;  // rows of one group (one per thread)
+    const double2 *vh, *w;
+    int m;
+    double (*red)[2 * kWyNb][NW];  // [block parity][reflector, real and imaginary][wavefront]
+    int wv, lane;
+    int row[NQ];  // rows from m on read row 0, which is zero in V and W
+    double2 y[NQ];
+    double2 va[kWyNb][NQ], wa[kWyNb][NQ], vb[kWyNb][NQ], wb[kWyNb][NQ];
+
+    // Rows of groups Q0 and up of the block from k0 (columns past the last reflector's are zero).
+    template <int Q0, int Q1>
+    __device__ __forceinline__ void fetch(const double2* src, double2 (&dst)[kWyNb][NQ], int k0) {
+#pragma unroll
+        for (int i = 0; i < kWyNb; ++i) {
+            const double2* c = src + (size_t)min(k0 + i, m - 1) * m;
+#pragma unroll
+            for (int q = Q0; q < Q1; ++q) dst[i][q] = c[row[q]];
+        }
+    }
+
+    template <int Q0, int Q1>
+    __device__ __forceinline__ void load(int kb) {
+        fetch<Q0, Q1>(vh, va, kb + kWyNb);
+        fetch<Q0, Q1>(w, wa, kb + kWyNb);
+        fetch<Q0, Q1>(vh, vb, kb);
+        fetch<Q0, Q1>(w, wb, kb);
+    }
+
+    // One block from its registers, which the block `next` takes over as they fall free.
+    template <int QB>
+    __device__ __forceinline__ void block(double2 (&v)[kWyNb][NQ], double2 (&u)[kWyNb][NQ], int par, int next) {
+        double acc[2 * kWyNb];
+#pragma unroll
+        for (int i = 0; i < kWyNb; ++i) {
+            acc[2 * i] = acc[2 * i + 1] = 0.0;
+#pragma unroll
+            for (int q = QB; q < NQ; ++q) {
+                const double2 p = cjm(v[i][q], y[q]);
+                acc[2 * i] += p.x;
+                acc[2 * i + 1] += p.y;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // the loads below go into registers just read
+        fetch<QB, NQ>(vh, v, next);
+        __builtin_amdgcn_sched_barrier(0);
+        // Sixteen sums at once: halves, then lane rows, hold different values; register i's lane
+        // rows 0..3 end with values 4 i + 0, 2, 1, 3.
+#pragma unroll
+        for (int i = 0; i < kWyNb; ++i) acc[i] = swap_add2<2>(acc[2 * i], acc[2 * i + 1]);
+#pragma unroll
+        for (int i = 0; i < kWyNb / 2; ++i) {
+            double s = swap_add2<1>(acc[2 * i], acc[2 * i + 1]);
+            s += dpp_rot<0x128>(s);
+            s += dpp_rot<0x124>(s);
+            s += dpp_rot<0x122>(s);
+            s += dpp_rot<0x121>(s);
+            acc[i] = s;
+        }
+        const int lr = lane >> 4, first = lr == 1 ? 2 : lr == 2 ? 1 : lr;
+        if ((lane & 15) == 0) {
+#pragma unroll
+            for (int i = 0; i < kWyNb / 2; ++i) red[par][4 * i + first][wv] = acc[i];
+        }
+        __syncthreads();
+        // Lane l adds the wavefronts' shares of value l; every lane then takes them from there.
+        double c = red[par][lane & (2 * kWyNb - 1)][0];
+#pragma unroll
+        for (int q = 1; q < NW; ++q) c += red[par][lane & (2 * kWyNb - 1)][q];
+#pragma unroll
+        for (int i = 0; i < kWyNb; ++i) {
+            const double2 ci = make_double2(read_lane(c, 2 * i), read_lane(c, 2 * i + 1));
+#pragma unroll
+            for (int q = QB; q < NQ; ++q) {
+                const double2 d = cm(u[i][q], ci);
+                y[q].x -= d.x;
+                y[q].y -= d.y;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        fetch<QB, NQ>(w, u, next);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
+    // Pairs of blocks that start in row group QB, from the last; then the groups above it.
+    template <int QB>
+    __device__ __forceinline__ void run(int last) {
+        constexpr int PB = 2 * kWyNb;
+        int kb = min(last, GR * QB + GR - PB);
+        if (kb >= GR * QB) {
+            // Group QB joins here: its rows of the pair already in flight.
+            if (kb == last) load<QB, NQ>(kb);
+            else load<QB, QB + 1>(kb);
+            for (; kb >= GR * QB; kb -= PB) {
+                const int next = max(kb - PB, 0);  // past the last pair: loaded, not used
+                block<QB>(va, wa, 1, next + kWyNb);
+                block<QB>(vb, wb, 0, next);
+            }
+        }
+        if constexpr (QB > 0) run<QB - 1>(last);
+    }
+};
+
+template <int NQ, int NW>
+__global__ __launch_bounds__(64 * NW, 1) void k_apply_q(const double2* __restrict__ vh, const double2* __restrict__ w,
+                                                        int m, const double* __restrict__ Z, int ldz,
+                                                        double2* __restrict__ Y, int ldy) {
+    __shared__ __align__(16) double red[2][2 * kWyNb][NW];
+    const int t = (int)threadIdx.x, col = (int)blockIdx.x;
+    ApplyQ<NQ, NW> k{vh, w, m, red, t >> 6, t & 63};
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int r = t + 64 * NW * q;
+        k.row[q] = r < m ? r : 0;
+        k.y[q] = make_double2(r < m ? Z[(size_t)col * ldz + r] : 0.0, 0.0);
+#pragma unroll
+        for (int i = 0; i < kWyNb; ++i) k.va[i][q] = k.wa[i][q] = k.vb[i][q] = k.wb[i][q] = make_double2(0.0, 0.0);
+    }
+    if (m > 1) k.template run<NQ - 1>((m - 2) / (2 * kWyNb) * 2 * kWyNb);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int r = t + 64 * NW * q;
+        if (r < m) Y[(size_t)col * ldy + r] = k.y[q];
+    }
+}
+
+// The instance and its wavefronts; above 768 rows eight wavefronts hold what four have no registers for.
+const void* apply_q_kernel(int m, int* waves) {
+    *waves = m <= 768 ? 4 : 8;
+    if (m <= 256) return (const void*)k_apply_q<1, 4>;
+    if (m <= 512) return (const void*)k_apply_q<2, 4>;
+    if (m <= 768) return (const void*)k_apply_q<3, 4>;
+    return (const void*)k_apply_q<2, 8>;
 }
 
 size_t stein_lds_bytes(int m) { return (size_t)7 * m * sizeof(double) + (size_t)m; }
@@ -875,7 +1006,6 @@ CoopInfo coop_info(int dev) {
         DZ_REQUIRE(coop != 0, DZHIP_ERR_HIP, "device does not support cooperative launches");
         for (const TrdKernel& k : kTrdKernels) set_max_dynamic_lds(k.fn, k.lds());
         set_max_dynamic_lds((const void*)k_stein, stein_lds_bytes(kHeevMaxM));
-        for (int mm : {256, 512, 768, kHeevMaxM}) set_max_dynamic_lds(unmtr_kernel(mm), unmtr_lds_bytes(kHeevMaxM));
         // Launch-shape override for sweeps: trailing columns per workgroup (4 or 8).
         if (const char* env = std::getenv("DZHIP_HEEV_COLS")) c.cols_per_group = std::max(0, std::atoi(env));
         c.groups = cus;
@@ -974,11 +1104,11 @@ unsigned shared_spin_limit() {
 
 void run_tridiag(const HeevBufs& b, const TrdKernel& k, int G, const double2* A, int lda, int m, hipStream_t s,
                  bool cooperative = true) {
-    // The exchange's entries unset and the error flag cleared by a kernel (not a memset node) on the
+    // The exchange's entries unset, the reflectors zero and the error flag cleared by a kernel (not a memset node) on the
     // same stream.
     const size_t npub = (size_t)m * m;
     hipLaunchKernelGGL(k_trd_init, dim3((unsigned)((npub + 255) / 256)), dim3(256), 0, s,
-                       reinterpret_cast<ulonglong2*>(b.pub), npub, b.err);
+                       reinterpret_cast<ulonglong2*>(b.pub), b.vh, npub, b.err);
     DZ_HIP(hipGetLastError());
     TrdArgs args{A, lda, m, b.vh, b.tau, b.d, b.e, b.pub, b.err, cooperative ? kSpinLimit : shared_spin_limit()};
     void* kargs[] = {&args};
@@ -1010,14 +1140,21 @@ void run_eig(const HeevBufs& b, int m, int nev, double* w_dev, double2* Y, int l
         DZ_HIP(hipGetLastError());
         std::swap(zc, zn);
     }
+    // W takes the exchange buffer, which the tridiagonalisation has done with.
+    double2* wy = reinterpret_cast<double2*>(b.pub);
+    if (m > 1) {
+        hipLaunchKernelGGL(k_wy, dim3((unsigned)((m - 1 + 2 * kWyNb - 1) / (2 * kWyNb))), dim3(256), 0, s, b.vh, b.tau,
+                           m, wy);
+        DZ_HIP(hipGetLastError());
+    }
     {
         const double2* vh = b.vh;
-        const double2* tau = b.tau;
+        const double2* w = wy;
         const double* zcc = zc;
-        int mm = m, nn = nev, ldz = m, ldyy = ldy;
-        void* kargs[] = {&vh, &tau, &mm, &nn, &zcc, &ldz, &Y, &ldyy};
-        DZ_HIP(hipLaunchKernel(unmtr_kernel(m), dim3((unsigned)((nev + kUnmtrWgCols - 1) / kUnmtrWgCols)), dim3(256),
-                               kargs, unmtr_lds_bytes(m), s));
+        int mm = m, ldz = m, ldyy = ldy, waves = 4;
+        const void* fn = apply_q_kernel(m, &waves);
+        void* kargs[] = {&vh, &w, &mm, &zcc, &ldz, &Y, &ldyy};
+        DZ_HIP(hipLaunchKernel(fn, dim3((unsigned)nev), dim3(64u * waves), kargs, 0, s));
     }
     DZ_HIP(hipGetLastError());
 }

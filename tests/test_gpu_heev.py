@@ -50,6 +50,15 @@ def test_heev_register_chunks(ctx, m):
     check(ctx, 0.5 * (g + g.conj().T) + np.diag(np.linspace(0.0, 20.0, m)), min(m, 24))
 
 
+@pytest.mark.parametrize("m", [7, 8, 9, 10, 16, 17, 18, 25, 256, 258, 272, 273, 274, 521, 769])
+def test_heev_reflector_blocks(ctx, m):
+    """Sizes at the edges of the back-transformation's blocks of eight reflectors, of its pairs of
+    blocks and of its 256-row groups; bars as above."""
+    rng = np.random.default_rng(3000 + m)
+    g = rng.standard_normal((m, m)) + 1j * rng.standard_normal((m, m))
+    check(ctx, 0.5 * (g + g.conj().T), min(m, 20))
+
+
 def test_heev_degenerate_and_clustered(ctx):
     """Exactly degenerate triplets and pairs (symmetry-degenerate bands), a cluster split by
     1e-13, and a zero off-diagonal block (a reducible tridiagonal)."""
