@@ -9,8 +9,8 @@
 //      launch it cooperatively; the solvers' Rayleigh-Ritz step launches it as an ordinary
 //      dispatch admitted by the device's tridiagonalisation gate (TrdAdmission), so that the
 //      grids of concurrent solves on different streams run side by side.
-//   2. The lowest nev eigenvalues of T by 64-way multisection with Sturm counts (one wavefront
-//      per eigenvalue).
+//   2. The lowest nev eigenvalues of T by 257-way multisection with Sturm counts (one workgroup
+//      per eigenvalue) and, in the same launch, the reflectors' compact form for stage 4.
 //   3. Eigenvectors of T by inverse iteration (tridiagonal LU with partial pivoting in LDS, one
 //      wavefront per eigenvalue); the members of a cluster of eigenvalues closer than a threshold
 //      are then orthonormalised together (two classical Gram-Schmidt passes), and two

@@ -420,47 +420,78 @@ __global__ __launch_bounds__(256) void k_trd_init(ulonglong2* pub, double2* vh, 
     }
 }
 
-// Sturm counts: numbers of eigenvalues of T(d, e) below x[0..NP) (e2 = e^2), with tiny pivots
-// replaced by -pivmin (LAPACK dlaebz's rule).  The NP recurrences are independent and interleaved.
-template <int NP>
-__device__ __forceinline__ void sturm_counts(const double* d, const double* e2, int m, const double (&x)[NP],
-                                             double pivmin, int (&cnt)[NP]) {
-    double q[NP];
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-        q[p] = d[0] - x[p];
-        if (fabs(q[p]) < pivmin) q[p] = -pivmin;
-        cnt[p] = q[p] < 0.0 ? 1 : 0;
+// Number of eigenvalues of T below x from a factorisation twisted at row h = (m - 1) / 2: pivots
+// q_i = d_i - x - e_{i-1}^2 / q_{i-1} down from the top, r_i = d_i - x - e_i^2 / r_{i+1} up from the
+// bottom, and g = d_h - x - e_{h-1}^2 / q_{h-1} - e_h^2 / r_{h+1}; by Sylvester's law of inertia as
+// many eigenvalues lie below x as pivots are negative.  The two recurrences are independent, so the
+// chain is half as long as one recurrence over all rows.  de: (d_i, e_i^2), e_{m-1} = 0.  Quotients
+// come from the hardware's reciprocal with one third-order Newton step and no test for small
+// pivots; one (tiny or zero) that overflows turns its recurrence into NaN within a step, and those
+// kSturmBlock rows are done again with divisions and pivots raised to pivmin (LAPACK dlaebz's rule).
+constexpr int kSturmBlock = 8;
+struct SturmState {
+    double f, b;  // e^2 / q and e^2 / r to subtract from the next rows
+    int cnt;
+};
+template <bool SAFE>
+__device__ __forceinline__ void sturm_step(double pivot_in, double e2, double pivmin, double* out, int* cnt) {
+    double q = pivot_in;
+    if (SAFE) {
+        if (fabs(q) < pivmin) q = -pivmin;
+        *out = e2 / q;
+    } else {
+        const double r = __builtin_amdgcn_rcp(q), t = e2 * r, e = fma(-q, r, 1.0);
+        *out = fma(t, fma(e, e, e), t);
     }
-    for (int k = 1; k < m; ++k) {
-        const double dk = d[k], ek = e2[k - 1];
+    *cnt += (int)((unsigned)__double2hiint(q) >> 31);
+}
+template <bool SAFE>
+__device__ __forceinline__ void sturm_rows(const double2* de, int m, int s, double x, double pivmin, SturmState& st) {
+    const double2 a = de[s], c = de[m - 1 - s];
+    sturm_step<SAFE>(a.x - x - st.f, a.y, pivmin, &st.f, &st.cnt);
+    sturm_step<SAFE>(c.x - x - st.b, de[m - 2 - s].y, pivmin, &st.b, &st.cnt);
+}
+__device__ __forceinline__ int sturm_count(const double2* de, int m, double x, double pivmin) {
+    const int h = (m - 1) / 2;
+    SturmState st{0.0, 0.0, 0};
+    for (int s = 0; s < h; s += kSturmBlock) {
+        const SturmState st0 = st;
+        const int n = min(kSturmBlock, h - s);
+        if (n == kSturmBlock) {
 #pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            q[p] = dk - x[p] - ek / q[p];
-            if (fabs(q[p]) < pivmin) q[p] = -pivmin;
-            cnt[p] += q[p] < 0.0 ? 1 : 0;
+            for (int k = 0; k < kSturmBlock; ++k) sturm_rows<false>(de, m, s + k, x, pivmin, st);
+        } else {
+            for (int k = 0; k < n; ++k) sturm_rows<false>(de, m, s + k, x, pivmin, st);
+        }
+        if (__any(st.f != st.f || st.b != st.b)) {
+            st = st0;
+            for (int k = 0; k < n; ++k) sturm_rows<true>(de, m, s + k, x, pivmin, st);
         }
     }
+    if (m - 1 - h > h) sturm_step<true>(de[h + 1].x - x - st.b, de[h].y, pivmin, &st.b, &st.cnt);
+    double unused;
+    sturm_step<true>(de[h].x - x - st.f - st.b, 0.0, pivmin, &unused, &st.cnt);
+    return st.cnt;
 }
 
-// Eigenvalue idx (ascending) of T by multisection: each round the 64 lanes of a wavefront count
-// at NP points each (64 NP interior points of [lo, hi]) and keep the sub-interval that holds
-// eigenvalue idx.  Also writes the Gershgorin scale of T to scal[0] (block 0).
-__global__ __launch_bounds__(256) void k_stebz(const double* __restrict__ d_in, const double* __restrict__ e_in, int m,
-                                               int nev, double* __restrict__ w, double* __restrict__ scal,
-                                               const int* __restrict__ err) {
-    extern __shared__ double sh[];
-    double* d = sh;
-    double* e2 = sh + m;
+// Eigenvalue blockIdx.x (ascending) of T by multisection: each round the workgroup's 256 lanes count
+// at 256 interior points of [lo, hi] and keep the sub-interval that holds the eigenvalue; seven
+// rounds reach the last bits, where 64 points took nine.  The FP64 issue rate bounds it, one
+// wavefront per SIMD.  Also writes the Gershgorin scale of T to scal[0] (block 0).  nev = 160, one
+// wavefront per eigenvalue, one recurrence and divisions before: m = 164 / 648 113 -> 65 us,
+// 418 -> 228 us, the reflectors' compact form (11 and 30 us before) included.
+__device__ __forceinline__ void stebz(const double* __restrict__ d_in, const double* __restrict__ e_in, int m,
+                                      double* __restrict__ w, double* __restrict__ scal, const int* __restrict__ err,
+                                      double2* de) {
     __shared__ double red[4 * 3];
-    const int t = (int)threadIdx.x;
+    __shared__ int s_low[2][4];
+    const int t = (int)threadIdx.x, idx = (int)blockIdx.x;
     double lo_l = 1e300, hi_l = -1e300, e2max = 0.0;
     for (int k = t; k < m; k += 256) {
         const double dk = d_in[k];
         const double el = k > 0 ? fabs(e_in[k - 1]) : 0.0;
         const double er = k + 1 < m ? fabs(e_in[k]) : 0.0;
-        d[k] = dk;
-        e2[k] = k + 1 < m ? e_in[k] * e_in[k] : 0.0;
+        de[k] = make_double2(dk, er * er);
         lo_l = fmin(lo_l, dk - el - er);
         hi_l = fmax(hi_l, dk + el + er);
         e2max = fmax(e2max, er * er);
@@ -490,46 +521,133 @@ __global__ __launch_bounds__(256) void k_stebz(const double* __restrict__ d_in, 
     const double wid = 2.220446049250313e-16 * 4.0 * bnorm + 2.0 * pivmin + 1e-300;
     gl -= wid + 1e-14 * (gu - gl);
     gu += wid + 1e-14 * (gu - gl);
-    if (blockIdx.x == 0 && t == 0) scal[0] = bnorm;
-    const int lane = t & 63;
-    const int idx = (int)blockIdx.x * 4 + (t >> 6);
-    if (idx >= nev) return;
+    if (idx == 0 && t == 0) scal[0] = bnorm;
     // A tridiagonalisation whose exchange did not complete leaves NaN eigenvalues (the signal
     // a caller without a synchronising check sees).
     if (*err != 0) {
-        if (lane == 0) w[idx] = __builtin_nan("");
+        if (t == 0) w[idx] = __builtin_nan("");
         return;
     }
-    constexpr int NP = 1;  // more points per lane lose: the FP64 divisions bound the issue rate
-    constexpr double kParts = 64.0 * NP + 1.0;
+    constexpr double kParts = 257.0;
     double lo = gl, hi = gu;
     for (int round = 0; round < 14; ++round) {
         const double width = hi - lo;
-        if (width <= 2.0 * 2.220446049250313e-16 * fmax(fabs(lo), fabs(hi)) + 2.0 * pivmin) break;
-        double x[NP];
-        int cnt[NP];
-#pragma unroll
-        for (int p = 0; p < NP; ++p) x[p] = lo + width * (double)(lane * NP + p + 1) / kParts;
-        sturm_counts<NP>(d, e2, m, x, pivmin, cnt);
-        // Highest point (lane * NP + p) that still has eigenvalue idx at or above it; -1 if none.
+        if (!(width > 2.0 * 2.220446049250313e-16 * fmax(fabs(lo), fabs(hi)) + 2.0 * pivmin)) break;
+        const int cnt = sturm_count(de, m, lo + width * (double)(t + 1) / kParts, pivmin);
+        // Highest point that still has the eigenvalue at or above it; -1 if none.
+        const unsigned long long below = __ballot(cnt <= idx);
+        if ((t & 63) == 0) s_low[round & 1][t >> 6] = below ? (t | (63 - __builtin_clzll(below))) : -1;
+        __syncthreads();
         int L = -1;
 #pragma unroll
-        for (int p = 0; p < NP; ++p)
-            if (cnt[p] <= idx) L = lane * NP + p;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) L = max(L, __shfl_xor(L, o, 64));
+        for (int q = 0; q < 4; ++q) L = max(L, s_low[round & 1][q]);
         double nlo = lo, nhi = hi;
         if (L < 0) {
             nhi = lo + width * 1.0 / kParts;
         } else {
             nlo = lo + width * (double)(L + 1) / kParts;
-            if (L < 64 * NP - 1) nhi = lo + width * (double)(L + 2) / kParts;
+            if (L < 255) nhi = lo + width * (double)(L + 2) / kParts;
         }
         lo = nlo;
         hi = nhi;
     }
-    if (lane == 0) w[idx] = 0.5 * (lo + hi);
+    if (t == 0) w[idx] = 0.5 * (lo + hi);
 }
+
+// The reflectors of A = Q T Q^H in compact form, blocks of kWyNb of them: H_k0 ... H_k1 = I - V T V^H
+// with T upper triangular (T[j][j] = tau_j, T[0:j, j] = -tau_j T[0:j, 0:j] V[:, 0:j]^H v_j), and
+// W = V T, so that a block acts on a vector as y - W (V^H y).  One workgroup per two blocks: the
+// Gram products V^H V on the matrix cores (FP64 16x16x4; both operands are the same registers, lane
+// l holding row l / 16 of a group of four of reflector l % 16), the two triangles by one lane per
+// row, W by one thread per row.  w: column k0 + j holds W_j, its rows up to
+// k0 zero like V's.
+constexpr int kWyNb = 8;
+typedef double wy_v4d __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void compact_reflectors(const double2* __restrict__ vh, const double2* __restrict__ tau, int m,
+                                                   double2* __restrict__ w, int group, double2* lds) {
+    auto gs = reinterpret_cast<double2(*)[16][17]>(lds);  // each wavefront's share of V^H V, then their sum in gs[0]
+    __shared__ double2 ts[2][kWyNb][kWyNb];
+    const int t = (int)threadIdx.x, wv = t >> 6, lane = t & 63, l16 = lane & 15, l4 = lane >> 4;
+    const int k0 = group * 2 * kWyNb, nref = m - 1;
+    // Row 0 of every reflector and the column past the last one are zero.
+    const double2* vcol = vh + (size_t)min(k0 + l16, nref) * m;
+    wy_v4d re = {0, 0, 0, 0}, im = {0, 0, 0, 0};
+#pragma unroll 8
+    for (int r0 = k0 + 1 + 4 * wv; r0 < m; r0 += 16) {
+        const double2 v = vcol[r0 + l4 < m ? r0 + l4 : 0];
+        re = __builtin_amdgcn_mfma_f64_16x16x4f64(v.x, v.x, re, 0, 0, 0);
+        im = __builtin_amdgcn_mfma_f64_16x16x4f64(v.x, v.y, im, 0, 0, 0);
+        re = __builtin_amdgcn_mfma_f64_16x16x4f64(v.y, v.y, re, 0, 0, 0);
+        im = __builtin_amdgcn_mfma_f64_16x16x4f64(-v.y, v.x, im, 0, 0, 0);
+    }
+    // D slot r: row l / 16 + 4 r, column l % 16.
+#pragma unroll
+    for (int r = 0; r < 4; ++r) gs[wv][l4 + 4 * r][l16] = make_double2(re[r], im[r]);
+    __syncthreads();
+    {
+        const int i = t >> 4, j = t & 15;
+        double2 g = gs[0][i][j];
+#pragma unroll
+        for (int q = 1; q < 4; ++q) {
+            g.x += gs[q][i][j].x;
+            g.y += gs[q][i][j].y;
+        }
+        __syncthreads();
+        gs[0][i][j] = g;
+    }
+    __syncthreads();
+    if (t < 2 * kWyNb) {
+        const int h = t / kWyNb, a = t % kWyNb;  // row a of block h
+        double2 row[kWyNb];
+#pragma unroll
+        for (int j = 0; j < kWyNb; ++j) {
+            const int kj = k0 + h * kWyNb + j;
+            const double2 tj = kj < nref ? tau[kj] : make_double2(0.0, 0.0);
+            double2 s = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int b = 0; b < j; ++b) {
+                const double2 u = cm(row[b], gs[0][h * kWyNb + b][h * kWyNb + j]);
+                s.x += u.x;
+                s.y += u.y;
+            }
+            const double2 u = cm(tj, s);
+            row[j] = a == j ? tj : (a < j ? make_double2(-u.x, -u.y) : make_double2(0.0, 0.0));
+            ts[h][a][j] = row[j];
+        }
+    }
+    __syncthreads();
+    for (int r = t; r < m; r += 256) {
+        double2 v[2 * kWyNb];
+#pragma unroll
+        for (int i = 0; i < 2 * kWyNb; ++i) v[i] = vh[(size_t)min(k0 + i, nref) * m + r];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < kWyNb; ++j) {
+                double2 s = make_double2(0.0, 0.0);
+#pragma unroll
+                for (int i = 0; i <= j; ++i) {
+                    const double2 u = cm(v[h * kWyNb + i], ts[h][i][j]);
+                    s.x += u.x;
+                    s.y += u.y;
+                }
+                const int k = k0 + h * kWyNb + j;
+                if (k < m) w[(size_t)k * m + r] = s;
+            }
+    }
+}
+
+// The eigenvalues of T (blocks 0..nev-1) and, beside them because neither needs the other, the
+// compact form of the reflectors (the blocks after them).
+__global__ __launch_bounds__(256) void k_stebz(const double* __restrict__ d_in, const double* __restrict__ e_in, int m,
+                                               int nev, double* __restrict__ w, double* __restrict__ scal,
+                                               const int* __restrict__ err, const double2* __restrict__ vh,
+                                               const double2* __restrict__ tau, double2* __restrict__ wy) {
+    extern __shared__ double2 sh2[];
+    if ((int)blockIdx.x < nev) stebz(d_in, e_in, m, w, scal, err, sh2);
+    else compact_reflectors(vh, tau, m, wy, (int)blockIdx.x - nev, sh2);
+}
+constexpr int kWyLds = 4 * 16 * 17 * (int)sizeof(double2);
 
 // Eigenvalues closer than this (consecutive gaps, relative to the Gershgorin scale) form a cluster
 // whose inverse-iteration vectors are orthonormalised together.
@@ -730,89 +848,6 @@ __global__ __launch_bounds__(256) void k_ns_update(const double* __restrict__ Z,
     out[(size_t)j * ldz + r] = acc;
 }
 
-// The reflectors of A = Q T Q^H in compact form, blocks of kWyNb of them: H_k0 ... H_k1 = I - V T V^H
-// with T upper triangular (T[j][j] = tau_j, T[0:j, j] = -tau_j T[0:j, 0:j] V[:, 0:j]^H v_j), and
-// W = V T, so that a block acts on a vector as y - W (V^H y).  One workgroup per two blocks: the
-// Gram products V^H V on the matrix cores (FP64 16x16x4; both operands are the same registers, lane
-// l holding row l / 16 of a group of four of reflector l % 16), the two triangles by one lane per
-// row, W by one thread per row.  w: column k0 + j holds W_j, its rows up to
-// k0 zero like V's.
-constexpr int kWyNb = 8;
-typedef double wy_v4d __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(256) void k_wy(const double2* __restrict__ vh, const double2* __restrict__ tau, int m,
-                                            double2* __restrict__ w) {
-    __shared__ double2 gs[4][16][17];  // each wavefront's share of V^H V, then their sum in gs[0]
-    __shared__ double2 ts[2][kWyNb][kWyNb];
-    const int t = (int)threadIdx.x, wv = t >> 6, lane = t & 63, l16 = lane & 15, l4 = lane >> 4;
-    const int k0 = (int)blockIdx.x * 2 * kWyNb, nref = m - 1;
-    // Row 0 of every reflector and the column past the last one are zero.
-    const double2* vcol = vh + (size_t)min(k0 + l16, nref) * m;
-    wy_v4d re = {0, 0, 0, 0}, im = {0, 0, 0, 0};
-#pragma unroll 8
-    for (int r0 = k0 + 1 + 4 * wv; r0 < m; r0 += 16) {
-        const double2 v = vcol[r0 + l4 < m ? r0 + l4 : 0];
-        re = __builtin_amdgcn_mfma_f64_16x16x4f64(v.x, v.x, re, 0, 0, 0);
-        im = __builtin_amdgcn_mfma_f64_16x16x4f64(v.x, v.y, im, 0, 0, 0);
-        re = __builtin_amdgcn_mfma_f64_16x16x4f64(v.y, v.y, re, 0, 0, 0);
-        im = __builtin_amdgcn_mfma_f64_16x16x4f64(-v.y, v.x, im, 0, 0, 0);
-    }
-    // D slot r: row l / 16 + 4 r, column l % 16.
-#pragma unroll
-    for (int r = 0; r < 4; ++r) gs[wv][l4 + 4 * r][l16] = make_double2(re[r], im[r]);
-    __syncthreads();
-    {
-        const int i = t >> 4, j = t & 15;
-        double2 g = gs[0][i][j];
-#pragma unroll
-        for (int q = 1; q < 4; ++q) {
-            g.x += gs[q][i][j].x;
-            g.y += gs[q][i][j].y;
-        }
-        __syncthreads();
-        gs[0][i][j] = g;
-    }
-    __syncthreads();
-    if (t < 2 * kWyNb) {
-        const int h = t / kWyNb, a = t % kWyNb;  // row a of block h
-        double2 row[kWyNb];
-#pragma unroll
-        for (int j = 0; j < kWyNb; ++j) {
-            const int kj = k0 + h * kWyNb + j;
-            const double2 tj = kj < nref ? tau[kj] : make_double2(0.0, 0.0);
-            double2 s = make_double2(0.0, 0.0);
-#pragma unroll
-            for (int b = 0; b < j; ++b) {
-                const double2 u = cm(row[b], gs[0][h * kWyNb + b][h * kWyNb + j]);
-                s.x += u.x;
-                s.y += u.y;
-            }
-            const double2 u = cm(tj, s);
-            row[j] = a == j ? tj : (a < j ? make_double2(-u.x, -u.y) : make_double2(0.0, 0.0));
-            ts[h][a][j] = row[j];
-        }
-    }
-    __syncthreads();
-    for (int r = t; r < m; r += 256) {
-        double2 v[2 * kWyNb];
-#pragma unroll
-        for (int i = 0; i < 2 * kWyNb; ++i) v[i] = vh[(size_t)min(k0 + i, nref) * m + r];
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int j = 0; j < kWyNb; ++j) {
-                double2 s = make_double2(0.0, 0.0);
-#pragma unroll
-                for (int i = 0; i <= j; ++i) {
-                    const double2 u = cm(v[h * kWyNb + i], ts[h][i][j]);
-                    s.x += u.x;
-                    s.y += u.y;
-                }
-                const int k = k0 + h * kWyNb + j;
-                if (k < m) w[(size_t)k * m + r] = s;
-            }
-    }
-}
-
 // Two values' lane exchange and sum (see swap_add): the first value's pairs land in the even lane
 // rows (the lower half), the second's in the odd ones (the upper half).
 template <int ROWS>
@@ -836,7 +871,7 @@ __device__ __forceinline__ double swap_add2(double a, double b) {
 // a block at about the same time, so its first reader on an XCD waits for memory).  The chain is one workgroup sum per kWyNb reflectors, where one reflector at a time (a
 // wavefront per column) took a wavefront sum each; V and W (16 m^2 bytes between them) stream through
 // every CU from L2, which sets the floor (m = 648: 45 us).  nev = 160, m = 164 / 648:
-// 109 -> 37 us and 918 -> 187 us, k_wy (11 and 30 us) included.
+// 109 -> 26 us and 918 -> 157 us (and the compact form, 11 and 30 us alone, beside the eigenvalues).
 template <int NQ, int NW>
 struct ApplyQ {
     static constexpr int GR = 64 * NW;  // rows of one group (one per thread)
@@ -1121,8 +1156,11 @@ void run_tridiag(const HeevBufs& b, const TrdKernel& k, int G, const double2* A,
 
 void run_eig(const HeevBufs& b, int m, int nev, double* w_dev, double2* Y, int ldy, hipStream_t s) {
     double* scal = b.gram + (size_t)nev * nev;
-    hipLaunchKernelGGL(k_stebz, dim3((unsigned)((nev + 3) / 4)), dim3(256), 2 * m * sizeof(double), s, b.d, b.e, m,
-                       nev, w_dev, scal, b.err);
+    // W takes the exchange buffer, which the tridiagonalisation has done with.
+    double2* wy = reinterpret_cast<double2*>(b.pub);
+    const int groups = (m - 1 + 2 * kWyNb - 1) / (2 * kWyNb);
+    hipLaunchKernelGGL(k_stebz, dim3((unsigned)(nev + groups)), dim3(256), std::max(m * (int)sizeof(double2), kWyLds), s,
+                       b.d, b.e, m, nev, w_dev, scal, b.err, b.vh, b.tau, wy);
     DZ_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_stein, dim3((unsigned)nev), dim3(64), stein_lds_bytes(m), s, b.d, b.e, m, nev, w_dev, scal,
                        b.z, m);
@@ -1139,13 +1177,6 @@ void run_eig(const HeevBufs& b, int m, int nev, double* w_dev, double2* Y, int l
                            nev, b.gram, zn);
         DZ_HIP(hipGetLastError());
         std::swap(zc, zn);
-    }
-    // W takes the exchange buffer, which the tridiagonalisation has done with.
-    double2* wy = reinterpret_cast<double2*>(b.pub);
-    if (m > 1) {
-        hipLaunchKernelGGL(k_wy, dim3((unsigned)((m - 1 + 2 * kWyNb - 1) / (2 * kWyNb))), dim3(256), 0, s, b.vh, b.tau,
-                           m, wy);
-        DZ_HIP(hipGetLastError());
     }
     {
         const double2* vh = b.vh;
