@@ -1404,35 +1404,57 @@ void launch_xline_conv(Ham& h, typename C2T<T>::type* tb, size_t nc, hipStream_t
     DZ_HIP(hipGetLastError());
 }
 
-// Workgroup tiles of the nonlocal GEMMs: 10 wavefronts = 5 band groups of 32 bands x 2 halves
-// of the projector (projection) or G (back-projection) tile, so one workgroup covers a 160-band
-// block, each projector row is read once per K-chunk, and two workgroups fit on a CU with the
-// wavefronts spread evenly over its four SIMDs.
-constexpr int kNlBandGroups = 5;
-constexpr int kNlWaves = 2 * kNlBandGroups;
-constexpr int kNlThreads = 64 * kNlWaves;
-constexpr int kNlBands = 32 * kNlBandGroups;  // bands per workgroup tile
-constexpr int kNlK = 32;                 // K (G or p) per LDS stage
-constexpr int kNlPitch = kNlK + 1;       // odd pitches (in complex elements) against bank conflicts
-// 16-wide MFMA blocks per workgroup tile along the projector (projection) and G
-// (back-projection) axes, split over the two wavefront halves: 4 in FP32; 2 in FP64, whose
-// accumulators are twice as wide.
-template <typename T> struct NlTile { static constexpr int kBlocks = 4; };
-template <> struct NlTile<double> { static constexpr int kBlocks = 2; };
-template <typename T> constexpr int nl_p_tile() { return 16 * NlTile<T>::kBlocks; }  // projectors / tile
-// Back-projection G tiles of two 16-wide blocks (one per wavefront half): at the bench size 746
-// tiles of 32 G even out the work per CU better than 373 tiles of 64 G on 256 CUs (two
-// workgroups fit per CU either way).
-template <typename T> struct NlBackTile { static constexpr int kBlocks = 2; };
-template <typename T> constexpr int nl_g_tile() { return 16 * NlBackTile<T>::kBlocks; }  // G / tile
+// Workgroup tiles of the nonlocal GEMMs: WB x WX wavefronts, each with BBW blocks of 16 bands and one
+// 16-wide block of projectors (projection) or G (back-projection), so that a tile holds the bands a
+// call has (16 BBW WB of them, up to 160: a projector row is read once per K-chunk) and its
+// wavefronts spread evenly over the four SIMDs.  K runs in stages of kNlK through two LDS buffers:
+// the next stage's loads are in flight while one is multiplied, and one barrier per stage suffices.
+// Ten wavefronts of 32 bands for every call, whose loads were masked (so waited for) before the
+// products, left SIMDs uneven (three against two wavefronts) at 160 bands and multiplied padding below.
+// Projection / back-projection: Si-64 FP64 (160 bands, 256 projectors) 151 / 151 -> 119 / 131 us
+// (matrix-core floor 75), FP32 77 / 91 -> 66 / 68; 12 bands of 36 Al-4 k-points 44 / 43 -> 9 / 7;
+// 37 bands, 112 projectors, 8,334 plane waves 30 / 47 -> 17 / 23; one band of Si-8 8.6 / 8.4 -> 3.9 / 4.2.
+constexpr int kNlMaxBlocks = 10;  // 16-band blocks per workgroup tile
+constexpr int kNlK = 16;          // K (G or p) per LDS stage
+constexpr int kNlPitch = kNlK + 1;  // odd pitches (in complex elements) against bank conflicts
+constexpr int kNlBackK = 8;       // the same for the back-projection: two workgroups' LDS fit a CU; 32 at
+                                  // few bands was slower (37 bands, 112 projectors 23 -> 29 us)
+constexpr int kNlGWaves = 2;      // wavefronts along G: 32-wide tiles even out the work per CU (Si-64: 750)
+constexpr int kNlG = 16 * kNlGWaves;
+
+// Split of a projection: btiles tiles of `blocks` 16-band blocks, ptiles tiles of 16 wx projectors,
+// nks K-chunks.  One workgroup of eight wavefronts per CU, two of four.  Every K-chunk is a multiple
+// of two stages.  A function of the sizes of one k-point alone, so that a set of k-points repeats it.
+struct NlShape {
+    int blocks, btiles, wx, ptiles, nks, kchunk;
+};
+static NlShape nl_shape(int P, int npw, int ncols) {
+    NlShape s;
+    const int nbk = (ncols + 15) / 16;
+    s.btiles = std::max(1, (nbk + kNlMaxBlocks - 1) / kNlMaxBlocks);
+    const int need = (nbk + s.btiles - 1) / s.btiles;
+    for (int b : {1, 2, 3, 5, 8, 10})
+        if (need <= b) {
+            s.blocks = b;
+            break;
+        }
+    s.wx = P <= 32 ? 2 : 4;
+    s.ptiles = std::max(1, (P + 16 * s.wx - 1) / (16 * s.wx));
+    const int tiles = s.ptiles * s.btiles, ktiles = (npw + 2 * kNlK - 1) / (2 * kNlK);
+    const int want = s.blocks > 5 ? 256 : 512;
+    s.nks = std::max(1, std::min(ktiles, (want + tiles - 1) / tiles));
+    s.kchunk = (int)round_up((npw + s.nks - 1) / s.nks, 2 * kNlK);
+    s.nks = (npw + s.kchunk - 1) / s.kchunk;
+    return s;
+}
 
 template <typename T>
-__host__ __device__ inline size_t nl_proj_lds_bytes() {
-    return (size_t)(kNlBands + nl_p_tile<T>()) * kNlPitch * sizeof(typename C2T<T>::type);
+__host__ __device__ constexpr size_t nl_proj_lds_bytes(int blocks, int wx) {
+    return (size_t)2 * 16 * (blocks + wx) * kNlPitch * sizeof(typename C2T<T>::type);
 }
 template <typename T>
-__host__ __device__ inline size_t nl_back_lds_bytes() {
-    return ((size_t)kNlBands * kNlPitch + (size_t)kNlK * (nl_g_tile<T>() + 1)) * sizeof(typename C2T<T>::type);
+__host__ __device__ constexpr size_t nl_back_lds_bytes(int blocks) {
+    return (size_t)2 * (16 * blocks * (kNlBackK + 1) + kNlBackK * (kNlG + 1)) * sizeof(typename C2T<T>::type);
 }
 
 // Block index -> logical tile so that consecutive logical tiles (which share operands)
@@ -1445,23 +1467,22 @@ __device__ __forceinline__ int xcd_tile(int bid, int nblocks) {
 }
 
 // partial[ks][b][p] = sum_{G in chunk ks} X[b][G] * A[p][G]   (= <beta_p|psi_b>, no 1/Omega yet)
-template <typename T>
-__global__ __launch_bounds__(kNlThreads) void k_nl_proj(const typename C2T<T>::type* __restrict__ a,
-                                                        const typename C2T<T>::type* __restrict__ x,
-                                                        size_t ldx, typename C2T<T>::type* __restrict__ partial,
-                                                        int P, int npw, int ncols, int kchunk, int ptiles,
-                                                        const int2* __restrict__ chunks, int lda) {
+template <typename T, int BBW, int WB, int WX>
+__global__ __launch_bounds__(64 * WB * WX) void k_nl_proj(const typename C2T<T>::type* __restrict__ a,
+                                                          const typename C2T<T>::type* __restrict__ x,
+                                                          size_t ldx, typename C2T<T>::type* __restrict__ partial,
+                                                          int P, int npw, int ncols, int kchunk, int ptiles,
+                                                          const int2* __restrict__ chunks, int lda) {
     using C = typename C2T<T>::type;
     using M = Mfma<T>;
+    constexpr int NT = 64 * WB * WX, XR = 16 * BBW * WB, AR = 16 * WX;
     extern __shared__ unsigned char smem_raw[];
-    C* xs = reinterpret_cast<C*>(smem_raw);  // [kNlBands][kNlPitch]
-    constexpr int kNlP = nl_p_tile<T>();
-    constexpr int PB = NlTile<T>::kBlocks / 2;  // projector blocks per wavefront
-    C* as = xs + kNlBands * kNlPitch;        // [kNlP][kNlPitch]
+    C* const lds = reinterpret_cast<C*>(smem_raw);  // two stages of [XR + AR rows][kNlPitch]
+    constexpr int kStage = (XR + AR) * kNlPitch;
     const int lin = xcd_tile(blockIdx.x, gridDim.x);
     const int pt = lin % ptiles, ks = lin / ptiles;
-    const int p0 = pt * kNlP;
-    const int b0 = blockIdx.z * kNlBands;
+    const int p0 = pt * AR;
+    const int b0 = blockIdx.z * XR;
     // G range of K-chunk ks: a fixed-size split of one context's sphere, or (batched apply over
     // several k-points, G of all k-points concatenated) the chunk table's range within one k-point.
     int k0 = ks * kchunk, k1 = min(npw, ks * kchunk + kchunk);
@@ -1471,112 +1492,92 @@ __global__ __launch_bounds__(kNlThreads) void k_nl_proj(const typename C2T<T>::t
         k1 = ck.y;
     }
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int bg = wave % kNlBandGroups, half = wave / kNlBandGroups;
+    const int wb = wave % WB, wx = wave / WB;
     const int i16 = lane & 15, k4 = lane >> 4;
-    const C zero = C{T(0), T(0)};
-    constexpr int kXPer = (kNlBands * kNlK + kNlThreads - 1) / kNlThreads;
-    constexpr int kAPer = (kNlP * kNlK + kNlThreads - 1) / kNlThreads;
-    T xre[kXPer], xim[kXPer], are[kAPer], aim[kAPer];
-#define DZ_PROJ_FETCH(KT)                                                                     \
-    _Pragma("unroll") for (int i = 0; i < kXPer; ++i) {                                      \
-        const int e = tid + i * kNlThreads;                                                   \
-        const int r = e >> 5, c = e & 31, g = (KT) + c, b = b0 + r;                           \
-        const bool ok = r < kNlBands && b < ncols && g < k1;                                  \
-        const C v = x[ok ? (size_t)b * ldx + g : 0];                                          \
-        xre[i] = ok ? v.x : T(0);                                                             \
-        xim[i] = ok ? v.y : T(0);                                                             \
-    }                                                                                         \
-    _Pragma("unroll") for (int i = 0; i < kAPer; ++i) {                                      \
-        const int e = tid + i * kNlThreads;                                                   \
-        const int r = e >> 5, c = e & 31, g = (KT) + c, p = p0 + r;                           \
-        const bool ok = r < kNlP && p < P && g < k1;                                          \
-        const C v = a[ok ? (size_t)p * lda + g : 0];                                          \
-        are[i] = ok ? v.x : T(0);                                                             \
-        aim[i] = ok ? v.y : T(0);                                                             \
-    }
-#define DZ_PROJ_STASH()                                                                       \
-    _Pragma("unroll") for (int i = 0; i < kXPer; ++i) {                                      \
-        const int e = tid + i * kNlThreads;                                                   \
-        if (e < kNlBands * kNlK) xs[(e >> 5) * kNlPitch + (e & 31)] = C{xre[i], xim[i]};     \
-    }                                                                                         \
-    _Pragma("unroll") for (int i = 0; i < kAPer; ++i) {                                      \
-        const int e = tid + i * kNlThreads;                                                   \
-        if (e < kNlP * kNlK) as[(e >> 5) * kNlPitch + (e & 31)] = C{are[i], aim[i]};         \
-    }
+    constexpr int kXPer = (XR * kNlK + NT - 1) / NT, kAPer = (AR * kNlK + NT - 1) / NT;
+    // Loads take whatever lies at a clamped address and nothing looks at them before the stage they
+    // overlap with is multiplied: rows beyond the last band or projector only feed results that are
+    // not stored, and K beyond the chunk is zeroed on its way to LDS.
+    C xr[kXPer], ar[kAPer];
+    auto fetch = [&](int kt) {
+#pragma unroll
+        for (int i = 0; i < kXPer; ++i) {
+            const int e = tid + i * NT;
+            xr[i] = x[(size_t)min(b0 + e / kNlK, ncols - 1) * ldx + min(kt + e % kNlK, k1 - 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < kAPer; ++i) {
+            const int e = tid + i * NT;
+            ar[i] = a[(size_t)min(p0 + e / kNlK, P - 1) * lda + min(kt + e % kNlK, k1 - 1)];
+        }
+    };
+    auto stash = [&](C* st, int kt) {
+        const bool tail = kt + kNlK > k1;
+#pragma unroll
+        for (int i = 0; i < kXPer; ++i) {
+            const int e = tid + i * NT;
+            if (tail && kt + e % kNlK >= k1) xr[i] = C{T(0), T(0)};
+            if (e < XR * kNlK) st[(e / kNlK) * kNlPitch + e % kNlK] = xr[i];
+        }
+#pragma unroll
+        for (int i = 0; i < kAPer; ++i) {
+            const int e = tid + i * NT;
+            if (tail && kt + e % kNlK >= k1) ar[i] = C{T(0), T(0)};
+            if (e < AR * kNlK) st[(XR + e / kNlK) * kNlPitch + e % kNlK] = ar[i];
+        }
+    };
     // Complex products by three real MFMAs (Gauss): with x = xr + i xi, a = ar + i ai,
     // acc1 = sum xr ar, acc2 = sum xi ai, acc3 = sum (xr + xi)(ar + ai);
     // Re = acc1 - acc2, Im = acc3 - acc1 - acc2.
-    typename M::acc acc1[2][PB], acc2[2][PB], acc3[2][PB];
+    typename M::acc acc1[BBW], acc2[BBW], acc3[BBW];
 #pragma unroll
-    for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-        for (int pb = 0; pb < PB; ++pb) {
-            acc1[bb][pb] = typename M::acc{0, 0, 0, 0};
-            acc2[bb][pb] = typename M::acc{0, 0, 0, 0};
-            acc3[bb][pb] = typename M::acc{0, 0, 0, 0};
-        }
-    if (k0 < k1) {
-        DZ_PROJ_FETCH(k0)
-        DZ_PROJ_STASH()
-    }
+    for (int bb = 0; bb < BBW; ++bb) acc1[bb] = acc2[bb] = acc3[bb] = typename M::acc{0, 0, 0, 0};
+    fetch(k0);
+    stash(lds, k0);
     __syncthreads();
-    for (int kt = k0; kt < k1; kt += kNlK) {
+    int buf = 0;
+    for (int kt = k0; kt < k1; kt += kNlK, buf ^= 1) {
         const bool more = kt + kNlK < k1;
-        if (more) {
-            DZ_PROJ_FETCH(kt + kNlK)
-        }
+        if (more) fetch(kt + kNlK);
+        __builtin_amdgcn_sched_barrier(0);  // the loads go out first
+        const C* xs = lds + buf * kStage + (wb * BBW * 16 + i16) * kNlPitch + k4;
+        const C* as = lds + buf * kStage + (XR + wx * 16 + i16) * kNlPitch + k4;
 #pragma unroll
         for (int kk = 0; kk < kNlK; kk += 4) {
-            C xa[2], ab[PB];
+            const C ab = as[kk];
+            const T asum = ab.x + ab.y;
 #pragma unroll
-            for (int bb = 0; bb < 2; ++bb) xa[bb] = xs[(bg * 32 + bb * 16 + i16) * kNlPitch + kk + k4];
-#pragma unroll
-            for (int pb = 0; pb < PB; ++pb) ab[pb] = as[((half * PB + pb) * 16 + i16) * kNlPitch + kk + k4];
-            T xsum[2], asum[PB];
-#pragma unroll
-            for (int bb = 0; bb < 2; ++bb) xsum[bb] = xa[bb].x + xa[bb].y;
-#pragma unroll
-            for (int pb = 0; pb < PB; ++pb) asum[pb] = ab[pb].x + ab[pb].y;
-#pragma unroll
-            for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-                for (int pb = 0; pb < PB; ++pb) {
-                    acc1[bb][pb] = M::mma(xa[bb].x, ab[pb].x, acc1[bb][pb]);
-                    acc2[bb][pb] = M::mma(xa[bb].y, ab[pb].y, acc2[bb][pb]);
-                    acc3[bb][pb] = M::mma(xsum[bb], asum[pb], acc3[bb][pb]);
-                }
+            for (int bb = 0; bb < BBW; ++bb) {
+                const C xa = xs[bb * 16 * kNlPitch + kk];
+                acc1[bb] = M::mma(xa.x, ab.x, acc1[bb]);
+                acc2[bb] = M::mma(xa.y, ab.y, acc2[bb]);
+                acc3[bb] = M::mma(xa.x + xa.y, asum, acc3[bb]);
+            }
         }
-        __syncthreads();
-        if (more) {
-            DZ_PROJ_STASH()
-        }
+        // The other buffer was last read before the barrier that ended the previous stage.
+        if (more) stash(lds + (buf ^ 1) * kStage, kt + kNlK);
         __syncthreads();
     }
-#undef DZ_PROJ_FETCH
-#undef DZ_PROJ_STASH
 #pragma unroll
-    for (int bb = 0; bb < 2; ++bb)
+    for (int bb = 0; bb < BBW; ++bb)
 #pragma unroll
-        for (int pb = 0; pb < PB; ++pb)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int b = b0 + bg * 32 + bb * 16 + M::row(k4, r);
-                const int p = p0 + (half * PB + pb) * 16 + i16;
-                const T c1 = acc1[bb][pb][r], c2 = acc2[bb][pb][r];
-                if (b < ncols && p < P)
-                    partial[((size_t)ks * ncols + b) * P + p] = C{c1 - c2, acc3[bb][pb][r] - c1 - c2};
-            }
+        for (int r = 0; r < 4; ++r) {
+            const int b = b0 + (wb * BBW + bb) * 16 + M::row(k4, r);
+            const int p = p0 + wx * 16 + i16;
+            const T c1 = acc1[bb][r], c2 = acc2[bb][r];
+            if (b < ncols && p < P) partial[((size_t)ks * ncols + b) * P + p] = C{c1 - c2, acc3[bb][r] - c1 - c2};
+        }
 }
 
 // One workgroup per band: sum the split-K partials of every projector into LDS (each partial
 // read once, coalesced over p; `split` interleaved subsets of the K-chunks per projector so
 // more loads are in flight, combined in a fixed order), then
 // q[b][p] = inv_vol * sum_r D[m][r] * sum[base + r] within the projector's atom block.
-constexpr int kDijSplit = 4;
 constexpr int kDijThreads = 1024;
-// K-chunk subsets the D kernel can stage for P projectors of element size esz, and its LDS bytes.
+// K-chunk subsets the D kernel stages for P projectors of element size esz (as many as it has
+// threads for, 4 to 16: the loads of a projector's chunks are what it waits for), and its LDS bytes.
 inline int dij_split(int P, size_t esz) {
-    for (int sp = kDijSplit; sp > 1; --sp)
+    for (int sp = std::min(16, std::max(4, kDijThreads / P)); sp > 1; --sp)
         if ((size_t)(sp + 1) * P * esz <= kMaxLdsBytes) return sp;
     return 1;
 }
@@ -1609,6 +1610,7 @@ __global__ __launch_bounds__(kDijThreads) void k_nl_dij(const typename C2T<T>::t
     for (int idx = tid; idx < split * P; idx += nthr) {
         const int j = idx / P, p = idx - j * P;
         C s = C{T(0), T(0)};
+#pragma unroll 8
         for (int ks = ks_lo + j; ks < ks_hi; ks += split) {
             const C v = partial[((size_t)ks * ncols + b) * P + p];
             s.x += v.x;
@@ -1642,20 +1644,18 @@ __global__ __launch_bounds__(kDijThreads) void k_nl_dij(const typename C2T<T>::t
 }
 
 // y[b][G] = sum_p q[b][p] * conj(A[p][G])   (written, not accumulated: runs before k_plane_fwd)
-template <typename T>
-__global__ __launch_bounds__(kNlThreads) void k_nl_back(const typename C2T<T>::type* __restrict__ a,
-                                                        const typename C2T<T>::type* __restrict__ q,
-                                                        typename C2T<T>::type* __restrict__ y, size_t ldy,
-                                                        int P, int npw, int ncols, const int4* __restrict__ tiles,
-                                                        int lda) {
+template <typename T, int BBW, int WB>
+__global__ __launch_bounds__(64 * WB * kNlGWaves, 2) void k_nl_back(const typename C2T<T>::type* __restrict__ a,
+                                                                 const typename C2T<T>::type* __restrict__ q,
+                                                                 typename C2T<T>::type* __restrict__ y, size_t ldy,
+                                                                 int P, int npw, int ncols,
+                                                                 const int4* __restrict__ tiles, int lda) {
     using C = typename C2T<T>::type;
     using M = Mfma<T>;
+    constexpr int NT = 64 * WB * kNlGWaves, QR = 16 * BBW * WB, GP = kNlG + 1, KS = kNlBackK, QP = KS + 1;
     extern __shared__ unsigned char smem_raw[];
-    C* qs = reinterpret_cast<C*>(smem_raw);  // [kNlBands][kNlPitch]  (band, p)
-    constexpr int kNlG = nl_g_tile<T>();
-    constexpr int kNlGPitch = kNlG + 1;
-    constexpr int GB = NlBackTile<T>::kBlocks / 2;  // G blocks per wavefront
-    C* as = qs + kNlBands * kNlPitch;        // [kNlK][kNlGPitch]     (p, G)
+    C* const lds = reinterpret_cast<C*>(smem_raw);  // two stages of [QR][QP] (band, p), [KS][GP] (p, G)
+    constexpr int kStage = QR * QP + KS * GP;
     // G tile: fixed-size tiles of one context's sphere, or (batched apply) the tile table's
     // (first G, end of its k-point's G range, k-point) with that k-point's q block.
     int g0 = blockIdx.x * kNlG, gend = npw;
@@ -1665,99 +1665,139 @@ __global__ __launch_bounds__(kNlThreads) void k_nl_back(const typename C2T<T>::t
         gend = tl.y;
         q += (size_t)tl.z * ncols * P;
     }
-    const int b0 = blockIdx.z * kNlBands;
+    const int b0 = blockIdx.z * QR;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int bg = wave % kNlBandGroups, half = wave / kNlBandGroups;
+    const int wb = wave % WB, wg = wave / WB;
     const int i16 = lane & 15, k4 = lane >> 4;
-    const C zero = C{T(0), T(0)};
-    constexpr int kQPer = (kNlBands * kNlK + kNlThreads - 1) / kNlThreads;
-    constexpr int kAPer = (kNlK * kNlG + kNlThreads - 1) / kNlThreads;
-    T qre[kQPer], qim[kQPer], are[kAPer], aim[kAPer];
-#define DZ_BACK_FETCH(PT)                                                                     \
-    _Pragma("unroll") for (int i = 0; i < kQPer; ++i) {                                      \
-        const int e = tid + i * kNlThreads;                                                   \
-        const int r = e >> 5, c = e & 31, b = b0 + r, p = (PT) + c;                           \
-        const bool ok = r < kNlBands && b < ncols && p < P;                                   \
-        const C v = q[ok ? b * P + p : 0];                                                    \
-        qre[i] = ok ? v.x : T(0);                                                             \
-        qim[i] = ok ? v.y : T(0);                                                             \
-    }                                                                                         \
-    _Pragma("unroll") for (int i = 0; i < kAPer; ++i) {                                      \
-        const int e = tid + i * kNlThreads;                                                   \
-        const int r = e / kNlG, c = e % kNlG, p = (PT) + r, g = g0 + c;                       \
-        const bool ok = r < kNlK && p < P && g < gend;                                        \
-        const C v = a[ok ? (size_t)p * lda + g : 0];                                          \
-        are[i] = ok ? v.x : T(0);                                                             \
-        aim[i] = ok ? v.y : T(0);                                                             \
-    }
-#define DZ_BACK_STASH()                                                                       \
-    _Pragma("unroll") for (int i = 0; i < kQPer; ++i) {                                      \
-        const int e = tid + i * kNlThreads;                                                   \
-        if (e < kNlBands * kNlK) qs[(e >> 5) * kNlPitch + (e & 31)] = C{qre[i], qim[i]};     \
-    }                                                                                         \
-    _Pragma("unroll") for (int i = 0; i < kAPer; ++i) {                                      \
-        const int e = tid + i * kNlThreads;                                                   \
-        if (e < kNlK * kNlG) as[(e / kNlG) * kNlGPitch + (e % kNlG)] = C{are[i], aim[i]};   \
-    }
+    constexpr int kQPer = (QR * KS + NT - 1) / NT, kAPer = (KS * kNlG + NT - 1) / NT;
+    // As in the projection: clamped loads, projectors beyond the last zeroed on their way to LDS.
+    C qr[kQPer], ar[kAPer];
+    auto fetch = [&](int pt) {
+#pragma unroll
+        for (int i = 0; i < kQPer; ++i) {
+            const int e = tid + i * NT;
+            qr[i] = q[(size_t)min(b0 + e / KS, ncols - 1) * P + min(pt + e % KS, P - 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < kAPer; ++i) {
+            const int e = tid + i * NT;
+            ar[i] = a[(size_t)min(pt + e / kNlG, P - 1) * lda + min(g0 + e % kNlG, gend - 1)];
+        }
+    };
+    auto stash = [&](C* st, int pt) {
+        const bool tail = pt + KS > P;
+#pragma unroll
+        for (int i = 0; i < kQPer; ++i) {
+            const int e = tid + i * NT;
+            if (tail && pt + e % KS >= P) qr[i] = C{T(0), T(0)};
+            if (e < QR * KS) st[(e / KS) * QP + e % KS] = qr[i];
+        }
+#pragma unroll
+        for (int i = 0; i < kAPer; ++i) {
+            const int e = tid + i * NT;
+            if (tail && pt + e / kNlG >= P) ar[i] = C{T(0), T(0)};
+            if (e < KS * kNlG) st[QR * QP + (e / kNlG) * GP + e % kNlG] = ar[i];
+        }
+    };
     // q conj(a) by three real MFMAs (Gauss) with a' = ar - i ai: acc1 = sum qr ar,
     // acc2 = sum qi (-ai), acc3 = sum (qr + qi)(ar - ai); Re = acc1 - acc2, Im = acc3 - acc1 - acc2.
-    typename M::acc acc1[2][GB], acc2[2][GB], acc3[2][GB];
+    typename M::acc acc1[BBW], acc2[BBW], acc3[BBW];
 #pragma unroll
-    for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-        for (int gb = 0; gb < GB; ++gb) {
-            acc1[bb][gb] = typename M::acc{0, 0, 0, 0};
-            acc2[bb][gb] = typename M::acc{0, 0, 0, 0};
-            acc3[bb][gb] = typename M::acc{0, 0, 0, 0};
-        }
-    DZ_BACK_FETCH(0)
-    DZ_BACK_STASH()
+    for (int bb = 0; bb < BBW; ++bb) acc1[bb] = acc2[bb] = acc3[bb] = typename M::acc{0, 0, 0, 0};
+    fetch(0);
+    stash(lds, 0);
     __syncthreads();
-    for (int pt = 0; pt < P; pt += kNlK) {
-        const bool more = pt + kNlK < P;
-        if (more) {
-            DZ_BACK_FETCH(pt + kNlK)
+    int buf = 0;
+    for (int pt = 0; pt < P; pt += KS, buf ^= 1) {
+        const bool more = pt + KS < P;
+        if (more) fetch(pt + KS);
+        __builtin_amdgcn_sched_barrier(0);  // the loads go out first
+        const C* qs = lds + buf * kStage + (wb * BBW * 16 + i16) * QP + k4;
+        const C* as = lds + buf * kStage + QR * QP + k4 * GP + wg * 16 + i16;
+#pragma unroll
+        for (int kk = 0; kk < KS; kk += 4) {
+            const C ab = as[kk * GP];
+            const T adif = ab.x - ab.y;
+#pragma unroll
+            for (int bb = 0; bb < BBW; ++bb) {
+                const C qa = qs[bb * 16 * QP + kk];
+                acc1[bb] = M::mma(qa.x, ab.x, acc1[bb]);
+                acc2[bb] = M::mma(qa.y, -ab.y, acc2[bb]);
+                acc3[bb] = M::mma(qa.x + qa.y, adif, acc3[bb]);
+            }
         }
-#pragma unroll
-        for (int kk = 0; kk < kNlK; kk += 4) {
-            C qa[2], ab[GB];
-#pragma unroll
-            for (int bb = 0; bb < 2; ++bb) qa[bb] = qs[(bg * 32 + bb * 16 + i16) * kNlPitch + kk + k4];
-#pragma unroll
-            for (int gb = 0; gb < GB; ++gb) ab[gb] = as[(kk + k4) * kNlGPitch + (half * GB + gb) * 16 + i16];
-            T qsum[2], adif[GB];
-#pragma unroll
-            for (int bb = 0; bb < 2; ++bb) qsum[bb] = qa[bb].x + qa[bb].y;
-#pragma unroll
-            for (int gb = 0; gb < GB; ++gb) adif[gb] = ab[gb].x - ab[gb].y;
-#pragma unroll
-            for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-                for (int gb = 0; gb < GB; ++gb) {
-                    acc1[bb][gb] = M::mma(qa[bb].x, ab[gb].x, acc1[bb][gb]);
-                    acc2[bb][gb] = M::mma(qa[bb].y, -ab[gb].y, acc2[bb][gb]);
-                    acc3[bb][gb] = M::mma(qsum[bb], adif[gb], acc3[bb][gb]);
-                }
-        }
-        __syncthreads();
-        if (more) {
-            DZ_BACK_STASH()
-        }
+        // The other buffer was last read before the barrier that ended the previous stage.
+        if (more) stash(lds + (buf ^ 1) * kStage, pt + KS);
         __syncthreads();
     }
-#undef DZ_BACK_FETCH
-#undef DZ_BACK_STASH
 #pragma unroll
-    for (int bb = 0; bb < 2; ++bb)
+    for (int bb = 0; bb < BBW; ++bb)
 #pragma unroll
-        for (int gb = 0; gb < GB; ++gb)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int b = b0 + bg * 32 + bb * 16 + M::row(k4, r);
-                const int g = g0 + (half * GB + gb) * 16 + i16;
-                const T c1 = acc1[bb][gb][r], c2 = acc2[bb][gb][r];
-                if (b < ncols && g < gend) y[(size_t)b * ldy + g] = C{c1 - c2, acc3[bb][gb][r] - c1 - c2};
-            }
+        for (int r = 0; r < 4; ++r) {
+            const int b = b0 + (wb * BBW + bb) * 16 + M::row(k4, r);
+            const int g = g0 + wg * 16 + i16;
+            const T c1 = acc1[bb][r], c2 = acc2[bb][r];
+            if (b < ncols && g < gend) y[(size_t)b * ldy + g] = C{c1 - c2, acc3[bb][r] - c1 - c2};
+        }
+}
+
+// The instances by 16-band blocks per tile (1, 2, 3, 5: one wavefront along the bands; 8, 10: two).
+template <typename T>
+using NlProjFn = void (*)(const typename C2T<T>::type*, const typename C2T<T>::type*, size_t, typename C2T<T>::type*, int,
+                          int, int, int, int, const int2*, int);
+template <typename T>
+using NlBackFn = void (*)(const typename C2T<T>::type*, const typename C2T<T>::type*, typename C2T<T>::type*, size_t, int,
+                          int, int, const int4*, int);
+template <typename T, int WX>
+static NlProjFn<T> nl_proj_of(int blocks) {
+    switch (blocks) {
+        case 1: return k_nl_proj<T, 1, 1, WX>;
+        case 2: return k_nl_proj<T, 2, 1, WX>;
+        case 3: return k_nl_proj<T, 3, 1, WX>;
+        case 5: return k_nl_proj<T, 5, 1, WX>;
+        case 8: return k_nl_proj<T, 4, 2, WX>;
+        default: return k_nl_proj<T, 5, 2, WX>;
+    }
+}
+template <typename T>
+static NlBackFn<T> nl_back_of(int blocks) {
+    switch (blocks) {
+        case 1: return k_nl_back<T, 1, 1>;
+        case 2: return k_nl_back<T, 2, 1>;
+        case 3: return k_nl_back<T, 3, 1>;
+        case 5: return k_nl_back<T, 5, 1>;
+        case 8: return k_nl_back<T, 4, 2>;
+        default: return k_nl_back<T, 5, 2>;
+    }
+}
+static int nl_band_waves(int blocks) { return blocks > 5 ? 2 : 1; }
+
+// LDS limits of a shape's kernels (before a capture).
+template <typename T>
+static void nl_prepare(const NlShape& sh) {
+    set_max_dynamic_lds(sh.wx == 4 ? (const void*)nl_proj_of<T, 4>(sh.blocks) : (const void*)nl_proj_of<T, 2>(sh.blocks),
+                        nl_proj_lds_bytes<T>(sh.blocks, sh.wx));
+    set_max_dynamic_lds((const void*)nl_back_of<T>(sh.blocks), nl_back_lds_bytes<T>(sh.blocks));
+}
+
+template <typename T>
+static void launch_nl_proj(const NlShape& sh, int nks, const typename C2T<T>::type* a, const typename C2T<T>::type* x,
+                           size_t ldx, typename C2T<T>::type* partial, int P, int npw, int ncols, const int2* chunks,
+                           int lda, hipStream_t s) {
+    hipLaunchKernelGGL((sh.wx == 4 ? nl_proj_of<T, 4>(sh.blocks) : nl_proj_of<T, 2>(sh.blocks)),
+                       dim3((unsigned)(sh.ptiles * nks), 1, (unsigned)sh.btiles),
+                       dim3((unsigned)(64 * nl_band_waves(sh.blocks) * sh.wx)), nl_proj_lds_bytes<T>(sh.blocks, sh.wx), s,
+                       a, x, ldx, partial, P, npw, ncols, sh.kchunk, sh.ptiles, chunks, lda);
+    DZ_HIP(hipGetLastError());
+}
+template <typename T>
+static void launch_nl_back(const NlShape& sh, int gtiles, const typename C2T<T>::type* a, const typename C2T<T>::type* q,
+                           typename C2T<T>::type* y, size_t ldy, int P, int npw, int ncols, const int4* tiles, int lda,
+                           hipStream_t s) {
+    hipLaunchKernelGGL(nl_back_of<T>(sh.blocks), dim3((unsigned)gtiles, 1, (unsigned)sh.btiles),
+                       dim3((unsigned)(64 * nl_band_waves(sh.blocks) * kNlGWaves)), nl_back_lds_bytes<T>(sh.blocks), s, a,
+                       q, y, ldy, P, npw, ncols, tiles, lda);
+    DZ_HIP(hipGetLastError());
 }
 
 template <typename T>
@@ -2494,16 +2534,9 @@ void ham_apply_dev(Ham& h, const void* xv, void* yv, size_t ncols, bool local, b
         const C* xc = x + c0 * ld;
         C* yc = y + c0 * ld;
         // Launch shapes and buffers first: nothing may reallocate once two streams run.
-        constexpr int kNlP = nl_p_tile<T>();
-        const int ptiles = (h.nproj + kNlP - 1) / kNlP;
-        const int btiles = (int)((nc + kNlBands - 1) / kNlBands);
-        const int ktiles = (int)((h.npw + kNlK - 1) / kNlK);
-        // Split K so that about one workgroup per CU runs; each K-chunk a multiple of kNlK.
-        int nks = std::max(1, std::min(ktiles, (256 + ptiles * btiles - 1) / std::max(1, ptiles * btiles)));
-        const int kchunk = (int)round_up((h.npw + nks - 1) / nks, kNlK);
-        nks = (int)((h.npw + kchunk - 1) / kchunk);
+        const NlShape sh = nl_shape(h.nproj, (int)h.npw, (int)nc);
         if (do_nl) {
-            h.partial.ensure((size_t)nks * nc * h.nproj * sizeof(C));
+            h.partial.ensure((size_t)sh.nks * nc * h.nproj * sizeof(C));
             h.qbuf.ensure(nc * h.nproj * sizeof(C));
         }
         C* tb = nullptr;
@@ -2531,29 +2564,20 @@ void ham_apply_dev(Ham& h, const void* xv, void* yv, size_t ncols, bool local, b
         hipEvent_t* evs = next_event_set(h);
         mark(h, evs, 0);
         if (do_nl) {
-            const size_t lds = nl_proj_lds_bytes<T>();
-            set_max_dynamic_lds((const void*)k_nl_proj<T>, lds);
-            hipLaunchKernelGGL(k_nl_proj<T>, dim3(ptiles * nks, 1, btiles), dim3(kNlThreads), lds, snl,
-                               Sel<T>::a(h), xc, ld, h.partial.as<C>(), h.nproj, (int)h.npw, (int)nc,
-                               kchunk, ptiles, (const int2*)nullptr, (int)h.npw);
-            DZ_HIP(hipGetLastError());
+            nl_prepare<T>(sh);
+            launch_nl_proj<T>(sh, sh.nks, Sel<T>::a(h), xc, ld, h.partial.as<C>(), h.nproj, (int)h.npw, (int)nc, nullptr,
+                              (int)h.npw, snl);
             const size_t lds_d = dij_lds_bytes(h.nproj, sizeof(C));
             set_max_dynamic_lds((const void*)k_nl_dij<T>, lds_d);
             hipLaunchKernelGGL(k_nl_dij<T>, dim3((unsigned)nc), dim3(kDijThreads), lds_d, snl, h.partial.as<C>(),
-                               nks, h.qbuf.as<C>(), h.meta.as<ProjMeta>(), Sel<T>::dm(h), h.nproj, (int)nc,
+                               sh.nks, h.qbuf.as<C>(), h.meta.as<ProjMeta>(), Sel<T>::dm(h), h.nproj, (int)nc,
                                (T)h.inv_volume, dij_split(h.nproj, sizeof(C)), (const int2*)nullptr);
             DZ_HIP(hipGetLastError());
         }
         mark(h, evs, 1);
         if (do_nl) {
-            const size_t lds = nl_back_lds_bytes<T>();
-            constexpr int kNlG = nl_g_tile<T>();
-            set_max_dynamic_lds((const void*)k_nl_back<T>, lds);
-            hipLaunchKernelGGL(k_nl_back<T>, dim3((unsigned)((h.npw + kNlG - 1) / kNlG), 1,
-                                                  (unsigned)((nc + kNlBands - 1) / kNlBands)),
-                               dim3(kNlThreads), lds, snl, Sel<T>::a(h), h.qbuf.as<C>(), yc, ld, h.nproj,
-                               (int)h.npw, (int)nc, (const int4*)nullptr, (int)h.npw);
-            DZ_HIP(hipGetLastError());
+            launch_nl_back<T>(sh, (int)((h.npw + kNlG - 1) / kNlG), Sel<T>::a(h), h.qbuf.as<C>(), yc, ld, h.nproj,
+                              (int)h.npw, (int)nc, nullptr, (int)h.npw, snl);
         }
         if (overlap) DZ_HIP(hipEventRecord(h.ev_join, snl));
         mark(h, evs, 2);
@@ -2729,24 +2753,17 @@ void hamset_build(HamSet& hs) {
 template <typename T>
 static void hamset_segments(HamSet& hs, size_t nc) {
     if (hs.seg_cols == nc && hs.seg_prec == (int)sizeof(T)) return;
-    constexpr int kNlP = nl_p_tile<T>();
-    constexpr int kNlG = nl_g_tile<T>();
-    const int ptiles = (hs.nproj + kNlP - 1) / kNlP;
-    const int btiles = (int)((nc + kNlBands - 1) / kNlBands);
     std::vector<int> chunks, kseg;
     std::vector<int> tiles;
     for (size_t k = 0; k < hs.ks.size(); ++k) {
         const int npw = (int)hs.ks[k]->npw;
         const int off = (int)hs.npw_off[k];
         // The same split as ham_apply_dev for this k-point alone.
-        const int ktiles = (npw + kNlK - 1) / kNlK;
-        int nks = std::max(1, std::min(ktiles, (256 + ptiles * btiles - 1) / std::max(1, ptiles * btiles)));
-        const int kchunk = (int)round_up((npw + nks - 1) / nks, kNlK);
-        nks = (npw + kchunk - 1) / kchunk;
+        const NlShape sh = nl_shape(hs.nproj, npw, (int)nc);
         kseg.push_back((int)chunks.size() / 2);
-        for (int c = 0; c < nks; ++c) {
-            chunks.push_back(off + c * kchunk);
-            chunks.push_back(off + std::min(npw, (c + 1) * kchunk));
+        for (int c = 0; c < sh.nks; ++c) {
+            chunks.push_back(off + c * sh.kchunk);
+            chunks.push_back(off + std::min(npw, (c + 1) * sh.kchunk));
         }
         kseg.push_back((int)chunks.size() / 2);
         for (int g = 0; g < npw; g += kNlG) {
@@ -2831,22 +2848,16 @@ static void hamset_launch(HamSet& hs, const void* xv, void* yv, size_t nc, int c
     const C* a = std::is_same<T, float>::value ? (const C*)hs.a32.ptr : (const C*)hs.a64.ptr;
     const T* kin = std::is_same<T, float>::value ? (const T*)hs.kinetic32.ptr : (const T*)hs.kinetic64.ptr;
     if (do_nl) {
-        constexpr int kNlP = nl_p_tile<T>();
-        const int ptiles = (hs.nproj + kNlP - 1) / kNlP;
-        const int btiles = (int)((nc + kNlBands - 1) / kNlBands);
-        hipLaunchKernelGGL(k_nl_proj<T>, dim3(ptiles * hs.nks_total, 1, btiles), dim3(kNlThreads),
-                           nl_proj_lds_bytes<T>(), s, a, x, ld, hs.partial.as<C>(), hs.nproj, (int)ld, (int)nc, 0,
-                           ptiles, hs.chunks.as<int2>(), (int)ld);
-        DZ_HIP(hipGetLastError());
+        // Tiles as one k-point's; its K-chunks come from the table.
+        const NlShape sh = nl_shape(hs.nproj, (int)h0.npw, (int)nc);
+        launch_nl_proj<T>(sh, hs.nks_total, a, x, ld, hs.partial.as<C>(), hs.nproj, (int)ld, (int)nc, hs.chunks.as<int2>(),
+                          (int)ld, s);
         hipLaunchKernelGGL(k_nl_dij<T>, dim3((unsigned)nc, (unsigned)nk), dim3(kDijThreads),
                            dij_lds_bytes(hs.nproj, sizeof(C)), s, hs.partial.as<C>(), hs.nks_total, hs.qbuf.as<C>(),
                            h0.meta.as<ProjMeta>(), Sel<T>::dm(h0), hs.nproj, (int)nc, (T)h0.inv_volume,
                            dij_split(hs.nproj, sizeof(C)), hs.kseg.as<int2>());
         DZ_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_nl_back<T>, dim3((unsigned)hs.ntiles, 1, (unsigned)((nc + kNlBands - 1) / kNlBands)),
-                           dim3(kNlThreads), nl_back_lds_bytes<T>(), s, a, hs.qbuf.as<C>(), y, ld, hs.nproj, (int)ld,
-                           (int)nc, hs.tiles.as<int4>(), (int)ld);
-        DZ_HIP(hipGetLastError());
+        launch_nl_back<T>(sh, hs.ntiles, a, hs.qbuf.as<C>(), y, ld, hs.nproj, (int)ld, (int)nc, hs.tiles.as<int4>(), (int)ld, s);
     }
     const PlaneArgs pa = plane_args(hs);
     launch_plane_inv<T>(pa, pkind, x, ld, tb, nc, tw, s);
@@ -2873,9 +2884,8 @@ void hamset_apply_dev(HamSet& hs, const void* x, void* y, size_t nc, bool use_gr
     if (hs.nproj > 0) {
         hs.partial.ensure((size_t)hs.nks_total * nc * hs.nproj * sizeof(C));
         hs.qbuf.ensure(hs.ks.size() * nc * hs.nproj * sizeof(C));
-        set_max_dynamic_lds((const void*)k_nl_proj<T>, nl_proj_lds_bytes<T>());
+        nl_prepare<T>(nl_shape(hs.nproj, (int)h0.npw, (int)nc));
         set_max_dynamic_lds((const void*)k_nl_dij<T>, dij_lds_bytes(hs.nproj, sizeof(C)));
-        set_max_dynamic_lds((const void*)k_nl_back<T>, nl_back_lds_bytes<T>());
     }
     const int pkind = hamset_plane_kind<T>(hs);
     plane_prepare<T>(plane_args(hs), pkind);

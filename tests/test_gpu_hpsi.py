@@ -490,3 +490,26 @@ def test_hpsi_overlap_is_bitwise_identical(dz, ctx, prec):
             assert np.array_equal(got, ref)
     finally:
         ham.close()
+
+
+@pytest.mark.parametrize("natoms", [1, 8, 11])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_hpsi_nonlocal_band_tiles(dz, ctx, prec, natoms):
+    """The nonlocal GEMMs at the edges of their band tiles (16-band blocks, 1 to 10 of them in a
+    workgroup, two workgroups beyond 160) and with 4, 32 and 44 projectors (part of a 16-wide block,
+    two whole ones, more than a two-wavefront tile), against the same products in numpy."""
+    w = workloads.si8(nbands=256)
+    rng = np.random.default_rng(natoms)
+    pos = rng.uniform(0.0, 1.0, size=(natoms, 3)) @ w.cell
+    species = [{"l_list": w.species[0].l_list, "dij": w.species[0].dij, "phi": w.phi(0)}]
+    ham = dz.Hamiltonian(ctx, w.grid, tables.fft_indices(w.basis, w.grid), w.basis.kinetic, w.basis.cart, w.local_r,
+                         w.inv_volume, species, pos, np.zeros(natoms, dtype=np.int32))
+    a = (np.exp(1j * (pos @ w.basis.cart.T))[:, None, :] * w.phi(0)[None]).reshape(-1, w.npw)
+    d = np.tile(np.repeat(np.diag(w.species[0].dij), [1, 3]), natoms) * w.inv_volume
+    ref = ((w.psi @ a.T) * d) @ a.conj()
+    for nb in (1, 15, 16, 17, 33, 48, 49, 80, 81, 128, 129, 160, 161, 256):
+        y = ham.apply_nonlocal(w.psi[:nb], prec)
+        err = relerr(y, ref[:nb])
+        print(f"natoms={natoms} prec={prec} nb={nb} err={err:.2e}", flush=True)
+        assert err < (TOL64 if prec == 0 else TOL32)
+    ham.close()
