@@ -1425,10 +1425,15 @@ constexpr int kNlG = 16 * kNlGWaves;
 // Split of a projection: btiles tiles of `blocks` 16-band blocks, ptiles tiles of 16 wx projectors,
 // nks K-chunks.  One workgroup of eight wavefronts per CU, two of four.  Every K-chunk is a multiple
 // of two stages.  A function of the sizes of one k-point alone, so that a set of k-points repeats it.
+// In FP32 the chunks are those of 64-projector by 160-band tiles whatever the tile, and k_nl_dij adds
+// them in four subsets: rounding there is 1e-7, and the order of the sums is kept so that FP32 results
+// are the same bits for every tile shape.
 struct NlShape {
     int blocks, btiles, wx, ptiles, nks, kchunk;
 };
+template <typename T>
 static NlShape nl_shape(int P, int npw, int ncols) {
+    constexpr bool fp32 = std::is_same<T, float>::value;
     NlShape s;
     const int nbk = (ncols + 15) / 16;
     s.btiles = std::max(1, (nbk + kNlMaxBlocks - 1) / kNlMaxBlocks);
@@ -1440,8 +1445,8 @@ static NlShape nl_shape(int P, int npw, int ncols) {
         }
     s.wx = P <= 32 ? 2 : 4;
     s.ptiles = std::max(1, (P + 16 * s.wx - 1) / (16 * s.wx));
-    const int tiles = s.ptiles * s.btiles, ktiles = (npw + 2 * kNlK - 1) / (2 * kNlK);
-    const int want = s.blocks > 5 ? 256 : 512;
+    const int tiles = fp32 ? std::max(1, (P + 63) / 64) * s.btiles : s.ptiles * s.btiles;
+    const int want = fp32 || s.blocks > 5 ? 256 : 512, ktiles = (npw + 2 * kNlK - 1) / (2 * kNlK);
     s.nks = std::max(1, std::min(ktiles, (want + tiles - 1) / tiles));
     s.kchunk = (int)round_up((npw + s.nks - 1) / s.nks, 2 * kNlK);
     s.nks = (npw + s.kchunk - 1) / s.kchunk;
@@ -1575,9 +1580,11 @@ __global__ __launch_bounds__(64 * WB * WX) void k_nl_proj(const typename C2T<T>:
 // q[b][p] = inv_vol * sum_r D[m][r] * sum[base + r] within the projector's atom block.
 constexpr int kDijThreads = 1024;
 // K-chunk subsets the D kernel stages for P projectors of element size esz (as many as it has
-// threads for, 4 to 16: the loads of a projector's chunks are what it waits for), and its LDS bytes.
+// threads for, 4 to 16, in FP64: the loads of a projector's chunks are what it waits for; 4 in FP32,
+// see NlShape), and its LDS bytes.
 inline int dij_split(int P, size_t esz) {
-    for (int sp = std::min(16, std::max(4, kDijThreads / P)); sp > 1; --sp)
+    const int most = esz == sizeof(float2) ? 4 : std::min(16, std::max(4, kDijThreads / P));
+    for (int sp = most; sp > 1; --sp)
         if ((size_t)(sp + 1) * P * esz <= kMaxLdsBytes) return sp;
     return 1;
 }
@@ -2534,7 +2541,7 @@ void ham_apply_dev(Ham& h, const void* xv, void* yv, size_t ncols, bool local, b
         const C* xc = x + c0 * ld;
         C* yc = y + c0 * ld;
         // Launch shapes and buffers first: nothing may reallocate once two streams run.
-        const NlShape sh = nl_shape(h.nproj, (int)h.npw, (int)nc);
+        const NlShape sh = nl_shape<T>(h.nproj, (int)h.npw, (int)nc);
         if (do_nl) {
             h.partial.ensure((size_t)sh.nks * nc * h.nproj * sizeof(C));
             h.qbuf.ensure(nc * h.nproj * sizeof(C));
@@ -2759,7 +2766,7 @@ static void hamset_segments(HamSet& hs, size_t nc) {
         const int npw = (int)hs.ks[k]->npw;
         const int off = (int)hs.npw_off[k];
         // The same split as ham_apply_dev for this k-point alone.
-        const NlShape sh = nl_shape(hs.nproj, npw, (int)nc);
+        const NlShape sh = nl_shape<T>(hs.nproj, npw, (int)nc);
         kseg.push_back((int)chunks.size() / 2);
         for (int c = 0; c < sh.nks; ++c) {
             chunks.push_back(off + c * sh.kchunk);
@@ -2849,7 +2856,7 @@ static void hamset_launch(HamSet& hs, const void* xv, void* yv, size_t nc, int c
     const T* kin = std::is_same<T, float>::value ? (const T*)hs.kinetic32.ptr : (const T*)hs.kinetic64.ptr;
     if (do_nl) {
         // Tiles as one k-point's; its K-chunks come from the table.
-        const NlShape sh = nl_shape(hs.nproj, (int)h0.npw, (int)nc);
+        const NlShape sh = nl_shape<T>(hs.nproj, (int)h0.npw, (int)nc);
         launch_nl_proj<T>(sh, hs.nks_total, a, x, ld, hs.partial.as<C>(), hs.nproj, (int)ld, (int)nc, hs.chunks.as<int2>(),
                           (int)ld, s);
         hipLaunchKernelGGL(k_nl_dij<T>, dim3((unsigned)nc, (unsigned)nk), dim3(kDijThreads),
@@ -2884,7 +2891,7 @@ void hamset_apply_dev(HamSet& hs, const void* x, void* y, size_t nc, bool use_gr
     if (hs.nproj > 0) {
         hs.partial.ensure((size_t)hs.nks_total * nc * hs.nproj * sizeof(C));
         hs.qbuf.ensure(hs.ks.size() * nc * hs.nproj * sizeof(C));
-        nl_prepare<T>(nl_shape(hs.nproj, (int)h0.npw, (int)nc));
+        nl_prepare<T>(nl_shape<T>(hs.nproj, (int)h0.npw, (int)nc));
         set_max_dynamic_lds((const void*)k_nl_dij<T>, dij_lds_bytes(hs.nproj, sizeof(C)));
     }
     const int pkind = hamset_plane_kind<T>(hs);
