@@ -83,205 +83,220 @@ __global__ void k_precondition(const double2* __restrict__ r, const int* __restr
     q[(size_t)j * ld + i] = make_double2(v.x * f, v.y * f);
 }
 
-// ----------------------------------------------------------------- Gram products C = A^H B
-// For the tall-skinny products of the solver (K = n_pw ~ 24k, M, N <= a few hundred), where the
-// library GEMM runs at a few TF/s: split-K over workgroups of a 64 x 64 output tile, FP64 MFMA
-// 16x16x4 with the complex product as four real MFMAs, operands staged through LDS with a
-// register prefetch of the next K-stage, partials reduced in a fixed order by a second kernel.
+// ----------------------------------------------------------------- basis products
+// The solver's tall-skinny products (n = n_pw rows, up to a few hundred columns), where the library
+// GEMM runs at a few TF/s.  A tile is WX wavefronts of 16 columns of A (Gram) or 16 rows (basis times
+// coefficients) by JB blocks of 16 columns of the other side, the same for each, on the FP64 matrix
+// cores (16x16x4) with each complex product as three real ones.  K runs in stages of 8 through two
+// LDS buffers: the next stage's loads are in flight (unmasked, from clamped addresses; what lies
+// beyond the end is zeroed on its way to LDS) while one is multiplied, with one barrier a stage, and
+// two workgroups share a CU.  The matrix cores' rate bounds the large shapes, latency the small
+// ones.  Before: 64 x 64 tiles whose loads were masked, and so waited for, ahead of the products.  Gram /
+// basis products of a Si-64 solve (n = 23,984, medians over m = 164..648) 173 / 376 -> 147 / 219 us, of a
+// Si-8 solve (n = 1,637, 20 bands) 23 / 13 -> 5 / 8 us.
 typedef double v4d_t __attribute__((ext_vector_type(4)));
-constexpr int kGramTile = 64, kGramK = 16, kGramPitch = kGramK + 1, kGramThreads = 256;
-constexpr int kGramPer = kGramTile * kGramK / kGramThreads;  // complex elements per thread per operand
+constexpr int kBpK = 8, kBpPitch = kBpK + 1, kBpMaxBlocks = 6;
 
-__global__ __launch_bounds__(kGramThreads) void k_gram_cn(const double2* __restrict__ A, int lda, int M,
-                                                          const double2* __restrict__ B, int ldb, int N, int K,
-                                                          int kchunk, int mtiles, double2* __restrict__ partial) {
-    __shared__ double2 As[kGramTile * kGramPitch];
-    __shared__ double2 Bs[kGramTile * kGramPitch];
+// Column blocks of one tile and the tiles of N columns.
+static void bp_tiles(int N, int* jb, int* tiles) {
+    const int nbk = (N + 15) / 16;
+    *tiles = (nbk + kBpMaxBlocks - 1) / kBpMaxBlocks;
+    *jb = (nbk + *tiles - 1) / *tiles;
+}
+
+// partial[ks][j][i] = sum over K-chunk ks of conj(A[k][i]) B[k][j]; k_gram_reduce adds the chunks.
+template <int WX, int JB>
+__global__ __launch_bounds__(64 * WX, 2) void k_gram_cn(const double2* __restrict__ A, int lda, int M,
+                                                        const double2* __restrict__ B, int ldb, int N, int K, int kchunk,
+                                                        int mtiles, double2* __restrict__ partial) {
+    constexpr int NT = 64 * WX, AR = 16 * WX, BR = 16 * JB;
+    constexpr int AP = (AR * kBpK + NT - 1) / NT, BP = (BR * kBpK + NT - 1) / NT;
+    __shared__ double2 lds[2][(AR + BR) * kBpPitch];
     const int mt = blockIdx.x % mtiles, ks = blockIdx.x / mtiles;
-    const int i_base = mt * kGramTile, j_base = blockIdx.y * kGramTile;
+    const int i_base = mt * AR, j_base = blockIdx.y * BR;
     const int k0 = ks * kchunk, k1 = min(K, k0 + kchunk);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int wi = wave & 1, wj = wave >> 1;
     const int l16 = lane & 15, l4 = lane >> 4;
-    double ar[kGramPer], ai[kGramPer], br[kGramPer], bi[kGramPer];
+    double2 ar[AP], br[BP];
     auto fetch = [&](int kt) {
 #pragma unroll
-        for (int q = 0; q < kGramPer; ++q) {
-            const int e = tid + q * kGramThreads;
-            const int c = e / kGramK, kk = e % kGramK, k = kt + kk;
-            const int i = i_base + c, j = j_base + c;
-            const bool oka = i < M && k < k1, okb = j < N && k < k1;
-            const double2 va = A[oka ? (size_t)i * lda + k : 0];
-            const double2 vb = B[okb ? (size_t)j * ldb + k : 0];
-            ar[q] = oka ? va.x : 0.0;
-            ai[q] = oka ? va.y : 0.0;
-            br[q] = okb ? vb.x : 0.0;
-            bi[q] = okb ? vb.y : 0.0;
+        for (int q = 0; q < AP; ++q) {
+            const int e = tid + q * NT;
+            ar[q] = A[(size_t)min(i_base + e / kBpK, M - 1) * lda + min(kt + e % kBpK, k1 - 1)];
+        }
+#pragma unroll
+        for (int q = 0; q < BP; ++q) {
+            const int e = tid + q * NT;
+            br[q] = B[(size_t)min(j_base + e / kBpK, N - 1) * ldb + min(kt + e % kBpK, k1 - 1)];
         }
     };
-    auto stash = [&]() {
+    auto stash = [&](double2* st, int kt) {
+        const bool tail = kt + kBpK > k1;
 #pragma unroll
-        for (int q = 0; q < kGramPer; ++q) {
-            const int e = tid + q * kGramThreads;
-            const int c = e / kGramK, kk = e % kGramK;
-            As[c * kGramPitch + kk] = make_double2(ar[q], ai[q]);
-            Bs[c * kGramPitch + kk] = make_double2(br[q], bi[q]);
+        for (int q = 0; q < AP; ++q) {
+            const int e = tid + q * NT;
+            if (tail && kt + e % kBpK >= k1) ar[q] = make_double2(0.0, 0.0);
+            if (e < AR * kBpK) st[(e / kBpK) * kBpPitch + e % kBpK] = ar[q];
+        }
+#pragma unroll
+        for (int q = 0; q < BP; ++q) {
+            const int e = tid + q * NT;
+            if (tail && kt + e % kBpK >= k1) br[q] = make_double2(0.0, 0.0);
+            if (e < BR * kBpK) st[(AR + e / kBpK) * kBpPitch + e % kBpK] = br[q];
         }
     };
     // conj(a) b = (ar br + ai bi) + i (ar bi - ai br) by three real MFMAs (Gauss):
     // p1 = sum ar br, p2 = sum ai bi, p3 = sum (ar - ai)(br + bi); Re = p1 + p2, Im = p3 - p1 + p2.
-    v4d_t p1[2][2], p2[2][2], p3[2][2];
+    v4d_t p1[JB], p2[JB], p3[JB];
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y) {
-            p1[x][y] = v4d_t{0, 0, 0, 0};
-            p2[x][y] = v4d_t{0, 0, 0, 0};
-            p3[x][y] = v4d_t{0, 0, 0, 0};
-        }
-    if (k0 < k1) {
-        fetch(k0);
-        stash();
-    }
+    for (int y = 0; y < JB; ++y) p1[y] = p2[y] = p3[y] = v4d_t{0, 0, 0, 0};
+    fetch(k0);
+    stash(lds[0], k0);
     __syncthreads();
-    for (int kt = k0; kt < k1; kt += kGramK) {
-        const bool more = kt + kGramK < k1;
-        if (more) fetch(kt + kGramK);
+    int buf = 0;
+    for (int kt = k0; kt < k1; kt += kBpK, buf ^= 1) {
+        const bool more = kt + kBpK < k1;
+        if (more) fetch(kt + kBpK);
+        __builtin_amdgcn_sched_barrier(0);  // the loads go out first
+        const double2* as = lds[buf] + (wave * 16 + l16) * kBpPitch + l4;
+        const double2* bs = lds[buf] + (AR + l16) * kBpPitch + l4;
 #pragma unroll
-        for (int kk = 0; kk < kGramK; kk += 4) {
-            double2 av[2], bv[2];
+        for (int kk = 0; kk < kBpK; kk += 4) {
+            const double2 a = as[kk];
+            const double adif = a.x - a.y;
 #pragma unroll
-            for (int x = 0; x < 2; ++x) av[x] = As[(wi * 32 + x * 16 + l16) * kGramPitch + kk + l4];
-#pragma unroll
-            for (int y = 0; y < 2; ++y) bv[y] = Bs[(wj * 32 + y * 16 + l16) * kGramPitch + kk + l4];
-#pragma unroll
-            for (int x = 0; x < 2; ++x)
-#pragma unroll
-                for (int y = 0; y < 2; ++y) {
-                    p1[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[x].x, bv[y].x, p1[x][y], 0, 0, 0);
-                    p2[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[x].y, bv[y].y, p2[x][y], 0, 0, 0);
-                    p3[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[x].x - av[x].y, bv[y].x + bv[y].y, p3[x][y],
-                                                                   0, 0, 0);
-                }
+            for (int y = 0; y < JB; ++y) {
+                const double2 b = bs[y * 16 * kBpPitch + kk];
+                p1[y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, p1[y], 0, 0, 0);
+                p2[y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.y, p2[y], 0, 0, 0);
+                p3[y] = __builtin_amdgcn_mfma_f64_16x16x4f64(adif, b.x + b.y, p3[y], 0, 0, 0);
+            }
         }
-        __syncthreads();
-        if (more) stash();
+        // The other buffer was last read before the barrier that ended the previous stage.
+        if (more) stash(lds[buf ^ 1], kt + kBpK);
         __syncthreads();
     }
     // D slot r of a 16x16 block: row (l/16) + 4 r, column l % 16.
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+    for (int y = 0; y < JB; ++y)
 #pragma unroll
-        for (int y = 0; y < 2; ++y)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = i_base + wi * 32 + x * 16 + l4 + 4 * r;
-                const int j = j_base + wj * 32 + y * 16 + l16;
-                const double a1 = p1[x][y][r], a2 = p2[x][y][r];
-                if (i < M && j < N) partial[((size_t)ks * N + j) * M + i] = make_double2(a1 + a2, p3[x][y][r] - a1 + a2);
-            }
+        for (int r = 0; r < 4; ++r) {
+            const int i = i_base + wave * 16 + l4 + 4 * r;
+            const int j = j_base + y * 16 + l16;
+            const double a1 = p1[y][r], a2 = p2[y][r];
+            if (i < M && j < N) partial[((size_t)ks * N + j) * M + i] = make_double2(a1 + a2, p3[y][r] - a1 + a2);
+        }
 }
 
 // C[:, 0:N] = alpha A[:, 0:K] B[0:K, 0:N] + beta C, alpha and beta real: A is n x K (leading
-// dimension lda), B is K x N (ldb), C is n x N (ldc), all column-major.  For the solver's products
-// of the tall basis with small coefficient blocks (n = n_pw ~ 24k rows; K, N up to a few hundred):
-// one workgroup per 64 x 64 tile of C, K in stages of 16 through LDS with a register prefetch of
-// the next stage, FP64 MFMA 16x16x4 with each complex product as three real MFMAs.  The MFMA
-// computes C^T = B^T A^T so that a wavefront's accumulator slots hold 16 consecutive rows of a
-// column of C (coalesced loads of the old C and stores).
-__global__ __launch_bounds__(kGramThreads) void k_gemm_nn(const double2* __restrict__ A, int lda,
-                                                          const double2* __restrict__ B, int ldb,
-                                                          double2* __restrict__ C, int ldc, int n, int K, int N,
-                                                          double alpha, double beta) {
-    __shared__ double2 As[kGramTile * kGramPitch];  // [row][k]
-    __shared__ double2 Bs[kGramTile * kGramPitch];  // [column][k]
-    const int r_base = blockIdx.x * kGramTile, c_base = blockIdx.y * kGramTile;
+// dimension lda), B is K x N (ldb), C is n x N (ldc), all column-major.  The MFMA computes
+// C^T = B^T A^T so that a wavefront's accumulator slots hold 16 consecutive rows of a column of C
+// (coalesced loads of the old C and stores).
+template <int WX, int JB>
+__global__ __launch_bounds__(64 * WX, 2) void k_gemm_nn(const double2* __restrict__ A, int lda,
+                                                        const double2* __restrict__ B, int ldb, double2* __restrict__ C,
+                                                        int ldc, int n, int K, int N, double alpha, double beta) {
+    constexpr int NT = 64 * WX, RA = 16 * WX, RP = RA + 1, CB = 16 * JB;
+    constexpr int AP = (RA * kBpK + NT - 1) / NT, BP = (CB * kBpK + NT - 1) / NT;
+    __shared__ double2 la[2][kBpK * RP];        // [k][row]
+    __shared__ double2 lb[2][CB * kBpPitch];    // [column][k]
+    const int r_base = blockIdx.x * RA, c_base = blockIdx.y * CB;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int wr = wave & 1, wc = wave >> 1;
     const int l16 = lane & 15, l4 = lane >> 4;
-    double2 av[kGramPer], bv[kGramPer];
+    double2 ar[AP], br[BP];
     auto fetch = [&](int kt) {
 #pragma unroll
-        for (int q = 0; q < kGramPer; ++q) {
-            const int e = tid + q * kGramThreads;
-            // A: consecutive threads read consecutive rows of one column (coalesced).
-            const int ra = e % kGramTile, ka = e / kGramTile;
-            const int row = r_base + ra, k = kt + ka;
-            av[q] = (row < n && k < K) ? A[(size_t)k * lda + row] : make_double2(0.0, 0.0);
-            // B: consecutive threads read consecutive k of one column.
-            const int kb = e % kGramK, cb = e / kGramK;
-            const int col = c_base + cb, k2 = kt + kb;
-            bv[q] = (col < N && k2 < K) ? B[(size_t)col * ldb + k2] : make_double2(0.0, 0.0);
+        for (int q = 0; q < AP; ++q) {  // consecutive threads read consecutive rows of one column
+            const int e = tid + q * NT;
+            ar[q] = A[(size_t)min(kt + e / RA, K - 1) * lda + min(r_base + e % RA, n - 1)];
+        }
+#pragma unroll
+        for (int q = 0; q < BP; ++q) {
+            const int e = tid + q * NT;
+            br[q] = B[(size_t)min(c_base + e / kBpK, N - 1) * ldb + min(kt + e % kBpK, K - 1)];
         }
     };
-    auto stash = [&]() {
+    auto stash = [&](int st, int kt) {
+        const bool tail = kt + kBpK > K;
 #pragma unroll
-        for (int q = 0; q < kGramPer; ++q) {
-            const int e = tid + q * kGramThreads;
-            As[(e % kGramTile) * kGramPitch + e / kGramTile] = av[q];
-            Bs[(e / kGramK) * kGramPitch + e % kGramK] = bv[q];
+        for (int q = 0; q < AP; ++q) {
+            const int e = tid + q * NT;
+            if (tail && kt + e / RA >= K) ar[q] = make_double2(0.0, 0.0);
+            if (e < RA * kBpK) la[st][(e / RA) * RP + e % RA] = ar[q];
+        }
+#pragma unroll
+        for (int q = 0; q < BP; ++q) {
+            const int e = tid + q * NT;
+            if (tail && kt + e % kBpK >= K) br[q] = make_double2(0.0, 0.0);
+            if (e < CB * kBpK) lb[st][(e / kBpK) * kBpPitch + e % kBpK] = br[q];
         }
     };
     // b a = (br ar - bi ai) + i (br ai + bi ar): p1 = sum br ar, p2 = sum bi ai,
     // p3 = sum (br + bi)(ar + ai); Re = p1 - p2, Im = p3 - p1 - p2.
-    v4d_t p1[2][2], p2[2][2], p3[2][2];
+    v4d_t p1[JB], p2[JB], p3[JB];
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y) {
-            p1[x][y] = v4d_t{0, 0, 0, 0};
-            p2[x][y] = v4d_t{0, 0, 0, 0};
-            p3[x][y] = v4d_t{0, 0, 0, 0};
-        }
+    for (int x = 0; x < JB; ++x) p1[x] = p2[x] = p3[x] = v4d_t{0, 0, 0, 0};
     fetch(0);
-    stash();
+    stash(0, 0);
     __syncthreads();
-    for (int kt = 0; kt < K; kt += kGramK) {
-        const bool more = kt + kGramK < K;
-        if (more) fetch(kt + kGramK);
+    int buf = 0;
+    for (int kt = 0; kt < K; kt += kBpK, buf ^= 1) {
+        const bool more = kt + kBpK < K;
+        if (more) fetch(kt + kBpK);
+        __builtin_amdgcn_sched_barrier(0);  // the loads go out first
+        const double2* as = la[buf] + l4 * RP + wave * 16 + l16;
+        const double2* bs = lb[buf] + l16 * kBpPitch + l4;
 #pragma unroll
-        for (int kk = 0; kk < kGramK; kk += 4) {
-            double2 bo[2], ao[2];
+        for (int kk = 0; kk < kBpK; kk += 4) {
+            const double2 a = as[kk * RP];
+            const double asum = a.x + a.y;
             // Operand 0 (MFMA rows): columns of C; operand 1 (MFMA columns): rows of C.
 #pragma unroll
-            for (int x = 0; x < 2; ++x) bo[x] = Bs[(wc * 32 + x * 16 + l16) * kGramPitch + kk + l4];
-#pragma unroll
-            for (int y = 0; y < 2; ++y) ao[y] = As[(wr * 32 + y * 16 + l16) * kGramPitch + kk + l4];
-#pragma unroll
-            for (int x = 0; x < 2; ++x)
-#pragma unroll
-                for (int y = 0; y < 2; ++y) {
-                    p1[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(bo[x].x, ao[y].x, p1[x][y], 0, 0, 0);
-                    p2[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(bo[x].y, ao[y].y, p2[x][y], 0, 0, 0);
-                    p3[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(bo[x].x + bo[x].y, ao[y].x + ao[y].y, p3[x][y],
-                                                                   0, 0, 0);
-                }
+            for (int x = 0; x < JB; ++x) {
+                const double2 b = bs[x * 16 * kBpPitch + kk];
+                p1[x] = __builtin_amdgcn_mfma_f64_16x16x4f64(b.x, a.x, p1[x], 0, 0, 0);
+                p2[x] = __builtin_amdgcn_mfma_f64_16x16x4f64(b.y, a.y, p2[x], 0, 0, 0);
+                p3[x] = __builtin_amdgcn_mfma_f64_16x16x4f64(b.x + b.y, asum, p3[x], 0, 0, 0);
+            }
         }
-        __syncthreads();
-        if (more) stash();
+        // The other buffer was last read before the barrier that ended the previous stage.
+        if (more) stash(buf ^ 1, kt + kBpK);
         __syncthreads();
     }
     // Slot r of a 16x16 block: MFMA row (l/16) + 4 r = column of C, MFMA column l % 16 = row of C.
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+    for (int x = 0; x < JB; ++x)
 #pragma unroll
-        for (int y = 0; y < 2; ++y)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int col = c_base + wc * 32 + x * 16 + l4 + 4 * r;
-                const int row = r_base + wr * 32 + y * 16 + l16;
-                if (col < N && row < n) {
-                    const double a1 = p1[x][y][r], a2 = p2[x][y][r];
-                    double2 v = make_double2(alpha * (a1 - a2), alpha * (p3[x][y][r] - a1 - a2));
-                    double2* cp = C + (size_t)col * ldc + row;
-                    if (beta != 0.0) {
-                        const double2 o = *cp;
-                        v.x += beta * o.x;
-                        v.y += beta * o.y;
-                    }
-                    *cp = v;
+        for (int r = 0; r < 4; ++r) {
+            const int col = c_base + x * 16 + l4 + 4 * r;
+            const int row = r_base + wave * 16 + l16;
+            if (col < N && row < n) {
+                const double a1 = p1[x][r], a2 = p2[x][r];
+                double2 v = make_double2(alpha * (a1 - a2), alpha * (p3[x][r] - a1 - a2));
+                double2* cp = C + (size_t)col * ldc + row;
+                if (beta != 0.0) {
+                    const double2 o = *cp;
+                    v.x += beta * o.x;
+                    v.y += beta * o.y;
                 }
+                *cp = v;
             }
+        }
+}
+
+using GramFn = void (*)(const double2*, int, int, const double2*, int, int, int, int, int, double2*);
+using GemmFn = void (*)(const double2*, int, const double2*, int, double2*, int, int, int, int, double, double);
+template <int WX>
+static GramFn gram_fn(int jb) {
+    static const GramFn f[kBpMaxBlocks] = {k_gram_cn<WX, 1>, k_gram_cn<WX, 2>, k_gram_cn<WX, 3>,
+                                           k_gram_cn<WX, 4>, k_gram_cn<WX, 5>, k_gram_cn<WX, 6>};
+    return f[jb - 1];
+}
+template <int WX>
+static GemmFn gemm_fn(int jb) {
+    static const GemmFn f[kBpMaxBlocks] = {k_gemm_nn<WX, 1>, k_gemm_nn<WX, 2>, k_gemm_nn<WX, 3>,
+                                           k_gemm_nn<WX, 4>, k_gemm_nn<WX, 5>, k_gemm_nn<WX, 6>};
+    return f[jb - 1];
 }
 
 // C[j * ldc + i] = sum_ks partial[ks][j][i]
@@ -291,6 +306,7 @@ __global__ void k_gram_reduce(const double2* __restrict__ partial, int nks, int 
     const int j = blockIdx.y;
     if (i >= M) return;
     double re = 0.0, im = 0.0;
+#pragma unroll 8
     for (int ks = 0; ks < nks; ++ks) {
         const double2 v = partial[((size_t)ks * N + j) * M + i];
         re += v.x;
@@ -659,15 +675,19 @@ struct Solver {
     void gram(const double2* A, int M, const double2* B, int N, double2* C, int ldc) {
         if (M <= 0 || N <= 0) return;
         const int K = (int)n;
-        const int mtiles = (M + kGramTile - 1) / kGramTile, ntiles = (N + kGramTile - 1) / kGramTile;
-        // K-chunks (multiples of the stage depth) so that about three workgroups per CU run.
-        const int want = std::max(1, 768 / (mtiles * ntiles));
+        // Two wavefronts a tile up to 96 columns of A (more, smaller workgroups where there are few),
+        // four beyond; K-chunks so that the tiles fill two workgroups (four small ones) per CU.
+        const int wx = M <= 96 ? 2 : 4;
+        int jb = 1, ntiles = 1;
+        bp_tiles(N, &jb, &ntiles);
+        const int mtiles = (M + 16 * wx - 1) / (16 * wx);
+        const int want = std::max(1, (wx == 4 ? 512 : 1024) / (mtiles * ntiles));
         int kchunk = (K + want - 1) / want;
-        kchunk = std::max(kGramK * 8, (kchunk + kGramK - 1) / kGramK * kGramK);
+        kchunk = std::max(kBpK * 4, (kchunk + kBpK - 1) / kBpK * kBpK);
         const int nks = (K + kchunk - 1) / kchunk;
         w.gram_part.ensure((size_t)nks * M * N * sizeof(double2));
-        hipLaunchKernelGGL(k_gram_cn, dim3((unsigned)(mtiles * nks), (unsigned)ntiles), dim3(kGramThreads), 0, s, A,
-                           K, M, B, K, N, K, kchunk, mtiles, w.gram_part.as<double2>());
+        hipLaunchKernelGGL((wx == 4 ? gram_fn<4>(jb) : gram_fn<2>(jb)), dim3((unsigned)(mtiles * nks), (unsigned)ntiles),
+                           dim3(64u * wx), 0, s, A, K, M, B, K, N, K, kchunk, mtiles, w.gram_part.as<double2>());
         DZ_HIP(hipGetLastError());
         hipLaunchKernelGGL(k_gram_reduce, dim3((unsigned)((M + 255) / 256), (unsigned)N), dim3(256), 0, s,
                            w.gram_part.as<double2>(), nks, M, N, C, ldc);
@@ -677,11 +697,15 @@ struct Solver {
     void gemm(rocblas_operation ta, rocblas_operation tb, int m, int nn, int k, zc alpha, const double2* A,
               int lda, const double2* B, int ldb, zc beta, double2* C, int ldc) {
         if (m <= 0 || nn <= 0) return;
-        if (ta == rocblas_operation_none && tb == rocblas_operation_none && alpha.imag() == 0.0 && beta.imag() == 0.0) {
+        if (ta == rocblas_operation_none && tb == rocblas_operation_none && k > 0 && alpha.imag() == 0.0 &&
+            beta.imag() == 0.0) {
             // Basis times coefficients: the library's own MFMA kernel.
-            hipLaunchKernelGGL(k_gemm_nn, dim3((unsigned)((m + kGramTile - 1) / kGramTile),
-                                               (unsigned)((nn + kGramTile - 1) / kGramTile)),
-                               dim3(kGramThreads), 0, s, A, lda, B, ldb, C, ldc, m, k, nn, alpha.real(), beta.real());
+            int jb = 1, ntiles = 1;
+            bp_tiles(nn, &jb, &ntiles);
+            const int wx = m <= 8192 ? 2 : 4;  // 32-row tiles where 64-row ones would not fill the CUs
+            hipLaunchKernelGGL((wx == 4 ? gemm_fn<4>(jb) : gemm_fn<2>(jb)),
+                               dim3((unsigned)((m + 16 * wx - 1) / (16 * wx)), (unsigned)ntiles), dim3(64u * wx), 0, s, A, lda,
+                               B, ldb, C, ldc, m, k, nn, alpha.real(), beta.real());
             DZ_HIP(hipGetLastError());
             return;
         }

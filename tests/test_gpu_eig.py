@@ -134,3 +134,21 @@ def test_density_solution_guard(dz, ctx):
         assert abs(rho.sum() * (1.0 / w.inv_volume) / rho.size - 2.0) < 1e-10
     finally:
         ham.close()
+
+
+@pytest.mark.parametrize("nbands", [1, 7, 13, 29, 45, 93, 97])
+def test_eig_product_tiles(dz, ctx, nbands):
+    """Band counts at the edges of the basis products' tiles (blocks of 16 columns, one to six of them
+    and a second tile, two or four wavefronts along the other side): eigenvalues against the dense
+    eigh of the oracle's Hamiltonian (2e-8 Ry, the bar of this file)."""
+    from dzhip import workloads
+    from oracle import adapters, hamiltonian
+
+    w = workloads.tiny(nbands=4) if nbands == 1 else workloads.si8(nbands=4)
+    h = hamiltonian.dense_hamiltonian(adapters.context_from_workload(w))
+    ref = np.linalg.eigvalsh(0.5 * (h + h.conj().T))[:nbands]
+    ham = dz.Hamiltonian.from_workload(ctx, w)
+    vals, _, st = ham.eig_solve(nbands, tol=1e-7, max_iter=300, want_vectors=False)
+    ham.close()
+    print(f"nbands={nbands} n={w.npw} it={st['iterations']} dv={np.max(np.abs(vals - ref)):.2e}", flush=True)
+    assert st["converged"] == 1 and np.max(np.abs(vals - ref)) < 2e-8
