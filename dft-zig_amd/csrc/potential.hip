@@ -16,9 +16,12 @@
 // Parseval) and the small system is scaled by its largest diagonal before elimination; a
 // singular system keeps only the newest pair and takes a linear step (the reference would
 // average the whole history).
+#include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
+#include "fft_lds.h"
 #include "potential.h"
 
 namespace dzhip {
@@ -27,34 +30,34 @@ namespace {
 
 constexpr int kRedThreads = 256;
 
-// |G|^2 on the FFT-order grid (index x + nx (y + ny z), wrapped frequencies); b rows = b1, b2, b3.
-__global__ void k_g2(double* __restrict__ g2, int nx, int ny, int nz, double3 b1, double3 b2, double3 b3) {
+// |G|^2 on the FFT-order grid (index x + nx (y + ny z), wrapped frequencies; b rows = b1, b2, b3), and
+// the Hartree kernel 8 pi / G^2 (0 at G = 0), the mean of its values at an index and at the mirrored
+// one (they differ at an even axis' Nyquist frequencies when the cell is not orthogonal).
+__device__ __forceinline__ double hartree_factor(double g2) { return g2 > 1e-12 ? 8.0 * M_PI / g2 : 0.0; }
+__global__ void k_g2(double* __restrict__ g2, double* __restrict__ kern, int nx, int ny, int nz, double3 b1, double3 b2,
+                     double3 b3) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t n = (size_t)nx * ny * nz;
     if (i >= n) return;
     const int x = (int)(i % nx), y = (int)((i / nx) % ny), z = (int)(i / ((size_t)nx * ny));
-    const int fx = x <= (nx - 1) / 2 ? x : x - nx;
-    const int fy = y <= (ny - 1) / 2 ? y : y - ny;
-    const int fz = z <= (nz - 1) / 2 ? z : z - nz;
-    const double gx = fx * b1.x + fy * b2.x + fz * b3.x;
-    const double gy = fx * b1.y + fy * b2.y + fz * b3.y;
-    const double gz = fx * b1.z + fy * b2.z + fz * b3.z;
-    g2[i] = gx * gx + gy * gy + gz * gz;
+    auto norm2 = [&](int ix, int iy, int iz) {
+        const int fx = ix <= (nx - 1) / 2 ? ix : ix - nx;
+        const int fy = iy <= (ny - 1) / 2 ? iy : iy - ny;
+        const int fz = iz <= (nz - 1) / 2 ? iz : iz - nz;
+        const double gx = fx * b1.x + fy * b2.x + fz * b3.x;
+        const double gy = fx * b1.y + fy * b2.y + fz * b3.y;
+        const double gz = fx * b1.z + fy * b2.z + fz * b3.z;
+        return gx * gx + gy * gy + gz * gz;
+    };
+    const double g = norm2(x, y, z);
+    g2[i] = g;
+    kern[i] = 0.5 * (hartree_factor(g) +
+                     hartree_factor(norm2(x ? nx - x : 0, y ? ny - y : 0, z ? nz - z : 0)));
 }
 
 __global__ void k_real_to_complex(const double* __restrict__ in, double2* __restrict__ out, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) out[i] = make_double2(in[i], 0.0);
-}
-
-// w(G) *= 8 pi / G^2 (G = 0 -> 0): unnormalised forward transform in, so the normalised inverse
-// gives V_H(r) = sum_G V_H(G) e^{iG.r}.
-__global__ void k_hartree_kernel(double2* __restrict__ w, const double* __restrict__ g2, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double g = g2[i];
-    const double f = g > 1e-12 ? 8.0 * M_PI / g : 0.0;
-    w[i] = make_double2(w[i].x * f, w[i].y * f);
 }
 
 __device__ inline void lda_pz(double n, double* f, double* v) {
@@ -143,95 +146,253 @@ __device__ inline void pbe(double n, double g2, double* f, double* fn, double* f
     *fg = 2.0 * (fx_g + n * dH_dt2 / den_c);
 }
 
-// Cartesian G of FFT-order point i (wrapped frequencies); b = reciprocal rows.
-__device__ inline double3 g_at(size_t i, int nx, int ny, int nz, double3 b1, double3 b2, double3 b3) {
-    const int x = (int)(i % nx), y = (int)((i / nx) % ny), z = (int)(i / ((size_t)nx * ny));
-    const int fx = x <= (nx - 1) / 2 ? x : x - nx;
-    const int fy = y <= (ny - 1) / 2 ? y : y - ny;
-    const int fz = z <= (nz - 1) / 2 ? z : z - nz;
-    return make_double3(fx * b1.x + fy * b2.x + fz * b3.x, fx * b1.y + fy * b2.y + fz * b3.y,
-                        fx * b1.z + fy * b2.z + fz * b3.z);
+// ----------------------------------------------------------------- V_H + V_xc on the grid
+// The density's transforms with everything point-wise folded into their passes.  An xy-pass holds one
+// plane of k_z in LDS, transforms forward, multiplies in G space and transforms back; a z-pass holds a
+// few columns of one y, back to r space, evaluates the functional and transforms forward (the columns
+// are many workgroups, and the functional is what costs there).  Real fields share complex transforms
+// in pairs: with i G_c taken as zero at an even axis' Nyquist frequency (whose term is imaginary in r
+// space, where the real part is kept) the derivative of a real field is real, so
+//   d_x n + i d_y n = IFFT[(-G_y + i G_x) n(G)],   d_z n + i s V_H = IFFT[i (G_z + s K) n(G)],
+//   div b = Re IFFT[(G_y + i G_x) FFT(b_x + i b_y) + i G_z FFT(b_z)],
+// K the Hartree kernel 8 pi / G^2 (the mean over +G and -G, which is what the real part sees) and s a
+// power of two that keeps the two halves of a pair of like size.  PBE: five launches and six
+// transforms where there were some forty and ten, which launches bounded: 249 -> 100 us at 20 x 20 x
+// 20 (the xy-passes 16 each, on 20 CUs; barriers of their short lines bound them, k_xc_z 10, k_rho_z
+// 7, k_div_z 4, the rest launch gaps and the copies around them).  LDA: three launches.
+struct GridAxes {
+    FftAxis ax, ay, az;
+    const double2* tw;
+    const int* perm;
+    double3 b1, b2, b3;
+};
+
+// Frequency of index i on an axis of n points, zero at an even axis' Nyquist index (derivatives).
+__device__ __forceinline__ double deriv_freq(int i, int n) {
+    return 2 * i == n ? 0.0 : (double)(i <= (n - 1) / 2 ? i : i - n);
+}
+__device__ __forceinline__ double3 deriv_g(int x, int y, int z, const GridAxes& g) {
+    const double fx = deriv_freq(x, g.ax.n), fy = deriv_freq(y, g.ay.n), fz = deriv_freq(z, g.az.n);
+    return make_double3(fx * g.b1.x + fy * g.b2.x + fz * g.b3.x, fx * g.b1.y + fy * g.b2.y + fz * g.b3.y,
+                        fx * g.b1.z + fy * g.b2.z + fz * g.b3.z);
 }
 
-__device__ inline double comp(double3 v, int c) { return c == 0 ? v.x : (c == 1 ? v.y : v.z); }
-
-// out(G) = i G_c w(G)
-__global__ void k_grad_comp(const double2* __restrict__ w, double2* __restrict__ out, int c, int nx, int ny, int nz,
-                            double3 b1, double3 b2, double3 b3) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t n = (size_t)nx * ny * nz;
-    if (i >= n) return;
-    const double g = comp(g_at(i, nx, ny, nz, b1, b2, b3), c);
-    out[i] = make_double2(-g * w[i].y, g * w[i].x);
-}
-
-// acc(G) (+)= i G_c w(G)
-__global__ void k_div_acc(const double2* __restrict__ w, double2* __restrict__ acc, int c, int first, int nx, int ny,
-                          int nz, double3 b1, double3 b2, double3 b3) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t n = (size_t)nx * ny * nz;
-    if (i >= n) return;
-    const double g = comp(g_at(i, nx, ny, nz, b1, b2, b3), c);
-    const double2 t = make_double2(-g * w[i].y, g * w[i].x);
-    acc[i] = first ? t : make_double2(acc[i].x + t.x, acc[i].y + t.y);
-}
-
-// f, df/dn and b_c = df/dg2 * (grad n)_c (overwriting the gradient components).
-__global__ void k_pbe_point(const double* __restrict__ rho, double* __restrict__ gx, double* __restrict__ gy,
-                            double* __restrict__ gz, double* __restrict__ fxc, double* __restrict__ vn, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double ax = gx[i], ay = gy[i], az = gz[i];
-    double f, fn, fg;
-    pbe(rho[i], ax * ax + ay * ay + az * az, &f, &fn, &fg);
-    fxc[i] = f;
-    vn[i] = fn;
-    gx[i] = fg * ax;
-    gy[i] = fg * ay;
-    gz[i] = fg * az;
-}
-
-// vn -= 2 Re(div)
-__global__ void k_gga_combine(double* __restrict__ vn, const double2* __restrict__ div, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) vn[i] -= 2.0 * div[i].x;
-}
-
-// V_out = Re(V_H) + v_xc; per-block partial sums of [V_H rho, f_xc, v_in rho, (rho - rho_in)^2].
-// With gga_f/gga_v (PBE fields computed before) those replace the point-wise LDA-PZ.
-__global__ void k_hxc(const double2* __restrict__ vh, const double* __restrict__ rho, const double* __restrict__ rho_in,
-                      const double* __restrict__ vin, const double* __restrict__ gga_f, const double* __restrict__ gga_v,
-                      double* __restrict__ vout, double* __restrict__ part, size_t n) {
-    __shared__ double red[4][kRedThreads];
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const double r = rho[i];
-        double f, v;
-        if (gga_f) {
-            f = gga_f[i];
-            v = gga_v[i];
+// xy-pass, out and back.  HARTREE: w1 = K w1.  GRADIENT: w1 = (-G_y + i G_x) w1 and w2 = i (G_z + s K)
+// w1.  DIVERGENCE: w1 = (G_y + i G_x) w1 + i G_z w2.  All times 1/N.  KP: points per thread.  DUAL
+// (planes whose two tiles fit LDS): where two fields go the same way, their planes lie side by side,
+// rows interleaved, in one transform (half the barriers).
+enum { kHartree = 0, kGradient = 1, kDivergence = 2 };
+template <int KIND, int KP, bool DUAL>
+__global__ __launch_bounds__(512) void k_gridxy(double2* __restrict__ w1, double2* __restrict__ w2,
+                                                const double* __restrict__ kern, double s, double scale, GridAxes g) {
+    extern __shared__ double2 lds[];
+    constexpr int F = DUAL ? 2 : 1;
+    const int nx = g.ax.n, ny = g.ay.n, half = nx + 1, pitch = F * half, tid = threadIdx.x, nthr = blockDim.x, np = nx * ny;
+    double2 *twx = lds + pitch * ny, *twy = twx + nx;
+    load_twiddles(twx, g.tw + g.ax.tw_off, nx, tid, nthr);
+    load_twiddles(twy, g.tw + g.ay.tw_off, ny, tid, nthr);
+    const size_t off = (size_t)blockIdx.x * np;
+    const int *px = g.perm + g.ax.perm_off, *py = g.perm + g.ay.perm_off;
+    const unsigned mx = div_magic(nx);
+    // Natural order in, digit-reversed out; fields: tiles in use.
+    auto lines = [&](auto sign, int fields) {
+        constexpr int S = decltype(sign)::value;
+        lds_fft_lines<double, double2, false, S>(lds, g.ax, twx, LineSet{fields == F ? F * ny : ny, 1, fields == F ? half : pitch, nullptr},
+                                                 tid, nthr);
+        lds_fft_lines<double, double2, false, S>(lds, g.ay, twy, LineSet{fields == 2 ? pitch : nx, pitch, 1, nullptr}, tid, nthr);
+    };
+    const std::integral_constant<int, -1> fwd;
+    const std::integral_constant<int, 1> inv;
+    auto load = [&](const double2* src, int shift) {
+        for (int i = tid; i < np; i += nthr) {
+            const int y = fdiv(i, nx, mx);
+            lds[i - y * nx + pitch * y + shift] = src[off + i];
+        }
+    };
+    auto store = [&](double2* dst, int shift) {
+        for (int i = tid; i < np; i += nthr) {
+            const int y = fdiv(i, nx, mx);
+            dst[off + i] = lds[px[i - y * nx] + pitch * py[y] + shift];
+        }
+    };
+    double2 a[KP], b[KP];
+    load(w1, 0);
+    if constexpr (KIND == kDivergence && DUAL) load(w2, half);
+    __syncthreads();
+    lines(fwd, KIND == kDivergence && DUAL ? 2 : 1);
+    if constexpr (KIND == kDivergence && !DUAL) {
+#pragma unroll
+        for (int k = 0; k < KP; ++k) {
+            const int i = tid + k * nthr, y = fdiv(i, nx, mx);
+            if (i < np) a[k] = lds[px[i - y * nx] + pitch * py[y]];
+        }
+        __syncthreads();
+        load(w2, 0);
+        __syncthreads();
+        lines(fwd, 1);
+    }
+#pragma unroll
+    for (int k = 0; k < KP; ++k) {
+        const int i = tid + k * nthr;
+        if (i >= np) continue;
+        const int y = fdiv(i, nx, mx), x = i - y * nx;
+        const double2* l = lds + px[x] + pitch * py[y];
+        const double3 q = deriv_g(x, y, blockIdx.x, g);
+        if constexpr (KIND == kHartree) {
+            const double f = kern[off + i] * scale;
+            a[k] = make_double2(f * l->x, f * l->y);
+        } else if constexpr (KIND == kGradient) {
+            const double f = q.z + s * kern[off + i];
+            const double2 v = make_double2(l->x * scale, l->y * scale);
+            a[k] = make_double2(-q.y * v.x - q.x * v.y, q.x * v.x - q.y * v.y);
+            b[k] = make_double2(-f * v.y, f * v.x);
         } else {
+            const double2 p = DUAL ? l[0] : a[k], r = DUAL ? l[half] : l[0];
+            const double2 v = make_double2(p.x * scale, p.y * scale), u = make_double2(r.x * scale, r.y * scale);
+            a[k] = make_double2(q.y * v.x - q.x * v.y - q.z * u.y, q.x * v.x + q.y * v.y + q.z * u.x);
+        }
+    }
+    __syncthreads();
+    auto put = [&](const double2 (&v)[KP], int shift) {
+#pragma unroll
+        for (int k = 0; k < KP; ++k) {
+            const int i = tid + k * nthr, y = fdiv(i, nx, mx);
+            if (i < np) lds[i - y * nx + pitch * y + shift] = v[k];
+        }
+    };
+    put(a, 0);
+    if constexpr (KIND == kGradient && DUAL) put(b, half);
+    __syncthreads();
+    lines(inv, KIND == kGradient && DUAL ? 2 : 1);
+    store(w1, 0);
+    if constexpr (KIND == kGradient) {
+        if constexpr (!DUAL) {
+            __syncthreads();
+            put(b, 0);
+            __syncthreads();
+            lines(inv, 1);
+        }
+        store(w2, DUAL ? half : 0);
+    }
+}
+
+// Columns of one z-pass workgroup (one y): kZCols of the first field, then as many of the second.  At the
+// longest axis (256) the tile is 72 KiB.
+constexpr int kZCols = 8, kZThreads = 256, kZPitch = 2 * kZCols + 1;
+struct ZCols {
+    int nx, y, x0, cols, cnt, ny;
+    __device__ __forceinline__ ZCols(const GridAxes& g)
+        : nx(g.ax.n), y(blockIdx.y), x0(blockIdx.x * kZCols), cols(min(kZCols, g.ax.n - (int)blockIdx.x * kZCols)),
+          cnt(kZCols * g.az.n), ny(g.ay.n) {}
+    __device__ __forceinline__ bool in(int i) const { return i % kZCols < cols; }
+    __device__ __forceinline__ size_t at(int i) const {
+        return (size_t)(x0 + i % kZCols) + (size_t)nx * (y + (size_t)ny * (i / kZCols));
+    }
+};
+
+// z-pass of the density, forward: w = FFT_z(rho).
+__global__ __launch_bounds__(kZThreads) void k_rho_z(const double* __restrict__ rho, double2* __restrict__ w, GridAxes g) {
+    extern __shared__ double2 lds[];
+    const ZCols c(g);
+    const int nz = g.az.n, tid = threadIdx.x;
+    const int* pz = g.perm + g.az.perm_off;
+    double2* tw = lds + kZPitch * nz;
+    load_twiddles(tw, g.tw + g.az.tw_off, nz, tid, kZThreads);
+    for (int i = tid; i < c.cnt; i += kZThreads)
+        lds[i % kZCols + kZPitch * (i / kZCols)] = make_double2(c.in(i) ? rho[c.at(i)] : 0.0, 0.0);
+    __syncthreads();
+    lds_fft_lines<double, double2, false, -1>(lds, g.az, tw, LineSet{kZCols, kZPitch, 1, nullptr}, tid, kZThreads);
+    for (int i = tid; i < c.cnt; i += kZThreads)
+        if (c.in(i)) w[c.at(i)] = lds[i % kZCols + kZPitch * pz[i / kZCols]];
+}
+
+// z-pass in r space: V_H (and the gradient), the functional at every point, the workgroup's sums
+// [V_H rho, f_xc, v_in rho, (rho - rho_in)^2], and, GGA, b's z-transforms back into w1 and w2.
+// vout = V_H + df/dn (LDA: V_H + v_xc).
+template <bool GGA>
+__global__ __launch_bounds__(kZThreads) void k_xc_z(double2* __restrict__ w1, double2* __restrict__ w2,
+                                                    const double* __restrict__ rho, const double* __restrict__ rho_in,
+                                                    const double* __restrict__ vin, double* __restrict__ vout,
+                                                    double* __restrict__ part, double inv_s, GridAxes g) {
+    extern __shared__ double2 lds[];
+    __shared__ double red[4][kZThreads / 64];
+    const ZCols c(g);
+    const int nz = g.az.n, tid = threadIdx.x;
+    const int* pz = g.perm + g.az.perm_off;
+    double2* tw = lds + kZPitch * nz;
+    load_twiddles(tw, g.tw + g.az.tw_off, nz, tid, kZThreads);
+    for (int i = tid; i < c.cnt; i += kZThreads) {
+        double2* l = lds + i % kZCols + kZPitch * pz[i / kZCols];
+        const bool in = c.in(i);
+        l[0] = in ? w1[c.at(i)] : make_double2(0.0, 0.0);
+        if constexpr (GGA) l[kZCols] = in ? w2[c.at(i)] : make_double2(0.0, 0.0);
+    }
+    __syncthreads();
+    lds_fft_lines<double, double2, true, 1>(lds, g.az, tw, LineSet{GGA ? 2 * kZCols : kZCols, kZPitch, 1, nullptr}, tid,
+                                            kZThreads);
+    double sums[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+    for (int i = tid; i < c.cnt; i += kZThreads) {
+        if (!c.in(i)) continue;
+        double2* l = lds + i % kZCols + kZPitch * (i / kZCols);
+        const size_t at = c.at(i);
+        const double r = rho[at];
+        double f, v, h;
+        if constexpr (GGA) {
+            const double gx = l[0].x, gy = l[0].y, gz = l[kZCols].x;
+            double fg;
+            h = l[kZCols].y * inv_s;
+            pbe(r, gx * gx + gy * gy + gz * gz, &f, &v, &fg);
+            l[0] = make_double2(fg * gx, fg * gy);
+            l[kZCols] = make_double2(fg * gz, 0.0);
+        } else {
+            h = l[0].x;
             lda_pz(r, &f, &v);
         }
-        const double h = vh[i].x;
-        vout[i] = h + v;
-        s0 += h * r;
-        s1 += f;
-        s2 += vin[i] * r;
-        const double d = r - rho_in[i];
-        s3 += d * d;
+        vout[at] = h + v;
+        const double d = r - rho_in[at];
+        sums[0] += h * r;
+        sums[1] += f;
+        sums[2] += vin[at] * r;
+        sums[3] += d * d;
     }
-    red[0][threadIdx.x] = s0;
-    red[1][threadIdx.x] = s1;
-    red[2][threadIdx.x] = s2;
-    red[3][threadIdx.x] = s3;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) sums[k] += __shfl_xor(sums[k], o, 64);
+        if ((tid & 63) == 0) red[k][tid >> 6] = sums[k];
+    }
     __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int c = 0; c < 4; ++c) red[c][threadIdx.x] += red[c][threadIdx.x + w];
-        __syncthreads();
+    if (tid < 4) {
+        double s = 0.0;
+        for (int q = 0; q < kZThreads / 64; ++q) s += red[tid][q];
+        part[4 * (blockIdx.x + gridDim.x * blockIdx.y) + tid] = s;
     }
-    if (threadIdx.x < 4) part[4 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
+    if constexpr (GGA) {
+        lds_fft_lines<double, double2, false, -1>(lds, g.az, tw, LineSet{2 * kZCols, kZPitch, 1, nullptr}, tid, kZThreads);
+        for (int i = tid; i < c.cnt; i += kZThreads) {
+            if (!c.in(i)) continue;
+            const double2* l = lds + i % kZCols + kZPitch * pz[i / kZCols];
+            w1[c.at(i)] = l[0];
+            w2[c.at(i)] = l[kZCols];
+        }
+    }
+}
+
+// z-pass of the divergence: vout -= 2 Re(div b).
+__global__ __launch_bounds__(kZThreads) void k_div_z(const double2* __restrict__ w, double* __restrict__ vout, GridAxes g) {
+    extern __shared__ double2 lds[];
+    const ZCols c(g);
+    const int nz = g.az.n, tid = threadIdx.x;
+    const int* pz = g.perm + g.az.perm_off;
+    double2* tw = lds + kZPitch * nz;
+    load_twiddles(tw, g.tw + g.az.tw_off, nz, tid, kZThreads);
+    for (int i = tid; i < c.cnt; i += kZThreads)
+        lds[i % kZCols + kZPitch * pz[i / kZCols]] = c.in(i) ? w[c.at(i)] : make_double2(0.0, 0.0);
+    __syncthreads();
+    lds_fft_lines<double, double2, true, 1>(lds, g.az, tw, LineSet{kZCols, kZPitch, 1, nullptr}, tid, kZThreads);
+    for (int i = tid; i < c.cnt; i += kZThreads)
+        if (c.in(i)) vout[c.at(i)] -= 2.0 * lds[i % kZCols + kZPitch * (i / kZCols)].x;
 }
 
 // part[b] = sum over block b of a[i] * c[i] (fixed order, reduced on the host).
@@ -319,61 +480,69 @@ double ScfGrid::dot(const double* a, const double* c) {
     return reduce(part.as<double>(), kRedBlocks, 1, 0);
 }
 
-void ScfGrid::gga(const double* rho) {
-    hipStream_t s = stream();
-    const unsigned nb = grid_blocks(n);
-    double* gc[3] = {grad.as<double>(), grad.as<double>() + n, grad.as<double>() + 2 * n};
-    double2* w = work.as<double2>();
-    double2* w2 = work2.as<double2>();
-    // grad n = IFFT(i G FFT(n)), real part kept.
-    hipLaunchKernelGGL(k_real_to_complex, dim3(nb), dim3(256), 0, s, rho, w, n);
-    DZ_HIP(hipGetLastError());
-    fft3d_device<double>(w, tab, false, s);
-    for (int c = 0; c < 3; ++c) {
-        hipLaunchKernelGGL(k_grad_comp, dim3(nb), dim3(256), 0, s, w, w2, c, nx, ny, nz, recip_rows[0], recip_rows[1],
-                           recip_rows[2]);
-        DZ_HIP(hipGetLastError());
-        fft3d_device<double>(w2, tab, true, s);
-        hipLaunchKernelGGL(k_real_part, dim3(nb), dim3(256), 0, s, w2, gc[c], n);
-        DZ_HIP(hipGetLastError());
-    }
-    hipLaunchKernelGGL(k_pbe_point, dim3(nb), dim3(256), 0, s, rho, gc[0], gc[1], gc[2], gga_f.as<double>(),
-                       gga_v.as<double>(), n);
-    DZ_HIP(hipGetLastError());
-    // div b = IFFT(sum_c i G_c FFT(b_c)), then v_xc = df/dn - 2 Re(div b).
-    for (int c = 0; c < 3; ++c) {
-        hipLaunchKernelGGL(k_real_to_complex, dim3(nb), dim3(256), 0, s, gc[c], w, n);
-        DZ_HIP(hipGetLastError());
-        fft3d_device<double>(w, tab, false, s);
-        hipLaunchKernelGGL(k_div_acc, dim3(nb), dim3(256), 0, s, w, w2, c, c == 0 ? 1 : 0, nx, ny, nz,
-                           recip_rows[0], recip_rows[1], recip_rows[2]);
-        DZ_HIP(hipGetLastError());
-    }
-    fft3d_device<double>(w2, tab, true, s);
-    hipLaunchKernelGGL(k_gga_combine, dim3(nb), dim3(256), 0, s, gga_v.as<double>(), w2, n);
+namespace {
+// Threads and points per thread of an xy-pass by the plane's points (its tile fits LDS: at most 10,240).
+template <int KIND>
+void launch_gridxy(int nx, int ny, int nz, hipStream_t s, double2* w1, double2* w2, const double* kern, double sc,
+                   double scale, const GridAxes& g) {
+    const int np = nx * ny;
+    size_t lds = fft_xy_lds_bytes(nx, ny, sizeof(double2));
+    const size_t lds2 = lds + (size_t)(nx + 1) * ny * sizeof(double2);
+    const bool dual = KIND != kHartree && lds2 <= kMaxLdsBytes;
+    if (dual) lds = lds2;
+    constexpr bool D = KIND != kHartree;
+    auto* fn = dual ? (np <= 1024 ? k_gridxy<KIND, 4, D> : k_gridxy<KIND, 12, D>)
+                    : (np <= 1024   ? k_gridxy<KIND, 4, false>
+                       : np <= 6144 ? k_gridxy<KIND, 12, false>
+                                    : k_gridxy<KIND, 20, false>);
+    set_max_dynamic_lds((const void*)fn, lds);
+    hipLaunchKernelGGL(fn, dim3((unsigned)nz), dim3(np <= 1024 ? 256 : 512), lds, s, w1, w2, kern, sc, scale, g);
     DZ_HIP(hipGetLastError());
 }
+}  // namespace
 
-void ScfGrid::hxc(const double* rho, const double* rho_ref, const double* vin, double* vout, double out[4]) {
+void ScfGrid::hxc(const double* rho, const double* rho_ref, const double* vin, double* vout, double* out) {
     hipStream_t s = stream();
-    if (xc == DZHIP_XC_PBE) gga(rho);
-    hipLaunchKernelGGL(k_real_to_complex, dim3(grid_blocks(n)), dim3(256), 0, s, rho, work.as<double2>(), n);
+    const bool gga = xc == DZHIP_XC_PBE;
+    const GridAxes g{tab.ax[0], tab.ax[1], tab.ax[2], tab.tw64, tab.perm, recip_rows[0], recip_rows[1], recip_rows[2]};
+    // The tiles of the plan's own passes bound the grids taken.
+    DZ_REQUIRE(fft_xy_lds_bytes(nx, ny, sizeof(double2)) <= kMaxLdsBytes &&
+                   fft_z_lds_bytes(nx, nz, sizeof(double2)) <= kMaxLdsBytes,
+               DZHIP_ERR_HIP, "SCF grid: plane too large for the FFT kernels' LDS");
+    double2 *w1 = work.as<double2>(), *w2 = work2.as<double2>();
+    double *kern = hartree.as<double>(), *sums = part.as<double>();
+    // s V_H is at most about n, as the gradient of a valence density (a bohr's scale) is.
+    double g2min = 1e300;
+    for (const double3& b : recip_rows) g2min = std::min(g2min, b.x * b.x + b.y * b.y + b.z * b.z);
+    const double sc = std::exp2(std::rint(std::log2(g2min / (8.0 * M_PI))));
+    const double scale = 1.0 / (double)n;
+    const dim3 gz((unsigned)((nx + kZCols - 1) / kZCols), (unsigned)ny);
+    const size_t ldsz = (size_t)(kZPitch + 1) * nz * sizeof(double2);
+    set_max_dynamic_lds((const void*)k_rho_z, ldsz);
+    hipLaunchKernelGGL(k_rho_z, gz, dim3(kZThreads), ldsz, s, rho, w1, g);
     DZ_HIP(hipGetLastError());
-    fft3d_device<double>(work.as<double2>(), tab, false, s);
-    hipLaunchKernelGGL(k_hartree_kernel, dim3(grid_blocks(n)), dim3(256), 0, s, work.as<double2>(), g2.as<double>(), n);
-    DZ_HIP(hipGetLastError());
-    fft3d_device<double>(work.as<double2>(), tab, true, s);
-    part.ensure(4 * kRedBlocks * sizeof(double));
-    const bool is_gga = xc == DZHIP_XC_PBE;
-    hipLaunchKernelGGL(k_hxc, dim3(kRedBlocks), dim3(kRedThreads), 0, s, work.as<double2>(), rho, rho_ref, vin,
-                       is_gga ? gga_f.as<double>() : nullptr, is_gga ? gga_v.as<double>() : nullptr, vout,
-                       part.as<double>(), n);
-    DZ_HIP(hipGetLastError());
-    std::vector<double> h((size_t)kRedBlocks * 4);
+    if (gga) {
+        launch_gridxy<kGradient>(nx, ny, nz, s, w1, w2, kern, sc, scale, g);
+        set_max_dynamic_lds((const void*)k_xc_z<true>, ldsz);
+        hipLaunchKernelGGL(k_xc_z<true>, gz, dim3(kZThreads), ldsz, s, w1, w2, rho, rho_ref, vin, vout, sums, 1.0 / sc, g);
+        DZ_HIP(hipGetLastError());
+        launch_gridxy<kDivergence>(nx, ny, nz, s, w1, w2, kern, sc, scale, g);
+        set_max_dynamic_lds((const void*)k_div_z, ldsz);
+        hipLaunchKernelGGL(k_div_z, gz, dim3(kZThreads), ldsz, s, w1, vout, g);
+        DZ_HIP(hipGetLastError());
+    } else {
+        launch_gridxy<kHartree>(nx, ny, nz, s, w1, w2, kern, sc, scale, g);
+        set_max_dynamic_lds((const void*)k_xc_z<false>, ldsz);
+        hipLaunchKernelGGL(k_xc_z<false>, gz, dim3(kZThreads), ldsz, s, w1, w2, rho, rho_ref, vin, vout, sums, 1.0, g);
+        DZ_HIP(hipGetLastError());
+    }
+    if (!out) return;
+    const size_t nparts = (size_t)gz.x * gz.y;
+    std::vector<double> h(nparts * 4);
     DZ_HIP(hipMemcpyAsync(h.data(), part.ptr, h.size() * sizeof(double), hipMemcpyDeviceToHost, s));
     DZ_HIP(hipStreamSynchronize(s));
     double t[4] = {0, 0, 0, 0};
-    for (int i = 0; i < kRedBlocks; ++i)
+    for (size_t i = 0; i < nparts; ++i)
         for (int c = 0; c < 4; ++c) t[c] += h[4 * i + c];
     const double dv = volume / (double)n;
     out[0] = 0.5 * t[0] * dv;
@@ -396,7 +565,9 @@ ScfGrid* scf_grid_create(Context* ctx, int nx, int ny, int nz, const double* rec
         g->tab.build(nx, ny, nz);
         const size_t n = g->n;
         g->g2.ensure(n * sizeof(double));
+        g->hartree.ensure(n * sizeof(double));
         g->work.ensure(n * sizeof(double2));
+        g->part.ensure(4 * std::max<size_t>((size_t)ny * ((nx + kZCols - 1) / kZCols), kRedBlocks) * sizeof(double));
         DevBuf* bufs[] = {&g->rho_in, &g->rho_out, &g->v_in, &g->v_out, &g->v_ion, &g->local};
         for (DevBuf* b : bufs) b->ensure(n * sizeof(double));
         if (history > 0) {
@@ -407,7 +578,7 @@ ScfGrid* scf_grid_create(Context* ctx, int nx, int ny, int nz, const double* rec
         }
         g->b.assign(std::max(history, 1), std::vector<double>(std::max(history, 1), 0.0));
         hipStream_t s = g->stream();
-        hipLaunchKernelGGL(k_g2, dim3(grid_blocks(n)), dim3(256), 0, s, g->g2.as<double>(), nx, ny, nz,
+        hipLaunchKernelGGL(k_g2, dim3(grid_blocks(n)), dim3(256), 0, s, g->g2.as<double>(), g->hartree.as<double>(), nx, ny, nz,
                            make_double3(recip[0], recip[1], recip[2]), make_double3(recip[3], recip[4], recip[5]),
                            make_double3(recip[6], recip[7], recip[8]));
         DZ_HIP(hipGetLastError());
@@ -424,7 +595,7 @@ ScfGrid* scf_grid_create(Context* ctx, int nx, int ny, int nz, const double* rec
 void scf_grid_destroy(ScfGrid* g) {
     if (!g) return;
     DevBuf* bufs[] = {&g->g2, &g->work, &g->rho_in, &g->rho_out, &g->v_in, &g->v_out, &g->v_ion, &g->local,
-                      &g->part, &g->hv, &g->hr, &g->slots, &g->coef, &g->work2, &g->grad, &g->gga_f, &g->gga_v};
+                      &g->part, &g->hv, &g->hr, &g->slots, &g->coef, &g->work2, &g->hartree};
     for (DevBuf* b : bufs) b->release();
     g->tab.release();
     delete g;
@@ -438,9 +609,8 @@ void scf_grid_init(ScfGrid& g, double nelec, const double* rho_host) {
         hipLaunchKernelGGL(k_fill, dim3(grid_blocks(g.n)), dim3(256), 0, s, g.rho_in.as<double>(), nelec / g.volume, g.n);
         DZ_HIP(hipGetLastError());
     }
-    double e[4];
-    // v_in = V_Hxc[rho_in]; the reference arguments for rho_ref/vin only feed the unused sums.
-    g.hxc(g.rho_in.as<double>(), g.rho_in.as<double>(), g.rho_in.as<double>(), g.v_in.as<double>(), e);
+    // v_in = V_Hxc[rho_in]; the reference arguments for rho_ref/vin only feed the sums, not read here.
+    g.hxc(g.rho_in.as<double>(), g.rho_in.as<double>(), g.rho_in.as<double>(), g.v_in.as<double>(), nullptr);
     g.order.clear();
     hipLaunchKernelGGL(k_fill, dim3(grid_blocks(g.n)), dim3(256), 0, s, g.rho_out.as<double>(), 0.0, g.n);
     DZ_HIP(hipGetLastError());
@@ -576,9 +746,6 @@ void scf_grid_mix(ScfGrid& g, double beta, int pulay) {
 void scf_grid_set_xc(ScfGrid& g, int functional) {
     if (functional == DZHIP_XC_PBE) {
         g.work2.ensure(g.n * sizeof(double2));
-        g.grad.ensure(3 * g.n * sizeof(double));
-        g.gga_f.ensure(g.n * sizeof(double));
-        g.gga_v.ensure(g.n * sizeof(double));
     }
     g.xc = functional;
 }

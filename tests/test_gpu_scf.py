@@ -193,6 +193,36 @@ def test_scf_grid_potential_matches_host(dz, ctx, system):
         drv.close()
 
 
+# Planes of up to 1,024 points, of two tiles in LDS, of one (two sizes), odd and even lengths, columns
+# that are no multiple of eight, and the longest axes.
+@pytest.mark.parametrize("xc", ["lda_pz", "pbe"])
+@pytest.mark.parametrize("shape", [(1, 1, 2), (5, 3, 9), (16, 15, 18), (30, 36, 25), (72, 81, 5), (90, 100, 3),
+                                   (4, 4, 256), (256, 9, 2)])
+def test_scf_grid_potential_shapes(dz, ctx, shape, xc):
+    """V_H + V_xc of a few low harmonics in an oblique cell of 0.4 bohr a point, against the oracle.
+    1e-11 of max |V|: the divergence amplifies rounding by |G|max^2 ~ 100, the paired V_H by the
+    cell's 8 pi / G_min^2 (4e-13 at the longest axis)."""
+    cell = 0.4 * np.diag(shape).astype(float)
+    cell[1, 0], cell[2, 1] = 0.1 * cell[0, 0], 0.2 * cell[1, 1]
+    recip = 2.0 * np.pi * np.linalg.inv(cell).T
+    volume = abs(np.linalg.det(cell))
+    x, y, z = np.meshgrid(*[np.arange(n) / n for n in shape], indexing="ij")
+    rho = 0.05 + 0.015 * np.cos(2 * np.pi * (x + 0.1)) * np.cos(2 * np.pi * y) + 0.02 * np.sin(2 * np.pi * (z + 0.3 + x))
+    rho = rho.transpose(2, 1, 0).reshape(-1)
+    vh, eh = oscf.hartree(rho, shape, recip, volume)
+    f, vx = oscf.xc_fields(rho, shape, recip, xc)
+    g = dz.ScfGrid(ctx, shape, recip, volume)
+    try:
+        g.set_xc(xc)
+        g.init_rho(rho)
+        got = g.read(dz.GRID_VIN)
+        scale = np.max(np.abs(vh + vx))
+        print("error", np.max(np.abs(got - vh - vx)) / scale)
+        np.testing.assert_allclose(got, vh + vx, rtol=0, atol=1e-11 * scale)
+    finally:
+        g.close()
+
+
 @pytest.mark.parametrize("concurrent,device_grid", [(False, False), (True, True)])
 def test_scf_smearing_al(dz, ctx, concurrent, device_grid):
     """Fermi-Dirac smearing (fermi_level.zig, kpoint/density.zig:398-404) on fcc Al, 8 k-points
