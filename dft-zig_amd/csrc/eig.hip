@@ -456,143 +456,150 @@ static void section_times(EigWork& w, double* out) {
 // into Y (leading dimension ldy) and the host vector returned (ascending).  The library's device
 // eigensolver up to m = kHeevMaxM; rocSOLVER zheevd beyond (it overwrites a copy of A in Y,
 // which must then hold m columns).
-// Upper Cholesky factorisation A = R^H R of a Hermitian k x k matrix (column-major, leading
-// dimension lda; the upper triangle is read and overwritten with R, the lower one is left alone),
-// k <= kPotrfMax, one workgroup of 256 threads, right-looking in blocks of kPotrfNb rows:
-//   1. the diagonal block by wavefront 0, lane l holding column l of it in registers; the row
-//      R[j, :] of each step reaches the other lanes by lane shuffles;
-//   2. the block's rows of R right of it, R_d^{-H} A[block, rest] by forward substitution, one
-//      thread per column (the rows also go to LDS);
-//   3. the trailing upper triangle minus the Gram products of those rows, 4 x 4 tiles per thread.
-// *info = 0, or j + 1 for the first pivot j that is not positive (the factorisation stops there),
-// as LAPACK's zpotrf reports it.
+// Upper Cholesky factorisation S = R^H R of a Hermitian k x k matrix (column-major, leading dimension
+// ld; the upper triangle of S is read, A gets R and zeros below it), k <= kPotrfMax, one workgroup,
+// right-looking in blocks of kPotrfNb rows:
+//   1. the block's rows, one column of them per thread in registers: a step posts row j of the diagonal
+//      block in LDS and every column, in the diagonal block or right of it, eliminates with it (one
+//      barrier a step; the next step's row is posted before the rest of the update);
+//   2. the trailing upper triangle minus the Gram products of those rows (in LDS) on the matrix cores,
+//      16 x 16 tiles per wavefront; the next block's rows stay in LDS.
+// info[0] = 0, or j + 1 for the first pivot j that is not positive (the factorisation stops there), as
+// LAPACK's zpotrf reports it.  info[1] = 1 when it succeeded and every pivot keeps at least 1e-7 of its
+// column's norm (R_jj > 1e-7 sqrt(S_jj)).
+// The steps' chain bounds it (k of them: an LDS round trip, a reciprocal square root, a barrier).
+// k = 24: 13 us, k = 164: 106 us (26 and 261 with wavefront 0 alone on the diagonal block by lane
+// shuffles, substitution as a second phase and 4 x 4 tiles a thread with uncoalesced updates, a copy
+// of S before and a check kernel after not counted).
 constexpr int kPotrfMax = 256;
 constexpr int kPotrfNb = 16;
-__global__ __launch_bounds__(256) void k_potrf_upper(double2* __restrict__ A, int lda, int k, int* __restrict__ info) {
-    __shared__ double2 dblk[kPotrfNb][kPotrfNb];              // R of the diagonal block [row][column]
-    __shared__ double2 rows[kPotrfNb][kPotrfMax - kPotrfNb];  // its rows right of it [row][column - c0]
-    __shared__ int s_fail;
-    const int tid = (int)threadIdx.x;
-    if (tid == 0) {
-        s_fail = 0;
-        *info = 0;
+constexpr int kPanelPitch = kPotrfNb + 1;
+static __host__ __device__ int potrf_row_pitch(int k) { return (k > kPotrfNb ? (k - 1) / 16 * 16 : 0) + 1; }
+static size_t potrf_lds_bytes(int k) {
+    return ((size_t)kPotrfNb * potrf_row_pitch(k) + (size_t)kPanelPitch * k) * sizeof(double2);
+}
+// 1 / sqrt(d): the hardware's estimate (relative error about 1e-8) and one third-order Newton step.
+static __device__ __forceinline__ double rsqrt_newton(double d) {
+    const double r = __builtin_amdgcn_rsq(d);
+    const double e = fma(-(d * r), r, 1.0);
+    return fma(r * e, fma(0.375, e, 0.5), r);
+}
+__global__ __launch_bounds__(512) void k_potrf_upper(const double2* S, double2* A, int ld, int k,
+                                                     int* __restrict__ info) {
+    extern __shared__ double2 lds[];
+    __shared__ double2 urow[2][kPotrfNb];  // row j of the diagonal block before its scaling
+    __shared__ int s_fail, s_bad;
+    const int tid = (int)threadIdx.x, nthr = (int)blockDim.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, l4 = lane >> 4;
+    const int P = potrf_row_pitch(k);
+    double2* rows = lds;                   // R right of the diagonal block [row][column - c0], pitch P
+    double2* panel = lds + kPotrfNb * P;   // the next block's rows before elimination [column - jb][row]
+    if (tid == 0) s_fail = s_bad = 0;
+    for (int e = tid; e < kPotrfNb * k; e += nthr) {
+        const int i = e & 15, c = e >> 4;
+        panel[c * kPanelPitch + i] = i < k ? S[(size_t)c * ld + i] : double2{0.0, 0.0};
     }
     __syncthreads();
+    int failed = 0;
     for (int jb = 0; jb < k; jb += kPotrfNb) {
-        const int nb = min(kPotrfNb, k - jb);
-        if (tid < 64) {
-            const int l = tid;
-            double2 col[kPotrfNb];  // A[jb + i][jb + l], i <= l
+        const int w = k - jb, nb = min(kPotrfNb, w), c0 = jb + nb, m = w - nb, mt = (m + 15) / 16;
+        const bool active = (tid & ~63) < w;  // the wavefront has columns
+        double2 col[kPotrfNb];                // A[jb + i][jb + tid]
+        double rjj = 0.0, gjj = 0.0;
+        int fail = 0;
+        if (active) {
 #pragma unroll
             for (int i = 0; i < kPotrfNb; ++i)
-                col[i] = (l < nb && i <= l) ? A[(size_t)(jb + l) * lda + jb + i] : double2{0.0, 0.0};
-            int fail = 0;
-#pragma unroll
-            for (int j = 0; j < kPotrfNb; ++j) {
-                if (j < nb && fail == 0) {  // uniform over the wavefront
-                    const double d = __shfl(col[j].x, j);
-                    if (!(d > 0.0)) {
-                        fail = jb + j + 1;
-                    } else {
-                        const double r = sqrt(d), inv = 1.0 / r;
-                        if (l == j) col[j] = double2{r, 0.0};
-                        if (l > j) col[j] = double2{col[j].x * inv, col[j].y * inv};  // R[j][l]
-                        // A[i][l] -= conj(R[j][i]) R[j][l] for j < i <= l
-#pragma unroll
-                        for (int i = j + 1; i < kPotrfNb; ++i) {
-                            const double rx = __shfl(col[j].x, i), ry = __shfl(col[j].y, i);  // R[j][i]
-                            if (l >= i && l < nb) {
-                                col[i].x -= rx * col[j].x + ry * col[j].y;
-                                col[i].y -= rx * col[j].y - ry * col[j].x;
-                            }
-                        }
-                    }
-                }
-            }
-            if (l < nb) {
-#pragma unroll
-                for (int i = 0; i < kPotrfNb; ++i) {
-                    if (i <= l) {
-                        A[(size_t)(jb + l) * lda + jb + i] = col[i];
-                        dblk[i][l] = col[i];
-                    }
-                }
-            }
-            if (l == 0 && fail) {
-                s_fail = fail;
-                *info = fail;
+                col[i] = tid < w && i < nb ? panel[tid * kPanelPitch + i] : double2{0.0, 0.0};
+            if (tid < nb) {
+                urow[0][tid] = col[0];
+                gjj = S[(size_t)(jb + tid) * (ld + 1)].x;
             }
         }
         __syncthreads();
-        if (s_fail) return;
-        const int c0 = jb + nb, m = k - c0;
-        if (m <= 0) break;
-        // Rows of R right of the block: solve R_d^H y = A[jb:jb+nb, c] for each column c.
-        if (tid < m) {
-            const int c = c0 + tid;
-            double2 y[kPotrfNb];
 #pragma unroll
-            for (int i = 0; i < kPotrfNb; ++i) {
-                if (i < nb) {
-                    double2 v = A[(size_t)c * lda + jb + i];
-#pragma unroll
-                    for (int t = 0; t < i; ++t) {  // v -= conj(R_d[t][i]) y[t]
-                        const double2 r = dblk[t][i];
-                        v.x -= r.x * y[t].x + r.y * y[t].y;
-                        v.y -= r.x * y[t].y - r.y * y[t].x;
+        for (int j = 0; j < kPotrfNb; ++j) {
+            if (j < nb) {
+                if (active) {
+                    const double2* u = urow[j & 1];
+                    const double d = u[j].x, rs = rsqrt_newton(d);
+                    fail = fail == 0 && !(d > 0.0) ? jb + j + 1 : fail;
+                    double2 t{col[j].x * rs, col[j].y * rs};  // R[j][c]
+                    if (tid == j) {
+                        t = double2{d * rs, 0.0};
+                        rjj = t.x;
                     }
-                    const double inv = 1.0 / dblk[i][i].x;
-                    y[i] = double2{v.x * inv, v.y * inv};
-                    A[(size_t)c * lda + jb + i] = y[i];
-                    rows[i][tid] = y[i];
+                    col[j] = t;
+                    const double2 v{t.x * rs, t.y * rs};
+                    // A[i][c] -= conj(R[j][i]) R[j][c], R[j][i] = u[i] rs
+#pragma unroll
+                    for (int i = j + 1; i < kPotrfNb; ++i) {
+                        col[i].x -= u[i].x * v.x + u[i].y * v.y;
+                        col[i].y -= u[i].x * v.y - u[i].y * v.x;
+                        if (i == j + 1 && tid < kPotrfNb) urow[(j + 1) & 1][tid] = col[i];
+                    }
                 }
+                __syncthreads();
             }
         }
+        if (active) {
+            if (tid < nb) {
+                if (!(rjj > 1e-7 * sqrt(fmax(gjj, 0.0)))) s_bad = 1;
+#pragma unroll
+                for (int i = 0; i < kPotrfNb; ++i)
+                    if (i < nb) A[(size_t)(jb + tid) * ld + jb + i] = i <= tid ? col[i] : double2{0.0, 0.0};
+            } else if (tid >= kPotrfNb && tid < kPotrfNb * (1 + mt)) {  // zeros up to the last tile's edge
+#pragma unroll
+                for (int i = 0; i < kPotrfNb; ++i) rows[i * P + tid - kPotrfNb] = col[i];
+            }
+            if (tid == 0) s_fail = fail;
+        }
         __syncthreads();
-        // Trailing upper triangle: A[i][c] -= sum_t conj(R[t][i]) R[t][c], c0 <= i <= c < k, in
-        // 4 x 4 tiles (ti <= tc) per thread: eight LDS reads per t feed 16 complex products.
-        const int nt = (m + 3) >> 2, ntiles = nt * (nt + 1) / 2;
-        for (int e = tid; e < ntiles; e += 256) {
-            int tc = (int)((sqrt(8.0 * e + 1.0) - 1.0) * 0.5);  // tile column: tc (tc + 1) / 2 <= e
-            while (tc * (tc + 1) / 2 > e) --tc;
-            while ((tc + 1) * (tc + 2) / 2 <= e) ++tc;
-            const int ti = e - tc * (tc + 1) / 2;
-            double2 acc[4][4];
+        failed = s_fail;
+        if (failed || m <= 0) break;
+        for (int e = tid; e < kPotrfNb * m; e += nthr) {
+            const int i = e & 15, c = e >> 4;
+            A[(size_t)(c0 + c) * ld + jb + i] = rows[i * P + c];
+        }
+        for (int c = wave; c < kPotrfNb; c += nthr >> 6)
+            for (int i = lane; i < m; i += 64) A[(size_t)(jb + c) * ld + c0 + i] = double2{0.0, 0.0};
+        // Trailing upper triangle: A[i][c] -= sum_t conj(R[t][i]) R[t][c]; MFMA rows are columns c, MFMA
+        // columns rows i, so that a load or store takes 16 consecutive rows.
+        const double2* src = jb == 0 ? S : A;
+        for (int e = wave; e < mt * (mt + 1) / 2; e += nthr >> 6) {
+            int tc = 0, ti = e;  // tile column tc, row ti <= tc
+            while (ti > tc) ti -= ++tc;
+            const int i = 16 * ti + l16;
+            double2 o[4];
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+            for (int r = 0; r < 4; ++r) {
+                const int c = 16 * tc + l4 + 4 * r;
+                o[r] = src[(size_t)(c0 + min(c, m - 1)) * ld + c0 + min(i, m - 1)];
+            }
+            v4d_t re{0, 0, 0, 0}, im{0, 0, 0, 0};
 #pragma unroll
-                for (int b = 0; b < 4; ++b) acc[a][b] = double2{0.0, 0.0};
-            for (int t = 0; t < nb; ++t) {
-                double2 ri[4], rc[4];
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    const int i = 4 * ti + a, c = 4 * tc + a;
-                    ri[a] = i < m ? rows[t][i] : double2{0.0, 0.0};
-                    rc[a] = c < m ? rows[t][c] : double2{0.0, 0.0};
-                }
-#pragma unroll
-                for (int a = 0; a < 4; ++a)
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) {
-                        acc[a][b].x += ri[a].x * rc[b].x + ri[a].y * rc[b].y;
-                        acc[a][b].y += ri[a].x * rc[b].y - ri[a].y * rc[b].x;
-                    }
+            for (int t = 0; t < kPotrfNb; t += 4) {
+                const double2 a = rows[(t + l4) * P + 16 * tc + l16], b = rows[(t + l4) * P + 16 * ti + l16];
+                re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, re, 0, 0, 0);
+                im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.x, im, 0, 0, 0);
+                re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.y, re, 0, 0, 0);
+                im = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.x, b.y, im, 0, 0, 0);
             }
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int c = 4 * tc + b;
+            for (int r = 0; r < 4; ++r) {
+                const int c = 16 * tc + l4 + 4 * r;
+                const double2 v{o[r].x - re[r], o[r].y - im[r]};
                 if (c >= m) continue;
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    const int i = 4 * ti + a;
-                    if (i > c) continue;
-                    double2* p = A + (size_t)(c0 + c) * lda + c0 + i;
-                    const double2 v = *p;
-                    *p = double2{v.x - acc[a][b].x, v.y - acc[a][b].y};
-                }
+                if (ti == 0)
+                    panel[c * kPanelPitch + l16] = v;
+                else if (i <= c)
+                    A[(size_t)(c0 + c) * ld + c0 + i] = v;
             }
         }
         __syncthreads();
+    }
+    if (tid == 0) {
+        info[0] = failed;
+        info[1] = failed == 0 && s_bad == 0 ? 1 : 0;
     }
 }
 
@@ -760,17 +767,24 @@ struct Solver {
         return kk;
     }
 
-    // G = R^H R in place (upper triangle, leading dimension k), the verdict in w.info[0]: the
-    // library's one-workgroup factorisation up to kPotrfMax, rocSOLVER's zpotrf beyond.
-    void potrf_upper(double2* G, int k) {
+    // S = R^H R for the k x k Gram matrix in S (left as it is, leading dimension k), R -> G; the verdicts
+    // in w.info[0:2] as k_potrf_upper leaves them: the library's one-workgroup factorisation up to
+    // kPotrfMax, rocSOLVER's zpotrf beyond.
+    void potrf_upper(int k) {
         static_assert(sizeof(rocblas_int) == sizeof(int), "info is read as int");
+        double2 *S = w.S.as<double2>(), *G = w.G.as<double2>();
+        int* info = w.info.as<int>();
         if (k <= kPotrfMax) {
-            hipLaunchKernelGGL(k_potrf_upper, dim3(1), dim3(256), 0, s, G, k, k, w.info.as<int>());
-            DZ_HIP(hipGetLastError());
+            const size_t lds = potrf_lds_bytes(k);
+            set_max_dynamic_lds((const void*)k_potrf_upper, lds);
+            // More than 96 columns: enough tiles for eight wavefronts.
+            hipLaunchKernelGGL(k_potrf_upper, dim3(1), dim3(k > 96 ? 512 : 256), lds, s, S, G, k, k, info);
         } else {
-            DZ_BLAS(rocsolver_zpotrf(w.blas, rocblas_fill_upper, k, reinterpret_cast<zc*>(G), k,
-                                     w.info.as<rocblas_int>()));
+            DZ_HIP(hipMemcpyAsync(G, S, (size_t)k * k * sizeof(double2), hipMemcpyDeviceToDevice, s));
+            DZ_BLAS(rocsolver_zpotrf(w.blas, rocblas_fill_upper, k, reinterpret_cast<zc*>(G), k, info));
+            hipLaunchKernelGGL(k_chol_check, dim3(1), dim3(256), 0, s, S, G, k, info, info + 1);
         }
+        DZ_HIP(hipGetLastError());
     }
 
     // Orthonormalise Q[:, 0:k] in place: Cholesky QR, or, when the Gram matrix is not
@@ -781,17 +795,11 @@ struct Solver {
     // ones before it, and dividing by its pivot would turn rounding noise into a basis vector.
     int ortho_block(double2* Q, int k) {
         const int ldn = (int)n;
-        gram(Q, k, Q, k, w.G.as<double2>(), k);
-        DZ_HIP(hipMemcpyAsync(w.S.ptr, w.G.ptr, (size_t)k * k * sizeof(double2), hipMemcpyDeviceToDevice, s));
-        potrf_upper(w.G.as<double2>(), k);
-        // The factorisation's verdict on the device (info and every pivot against its column's norm,
-        // the latter from the copy in S), one int back to the host.
-        int* ok_dev = w.info.as<int>() + 1;
-        hipLaunchKernelGGL(k_chol_check, dim3(1), dim3(256), 0, s, w.S.as<double2>(), w.G.as<double2>(), k,
-                           w.info.as<rocblas_int>(), ok_dev);
-        DZ_HIP(hipGetLastError());
+        gram(Q, k, Q, k, w.S.as<double2>(), k);
+        potrf_upper(k);
+        // Decided on the device; one int back to the host.
         int ok = 0;
-        DZ_HIP(hipMemcpyAsync(&ok, ok_dev, sizeof(int), hipMemcpyDeviceToHost, s));
+        DZ_HIP(hipMemcpyAsync(&ok, w.info.as<int>() + 1, sizeof(int), hipMemcpyDeviceToHost, s));
         DZ_HIP(hipStreamSynchronize(s));
         const zc one(1.0, 0.0), zero(0.0, 0.0);
         if (ok) {
@@ -800,7 +808,7 @@ struct Solver {
             return k;
         }
         st.ortho_fallbacks++;
-        // Eigen-decomposition of the Gram matrix (its copy in S, lower triangle) into G.
+        // Eigen-decomposition of the Gram matrix (S, lower triangle) into G.
         const std::vector<double> lam = subspace_eigh(w, w.S.as<double2>(), k, k, k, w.G.as<double2>(), k, s);
         const double thr = 1e-12 * std::max(lam[k - 1], 0.0);
         int first = 0;
@@ -827,8 +835,8 @@ struct Solver {
     // Q <- Q R^{-1} with G = Q^H Q = R^H R.  Throws if G is not positive definite.
     void cholqr(double2* Q, int k) {
         const int ldn = (int)n;
-        gram(Q, k, Q, k, w.G.as<double2>(), k);
-        potrf_upper(w.G.as<double2>(), k);
+        gram(Q, k, Q, k, w.S.as<double2>(), k);
+        potrf_upper(k);
         rocblas_int info = 0;
         DZ_HIP(hipMemcpyAsync(&info, w.info.ptr, sizeof(info), hipMemcpyDeviceToHost, s));
         DZ_HIP(hipStreamSynchronize(s));

@@ -152,3 +152,25 @@ def test_eig_product_tiles(dz, ctx, nbands):
     ham.close()
     print(f"nbands={nbands} n={w.npw} it={st['iterations']} dv={np.max(np.abs(vals - ref)):.2e}", flush=True)
     assert st["converged"] == 1 and np.max(np.abs(vals - ref)) < 2e-8
+
+
+@pytest.mark.parametrize("k", [15, 16, 17, 33, 96, 97, 256, 257])
+def test_eig_cholesky_blocks(dz, ctx, k):
+    """Start blocks of k columns at the edges of the Cholesky factorisation's 16-row blocks, of its two
+    launch widths and of its range (257: rocSOLVER): eigenvalues against the dense eigh (2e-8 Ry, the
+    bar of this file) and orthonormal vectors (1e-12: Cholesky QR twice leaves a few eps sqrt(n))."""
+    from dzhip import workloads
+    from oracle import adapters, hamiltonian
+
+    w = workloads.si8(nbands=4)
+    h = hamiltonian.dense_hamiltonian(adapters.context_from_workload(w))
+    nbands = k - 4
+    ref = np.linalg.eigvalsh(0.5 * (h + h.conj().T))[:nbands]
+    ham = dz.Hamiltonian.from_workload(ctx, w)
+    vals, vecs, st = ham.eig_solve(nbands, tol=1e-7, max_iter=300, max_subspace=min(w.npw, 2 * k))
+    ham.close()
+    v = vecs.reshape(nbands, -1)
+    err = np.max(np.abs(v.conj() @ v.T - np.eye(nbands)))
+    print(f"k={k} n={w.npw} it={st['iterations']} dv={np.max(np.abs(vals - ref)):.2e} orth={err:.1e}", flush=True)
+    assert st["converged"] == 1 and st["ortho_fallbacks"] == 0
+    assert np.max(np.abs(vals - ref)) < 2e-8 and err < 1e-12
