@@ -368,6 +368,44 @@ __global__ void k_gather_cols(const double2* __restrict__ src, const int* __rest
     dst[(size_t)j * ld + i] = make_double2(v.x * s, v.y * s);
 }
 
+// New directions to keep: idx[0:k] (ascending), the columns whose norm after projection (n2, squared)
+// exceeds 1e-8 of the one before (n2_0), scl their 1 / norm; *kept = k.  One workgroup.  On the device
+// because only the count is needed by the host: two readbacks, two uploads and a wait fewer per block.
+__global__ __launch_bounds__(256) void k_keep_cols(const double* __restrict__ n2_0, const double* __restrict__ n2, int a,
+                                                   int* __restrict__ idx, double* __restrict__ scl, int* __restrict__ kept) {
+    __shared__ int cnt[4];
+    const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    int k = 0;
+    for (int b = 0; b < a; b += 256) {
+        const int j = b + tid;
+        const double before = j < a ? sqrt(n2_0[j]) : 0.0, norm = j < a ? sqrt(n2[j]) : 0.0;
+        const bool keep = before > 0.0 && norm > 1e-8 * before;
+        const unsigned long long mask = __ballot(keep);
+        if (lane == 0) cnt[wave] = __popcll(mask);
+        __syncthreads();
+        int at = k + __popcll(mask & ((1ull << lane) - 1));
+        for (int q = 0; q < 4; ++q) {
+            if (q < wave) at += cnt[q];
+            k += cnt[q];
+        }
+        if (keep) {
+            idx[at] = j;
+            scl[at] = 1.0 / norm;
+        }
+        __syncthreads();
+    }
+    if (tid == 0) *kept = k;
+}
+
+// Q[:, j] *= scale[j]
+__global__ void k_scale_cols(double2* __restrict__ q, const double* __restrict__ scale, size_t ld, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double2* p = q + (size_t)blockIdx.y * ld + i;
+    const double f = scale[blockIdx.y];
+    *p = make_double2(p->x * f, p->y * f);
+}
+
 // T[m0 + i, j] = conj(T[j, m0 + i]) for j < m0 (mirror of the new columns), and the new
 // a x a diagonal block made Hermitian with a real diagonal (common.zig:247-258).
 __global__ void k_mirror_new(double2* __restrict__ t, int ld, int m0, int a) {
@@ -399,7 +437,7 @@ struct EigWork {
     hipStream_t stream = nullptr;
     size_t n = 0;
     int max_sub = 0, nb = 0;
-    DevBuf V, W, X, HX, R, Q, HQ, T, Tw, S, G, evals, ework, info, norms, lam, ekin, diag, sel, scl, idx;
+    DevBuf V, W, X, HX, R, Q, HQ, T, Tw, S, G, evals, ework, info, norms, norms0, ekin, diag, sel, scl, idx;
     DevBuf x32, y32;
     uint64_t x_cols = 0;  // columns of X holding the last solve's Ritz vectors (0: none)
     bool x_converged = false;
@@ -412,12 +450,34 @@ struct EigWork {
     std::vector<int> ev_tag;
     size_t ev_used = 0;
     HeevWork heev;  // dense Hermitian eigensolver workspace (subspace problems)
+    // What the host reads back in every iteration, in pinned memory that the kernels write (valid once
+    // the stream is synchronised): column norms, Ritz values, and verdicts (the Cholesky
+    // factorisation's two, the columns kept).  A copy after the kernel takes 3 us and a launch.
+    double *host_norms = nullptr, *host_evals = nullptr;
+    int* host_info = nullptr;
+    size_t host_cap = 0;
+    void ensure_host(size_t cols) {
+        if (cols <= host_cap) return;
+        release_host();
+        void* p = nullptr;
+        DZ_HIP(hipHostMalloc(&p, 2 * cols * sizeof(double) + 64, hipHostMallocDefault));
+        host_norms = static_cast<double*>(p);
+        host_evals = host_norms + cols;
+        host_info = reinterpret_cast<int*>(host_evals + cols);
+        host_cap = cols;
+    }
+    void release_host() {
+        if (host_norms) (void)hipHostFree(host_norms);
+        host_norms = nullptr;
+        host_cap = 0;
+    }
     ~EigWork() {
+        release_host();
         heev.release();
         for (hipEvent_t e : ev_pool) (void)hipEventDestroy(e);
         if (blas) rocblas_destroy_handle(blas);
         DevBuf* bufs[] = {&V, &W, &X, &HX, &R, &Q, &HQ, &T, &Tw, &S, &G, &evals, &ework, &info,
-                          &norms, &lam, &ekin, &diag, &sel, &scl, &idx, &x32, &y32, &rnorm,
+                          &norms, &norms0, &ekin, &diag, &sel, &scl, &idx, &x32, &y32, &rnorm,
                           &snapX, &snapR, &snapLam, &snapRn, &snapEk, &bandsum, &samples, &gram_part};
         for (DevBuf* b : bufs) b->release();
     }
@@ -603,39 +663,39 @@ __global__ __launch_bounds__(512) void k_potrf_upper(const double2* S, double2* 
     }
 }
 
-// ok = 1 when the Cholesky factorisation of the Gram matrix succeeded (info == 0) and every pivot
-// keeps at least 1e-7 of its column's norm (R_jj > 1e-7 sqrt(G_jj); G's diagonal from its copy
-// gcopy, R in r, both k x k with leading dimension k).  One workgroup.
+// The verdicts of k_potrf_upper (out[0:2]) on another factorisation: its info, and ok = 1 when info is 0
+// and every pivot keeps at least 1e-7 of its column's norm (the diagonal of G from its copy gcopy, R in
+// r, both k x k with leading dimension k).  One workgroup.
 __global__ __launch_bounds__(256) void k_chol_check(const double2* __restrict__ gcopy, const double2* __restrict__ r,
-                                                    int k, const rocblas_int* __restrict__ info, int* __restrict__ ok) {
+                                                    int k, const rocblas_int* __restrict__ info, int* __restrict__ out) {
     int bad = 0;
     for (int j = (int)threadIdx.x; j < k; j += 256) {
         const double g = gcopy[(size_t)j * (k + 1)].x, rj = r[(size_t)j * (k + 1)].x;
         if (!(rj > 1e-7 * sqrt(fmax(g, 0.0)))) bad = 1;
     }
     bad = __syncthreads_or(bad);
-    if (threadIdx.x == 0) *ok = (*info == 0 && !bad) ? 1 : 0;
+    if (threadIdx.x == 0) {
+        out[0] = *info;
+        out[1] = (*info == 0 && !bad) ? 1 : 0;
+    }
 }
 
-static std::vector<double> subspace_eigh(EigWork& w, const double2* A, int lda, int m, int nev, double2* Y, int ldy,
-                                         hipStream_t s) {
-    std::vector<double> ev(nev);
+// Lowest nev eigenpairs of A; the eigenvalues in w.evals and, once s is synchronised, w.host_evals.
+static void subspace_eigh(EigWork& w, const double2* A, int lda, int m, int nev, double2* Y, int ldy, hipStream_t s) {
     if (m <= kHeevMaxM) {
         heev_lowest_shared(w.heev, A, lda, m, nev, w.evals.as<double>(), Y, ldy, s);
-        DZ_HIP(hipMemcpyAsync(ev.data(), w.evals.ptr, nev * sizeof(double), hipMemcpyDeviceToHost, s));
-        DZ_HIP(hipStreamSynchronize(s));
-        return ev;
+        DZ_HIP(hipMemcpyAsync(w.host_evals, w.evals.ptr, nev * sizeof(double), hipMemcpyDeviceToHost, s));
+        return;
     }
     DZ_HIP(hipMemcpy2DAsync(Y, (size_t)ldy * sizeof(double2), A, (size_t)lda * sizeof(double2),
                             (size_t)m * sizeof(double2), m, hipMemcpyDeviceToDevice, s));
     DZ_BLAS(rocsolver_zheevd(w.blas, rocblas_evect_original, rocblas_fill_lower, m, reinterpret_cast<zc*>(Y), ldy,
                              w.evals.as<double>(), w.ework.as<double>(), w.info.as<rocblas_int>()));
     rocblas_int info = 0;
-    DZ_HIP(hipMemcpyAsync(ev.data(), w.evals.ptr, nev * sizeof(double), hipMemcpyDeviceToHost, s));
+    DZ_HIP(hipMemcpyAsync(w.host_evals, w.evals.ptr, nev * sizeof(double), hipMemcpyDeviceToHost, s));
     DZ_HIP(hipMemcpyAsync(&info, w.info.ptr, sizeof(info), hipMemcpyDeviceToHost, s));
     DZ_HIP(hipStreamSynchronize(s));
     DZ_REQUIRE(info == 0, DZHIP_ERR_HIP, "zheevd did not converge");
-    return ev;
 }
 
 static void eig_work_release(Ham& h) {
@@ -720,15 +780,11 @@ struct Solver {
                               reinterpret_cast<const zc*>(B), ldb, &beta, reinterpret_cast<zc*>(C), ldc));
     }
 
-    std::vector<double> col_norms(const double2* v, int cols) {
-        std::vector<double> out(cols);
-        if (cols == 0) return out;
-        hipLaunchKernelGGL(k_col_norm2, dim3(cols), dim3(256), 0, s, v, n, (int)n, w.norms.as<double>());
+    // Squared column norms into out (device or pinned memory).
+    void col_norms2(const double2* v, int cols, double* out) {
+        if (cols == 0) return;
+        hipLaunchKernelGGL(k_col_norm2, dim3(cols), dim3(256), 0, s, v, n, (int)n, out);
         DZ_HIP(hipGetLastError());
-        DZ_HIP(hipMemcpyAsync(out.data(), w.norms.ptr, cols * sizeof(double), hipMemcpyDeviceToHost, s));
-        DZ_HIP(hipStreamSynchronize(s));
-        for (double& v2 : out) v2 = std::sqrt(v2);
-        return out;
     }
 
     // Orthogonalise Q[:, 0:a] against V[:, 0:m] (two block CGS passes) and orthonormalise it
@@ -738,51 +794,53 @@ struct Solver {
     // columns kept (compacted to the front).
     int orthonormalize_new(double2* Q, int a, int m) {
         const int ldn = (int)n;
-        const std::vector<double> nrm0 = col_norms(Q, a);
+        if (a <= 0) return 0;
+        col_norms2(Q, a, w.norms0.as<double>());
         for (int pass = 0; pass < 2 && m > 0; ++pass) {
             // S = V^H Q ; Q -= V S
             gram(V(), m, Q, a, w.S.as<double2>(), max_sub);
             gemm(rocblas_operation_none, rocblas_operation_none, ldn, a, m, zc(-1.0, 0.0), V(), ldn,
                  w.S.as<double2>(), max_sub, zc(1.0, 0.0), Q, ldn);
         }
-        std::vector<double> nrm = col_norms(Q, a);
-        std::vector<int> keep;
-        std::vector<double> inv;
-        for (int j = 0; j < a; ++j)
-            if (nrm0[j] > 0.0 && nrm[j] > 1e-8 * nrm0[j]) {
-                keep.push_back(j);
-                inv.push_back(1.0 / nrm[j]);
-            }
-        const int k = (int)keep.size();
-        if (k == 0) return 0;
-        // Compact and normalise into HQ (scratch), then copy back to Q.
-        DZ_HIP(hipMemcpyAsync(w.idx.ptr, keep.data(), k * sizeof(int), hipMemcpyHostToDevice, s));
-        DZ_HIP(hipMemcpyAsync(w.scl.ptr, inv.data(), k * sizeof(double), hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(k_gather_cols, cols_grid(k), dim3(256), 0, s, Q, w.idx.as<int>(), w.scl.as<double>(),
-                           w.HQ.as<double2>(), n, (int)n);
+        col_norms2(Q, a, w.norms.as<double>());
+        hipLaunchKernelGGL(k_keep_cols, dim3(1), dim3(256), 0, s, w.norms0.as<double>(), w.norms.as<double>(), a,
+                           w.idx.as<int>(), w.scl.as<double>(), w.host_info + 2);
         DZ_HIP(hipGetLastError());
-        DZ_HIP(hipMemcpyAsync(Q, w.HQ.ptr, n * k * sizeof(double2), hipMemcpyDeviceToDevice, s));
+        DZ_HIP(hipStreamSynchronize(s));
+        const int k = w.host_info[2];
+        if (k == 0) return 0;
+        // Normalise, compacted through HQ (scratch) where a column was dropped.
+        if (k == a) {
+            hipLaunchKernelGGL(k_scale_cols, cols_grid(k), dim3(256), 0, s, Q, w.scl.as<double>(), n, (int)n);
+            DZ_HIP(hipGetLastError());
+        } else {
+            hipLaunchKernelGGL(k_gather_cols, cols_grid(k), dim3(256), 0, s, Q, w.idx.as<int>(), w.scl.as<double>(),
+                               w.HQ.as<double2>(), n, (int)n);
+            DZ_HIP(hipGetLastError());
+            DZ_HIP(hipMemcpyAsync(Q, w.HQ.ptr, n * k * sizeof(double2), hipMemcpyDeviceToDevice, s));
+        }
         int kk = k;
         for (int pass = 0; pass < 2 && kk > 0; ++pass) kk = ortho_block(Q, kk);
         return kk;
     }
 
     // S = R^H R for the k x k Gram matrix in S (left as it is, leading dimension k), R -> G; the verdicts
-    // in w.info[0:2] as k_potrf_upper leaves them: the library's one-workgroup factorisation up to
+    // in w.host_info[0:2] as k_potrf_upper leaves them: the library's one-workgroup factorisation up to
     // kPotrfMax, rocSOLVER's zpotrf beyond.
     void potrf_upper(int k) {
         static_assert(sizeof(rocblas_int) == sizeof(int), "info is read as int");
         double2 *S = w.S.as<double2>(), *G = w.G.as<double2>();
-        int* info = w.info.as<int>();
         if (k <= kPotrfMax) {
             const size_t lds = potrf_lds_bytes(k);
             set_max_dynamic_lds((const void*)k_potrf_upper, lds);
             // More than 96 columns: enough tiles for eight wavefronts.
-            hipLaunchKernelGGL(k_potrf_upper, dim3(1), dim3(k > 96 ? 512 : 256), lds, s, S, G, k, k, info);
+            hipLaunchKernelGGL(k_potrf_upper, dim3(1), dim3(k > 96 ? 512 : 256), lds, s, S, G, k, k,
+                               w.host_info);
         } else {
             DZ_HIP(hipMemcpyAsync(G, S, (size_t)k * k * sizeof(double2), hipMemcpyDeviceToDevice, s));
-            DZ_BLAS(rocsolver_zpotrf(w.blas, rocblas_fill_upper, k, reinterpret_cast<zc*>(G), k, info));
-            hipLaunchKernelGGL(k_chol_check, dim3(1), dim3(256), 0, s, S, G, k, info, info + 1);
+            DZ_BLAS(rocsolver_zpotrf(w.blas, rocblas_fill_upper, k, reinterpret_cast<zc*>(G), k,
+                                     w.info.as<rocblas_int>()));
+            hipLaunchKernelGGL(k_chol_check, dim3(1), dim3(256), 0, s, S, G, k, w.info.as<rocblas_int>(), w.host_info);
         }
         DZ_HIP(hipGetLastError());
     }
@@ -797,19 +855,18 @@ struct Solver {
         const int ldn = (int)n;
         gram(Q, k, Q, k, w.S.as<double2>(), k);
         potrf_upper(k);
-        // Decided on the device; one int back to the host.
-        int ok = 0;
-        DZ_HIP(hipMemcpyAsync(&ok, w.info.as<int>() + 1, sizeof(int), hipMemcpyDeviceToHost, s));
         DZ_HIP(hipStreamSynchronize(s));
         const zc one(1.0, 0.0), zero(0.0, 0.0);
-        if (ok) {
+        if (w.host_info[1]) {
             DZ_BLAS(rocblas_ztrsm(w.blas, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
                                   rocblas_diagonal_non_unit, ldn, k, &one, w.G.as<zc>(), k, reinterpret_cast<zc*>(Q), ldn));
             return k;
         }
         st.ortho_fallbacks++;
         // Eigen-decomposition of the Gram matrix (S, lower triangle) into G.
-        const std::vector<double> lam = subspace_eigh(w, w.S.as<double2>(), k, k, k, w.G.as<double2>(), k, s);
+        subspace_eigh(w, w.S.as<double2>(), k, k, k, w.G.as<double2>(), k, s);
+        DZ_HIP(hipStreamSynchronize(s));
+        const double* lam = w.host_evals;
         const double thr = 1e-12 * std::max(lam[k - 1], 0.0);
         int first = 0;
         while (first < k && !(lam[first] > thr)) ++first;
@@ -837,10 +894,8 @@ struct Solver {
         const int ldn = (int)n;
         gram(Q, k, Q, k, w.S.as<double2>(), k);
         potrf_upper(k);
-        rocblas_int info = 0;
-        DZ_HIP(hipMemcpyAsync(&info, w.info.ptr, sizeof(info), hipMemcpyDeviceToHost, s));
         DZ_HIP(hipStreamSynchronize(s));
-        DZ_REQUIRE(info == 0, DZHIP_ERR_HIP, "Cholesky QR: Gram matrix not positive definite");
+        DZ_REQUIRE(w.host_info[0] == 0, DZHIP_ERR_HIP, "Cholesky QR: Gram matrix not positive definite");
         const zc one(1.0, 0.0);
         DZ_BLAS(rocblas_ztrsm(w.blas, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
                               rocblas_diagonal_non_unit, ldn, k, &one, w.G.as<zc>(), k, reinterpret_cast<zc*>(Q), ldn));
@@ -927,10 +982,10 @@ struct Solver {
         extend_T(0, m);
     }
 
-    // Lowest nb eigenpairs of T[0:m, 0:m] (m >= nb); eigenvectors land in Tw, eigenvalues (host)
-    // returned.
-    std::vector<double> rayleigh_ritz(int m) {
-        return subspace_eigh(w, T(), max_sub, m, std::min(m, nb), w.Tw.as<double2>(), max_sub, s);
+    // Lowest nb eigenpairs of T[0:m, 0:m] (m >= nb); eigenvectors land in Tw, eigenvalues in w.evals and
+    // w.host_evals.
+    void rayleigh_ritz(int m) {
+        subspace_eigh(w, T(), max_sub, m, std::min(m, nb), w.Tw.as<double2>(), max_sub, s);
     }
 
     void ritz(int m) {
@@ -970,6 +1025,7 @@ static void ensure_work(Ham& h, int max_sub, int nb) {
     if (w->X.bytes < n * nb * c) w->x_cols = 0;  // X is reallocated below
     w->V.ensure(n * max_sub * c);
     w->W.ensure(n * max_sub * c);
+    w->ensure_host((size_t)max_sub);
     w->X.ensure(n * nb * c);
     w->HX.ensure(n * nb * c);
     w->R.ensure(n * nb * c);
@@ -983,7 +1039,7 @@ static void ensure_work(Ham& h, int max_sub, int nb) {
     w->ework.ensure(max_sub * sizeof(double));
     w->info.ensure(64);
     w->norms.ensure(max_sub * sizeof(double));
-    w->lam.ensure(max_sub * sizeof(double));
+    w->norms0.ensure(max_sub * sizeof(double));
     w->ekin.ensure(max_sub * sizeof(double));
     w->diag.ensure(n * sizeof(double));
     w->sel.ensure(max_sub * sizeof(int));
@@ -1052,23 +1108,24 @@ void eig_solve(Ham& h, const double* diag, uint64_t nbands, const dzhip_eig_opts
     const bool mlp_ran = precond == DZHIP_PRECOND_MLP;
     std::vector<double> res_hist;
     const int nconv = (o.nconv == 0 || o.nconv > (uint64_t)nb) ? nb : (int)o.nconv;
-    std::vector<double> lam(nb), best(nb);
+    std::vector<double> lam(nb), best(nb), rn(nb);
     bool have_best = false;
     uint64_t iter = 0;
     w.ev_used = 0;
     for (; iter < o.max_iter; ++iter) {
         mark(w, s, SEC_RR);
-        std::vector<double> ev = S.rayleigh_ritz(m);
-        for (int b = 0; b < nb; ++b) lam[b] = ev[b];
-        best = lam;
-        have_best = true;
+        S.rayleigh_ritz(m);
         mark(w, s, SEC_RITZ);
         S.ritz(m);
-        DZ_HIP(hipMemcpyAsync(w.lam.ptr, lam.data(), nb * sizeof(double), hipMemcpyHostToDevice, s));
         hipLaunchKernelGGL(k_residual, S.cols_grid(nb), dim3(256), 0, s, w.HX.as<double2>(), w.X.as<double2>(),
-                           w.lam.as<double>(), w.R.as<double2>(), n, (int)n);
+                           w.evals.as<double>(), w.R.as<double2>(), n, (int)n);
         DZ_HIP(hipGetLastError());
-        std::vector<double> rn = S.col_norms(w.R.as<double2>(), nb);
+        S.col_norms2(w.R.as<double2>(), nb, w.host_norms);
+        DZ_HIP(hipStreamSynchronize(s));
+        lam.assign(w.host_evals, w.host_evals + nb);
+        best = lam;
+        have_best = true;
+        for (int b = 0; b < nb; ++b) rn[b] = std::sqrt(w.host_norms[b]);
         // Convergence is judged on the first nconv bands (all by default); the others are a buffer.
         const double max_res = *std::max_element(rn.begin(), rn.begin() + nconv);
         S.st.max_residual = max_res;
@@ -1127,6 +1184,10 @@ void eig_solve(Ham& h, const double* diag, uint64_t nbands, const dzhip_eig_opts
         for (int b = 0; b < nb && (int)sel.size() < room; ++b)
             if (rn[b] >= o.tol) sel.push_back(b);
         int a = 0;
+        // The new block is built at its place in the basis, its H image in W, where they fit; before a
+        // restart in Q and HQ.
+        const bool in_place = m + (int)sel.size() <= max_sub;
+        double2 *qn = in_place ? S.V() + (size_t)m * n : w.Q.as<double2>(), *hqn = in_place ? S.W() + (size_t)m * n : w.HQ.as<double2>();
         if (!sel.empty()) {
             mark(w, s, SEC_PRECOND);
             DZ_HIP(hipMemcpyAsync(w.sel.ptr, sel.data(), sel.size() * sizeof(int), hipMemcpyHostToDevice, s));
@@ -1137,17 +1198,17 @@ void eig_solve(Ham& h, const double* diag, uint64_t nbands, const dzhip_eig_opts
             }
             if (precond == DZHIP_PRECOND_MLP) {
                 DZ_HIP(hipMemcpyAsync(w.rnorm.ptr, rn.data(), nb * sizeof(double), hipMemcpyHostToDevice, s));
-                precondition_mlp(w.R.as<double2>(), w.sel.as<int>(), (int)sel.size(), w.lam.as<double>(),
+                precondition_mlp(w.R.as<double2>(), w.sel.as<int>(), (int)sel.size(), w.evals.as<double>(),
                                  w.ekin.as<double>(), w.rnorm.as<double>(), w.diag.as<double>(), h.mlp_params.as<float>(),
-                                 h.mlp_energy_scale, h.mlp_base, w.Q.as<double2>(), n, (int)n, s);
+                                 h.mlp_energy_scale, h.mlp_base, qn, n, (int)n, s);
             } else {
                 hipLaunchKernelGGL(k_precondition, S.cols_grid((int)sel.size()), dim3(256), 0, s, w.R.as<double2>(),
-                                   w.sel.as<int>(), w.lam.as<double>(), w.ekin.as<double>(), w.diag.as<double>(),
-                                   w.Q.as<double2>(), n, (int)n, precond == DZHIP_PRECOND_TPA ? 1 : 0);
+                                   w.sel.as<int>(), w.evals.as<double>(), w.ekin.as<double>(), w.diag.as<double>(),
+                                   qn, n, (int)n, precond == DZHIP_PRECOND_TPA ? 1 : 0);
                 DZ_HIP(hipGetLastError());
             }
             mark(w, s, SEC_ORTHO);
-            a = S.orthonormalize_new(w.Q.as<double2>(), (int)sel.size(), m);
+            a = S.orthonormalize_new(qn, (int)sel.size(), m);
         }
         if (a == 0) {
             // Nothing could be added: every residual is individually below tol
@@ -1160,7 +1221,7 @@ void eig_solve(Ham& h, const double* diag, uint64_t nbands, const dzhip_eig_opts
             break;
         }
         mark(w, s, SEC_APPLY);
-        S.apply(w.Q.as<double2>(), w.HQ.as<double2>(), a);
+        S.apply(qn, hqn, a);
         mark(w, s, SEC_EXTEND);
         if (m + a > max_sub) {
             // Thick restart from [Ritz vectors, new block]; their H images are W c and H Q.
@@ -1169,8 +1230,10 @@ void eig_solve(Ham& h, const double* diag, uint64_t nbands, const dzhip_eig_opts
             S.st.restarts++;
             continue;
         }
-        DZ_HIP(hipMemcpyAsync(S.V() + (size_t)m * n, w.Q.ptr, n * a * sizeof(double2), hipMemcpyDeviceToDevice, s));
-        DZ_HIP(hipMemcpyAsync(S.W() + (size_t)m * n, w.HQ.ptr, n * a * sizeof(double2), hipMemcpyDeviceToDevice, s));
+        if (!in_place) {
+            DZ_HIP(hipMemcpyAsync(S.V() + (size_t)m * n, w.Q.ptr, n * a * sizeof(double2), hipMemcpyDeviceToDevice, s));
+            DZ_HIP(hipMemcpyAsync(S.W() + (size_t)m * n, w.HQ.ptr, n * a * sizeof(double2), hipMemcpyDeviceToDevice, s));
+        }
         S.extend_T(m, a);
         m += a;
     }
@@ -1454,7 +1517,9 @@ void cg_solve(Ham& h, const double* diag, uint64_t nbands, const dzhip_eig_opts&
                           reinterpret_cast<const zc*>(V), (int)n, reinterpret_cast<const zc*>(HV), (int)n, &zero,
                           w.Tw.as<zc>(), nb));
     // Eigenvectors of T (in Tw) into S (nb x nb).
-    const std::vector<double> ev = subspace_eigh(w, w.Tw.as<double2>(), nb, nb, nb, w.S.as<double2>(), nb, s);
+    subspace_eigh(w, w.Tw.as<double2>(), nb, nb, nb, w.S.as<double2>(), nb, s);
+    DZ_HIP(hipStreamSynchronize(s));
+    const std::vector<double> ev(w.host_evals, w.host_evals + nb);
     DZ_BLAS(rocblas_zgemm(w.blas, rocblas_operation_none, rocblas_operation_none, (int)n, nb, nb, &one,
                           reinterpret_cast<const zc*>(V), (int)n, w.S.as<zc>(), nb, &zero, w.X.as<zc>(), (int)n));
     std::copy(ev.begin(), ev.end(), values);

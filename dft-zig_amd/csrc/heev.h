@@ -26,6 +26,7 @@ constexpr int kHeevMaxM = 1024;
 
 struct HeevWork {
     DevBuf vh, tau, d, e, pub, err, z, zt, gram;
+    int* flag = nullptr;  // pinned: the error flag's readback
     void release();
 };
 

@@ -1320,6 +1320,8 @@ void heev_lowest_noalloc(int device, const double2* A, int lda, int m, int nev, 
 void HeevWork::release() {
     DevBuf* bufs[] = {&vh, &tau, &d, &e, &pub, &err, &z, &zt, &gram};
     for (DevBuf* b : bufs) b->release();
+    if (flag) (void)hipHostFree(flag);
+    flag = nullptr;
 }
 
 void heev_tridiag_only(HeevWork& w, const double2* A, int lda, int m, hipStream_t s) {
@@ -1378,11 +1380,11 @@ void heev_lowest_shared(HeevWork& w, const double2* A, int lda, int m, int nev, 
 unsigned long long heev_shared_retries() { return g_trd_retries.load(std::memory_order_relaxed); }
 
 int heev_error_flag(HeevWork& w, hipStream_t s) {
-    int flag = 0;
     if (!w.err.ptr) return 0;
-    DZ_HIP(hipMemcpyAsync(&flag, w.err.ptr, sizeof(int), hipMemcpyDeviceToHost, s));
+    if (!w.flag) DZ_HIP(hipHostMalloc(reinterpret_cast<void**>(&w.flag), sizeof(int), hipHostMallocDefault));
+    DZ_HIP(hipMemcpyAsync(w.flag, w.err.ptr, sizeof(int), hipMemcpyDeviceToHost, s));
     DZ_HIP(hipStreamSynchronize(s));
-    return flag;
+    return *w.flag;
 }
 
 }  // namespace dzhip
