@@ -663,6 +663,106 @@ __global__ __launch_bounds__(512) void k_potrf_upper(const double2* S, double2* 
     }
 }
 
+// Q <- Q R^{-1} in place, Q n x k and R upper triangular (its upper triangle is read; column-major,
+// leading dimensions ldq, ldr).  A wavefront takes 16 rows through the 16-column blocks from left to
+// right: the products with the finished blocks on the matrix cores, then substitution with the diagonal
+// block (in LDS).  MFMA rows are columns of Q and MFMA columns its rows, so that the result's register
+// layout (row l % 16, columns l / 16 + 4 r) is the next products' operand layout and a finished block is
+// read back by the lane that wrote it: no exchange but the substitution's row broadcasts.  One
+// wavefront a workgroup while there are fewer of them than SIMDs, four (sharing R in L1) beyond.
+// The chain bounds it: n = 1,637, k = 24: 7.8 us (rocBLAS' trsm 13.9); n = 20,000, k = 164: 102 us (147
+// in several launches; 55 at the matrix cores' rate).
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_trsm_right(double2* Q, size_t ldq, int n, int k, const double2* __restrict__ R,
+                                                        int ldr) {
+    __shared__ double2 diag[2][16][16];  // the diagonal block above its diagonal, zeros elsewhere [row][column]
+    __shared__ double inv[2][16];
+    const int tid = (int)threadIdx.x, lane = tid & 63, l16 = lane & 15, l4 = lane >> 4;
+    const int row = ((int)blockIdx.x * NW + (tid >> 6)) * 16 + l16;
+    double2* qrow = Q + min(row, n - 1);
+    constexpr int ND = 4 / NW;  // elements of the diagonal block per thread
+    double2 dn[ND], qn[4];      // the next block's, loaded before this one's substitution
+    auto fetch_block = [&](int c0) {
+        c0 = min(c0, (k - 1) / 16 * 16);
+#pragma unroll
+        for (int q = 0; q < ND; ++q) {
+            const int e = tid + q * 64 * NW;
+            dn[q] = R[(size_t)min(c0 + (e >> 4), k - 1) * ldr + min(c0 + (e & 15), k - 1)];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) qn[r] = qrow[(size_t)min(c0 + l4 + 4 * r, k - 1) * ldq];
+    };
+    fetch_block(0);
+    int buf = 0;
+    for (int c0 = 0; c0 < k; c0 += 16, buf ^= 1) {
+        const int nb = min(16, k - c0);
+#pragma unroll
+        for (int q = 0; q < ND; ++q) {
+            const int e = tid + q * 64 * NW, i = e & 15, c = e >> 4;
+            if (i == c) inv[buf][c] = c < nb ? 1.0 / dn[q].x : 1.0;
+            diag[buf][i][c] = i < c && c < nb ? dn[q] : double2{0.0, 0.0};
+        }
+        v4d_t re, im;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            re[r] = qn[r].x;
+            im[r] = qn[r].y;
+        }
+        // Q[:, block] -= Y[:, p] R[p, block]
+        const double2* rc = R + (size_t)min(c0 + l16, k - 1) * ldr + l4;
+        double2 a[4], y[4];
+        auto fetch = [&](int p, double2 (&av)[4], double2 (&yv)[4]) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                av[t] = rc[p + 4 * t];
+                yv[t] = qrow[(size_t)(p + l4 + 4 * t) * ldq];
+            }
+        };
+        if (c0 > 0) fetch(0, a, y);
+        for (int p = 0; p < c0; p += 16) {
+            double2 an[4], yn[4];
+            fetch(min(p + 16, c0 - 16), an, yn);
+            __builtin_amdgcn_sched_barrier(0);  // the loads go out first
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[t].x, y[t].x, re, 0, 0, 0);
+                im = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[t].x, y[t].y, im, 0, 0, 0);
+                re = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t].y, y[t].y, re, 0, 0, 0);
+                im = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[t].y, y[t].x, im, 0, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                a[t] = an[t];
+                y[t] = yn[t];
+            }
+        }
+        __syncthreads();  // diag; the other buffer was read before the previous one
+        fetch_block(c0 + 16);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int src = 16 * (j & 3) + l16;
+            const double f = inv[buf][j];
+            const double yx = __shfl(re[j >> 2], src) * f, yy = __shfl(im[j >> 2], src) * f;
+            if (l4 == (j & 3)) {
+                re[j >> 2] = yx;
+                im[j >> 2] = yy;
+            }
+#pragma unroll
+            for (int r = j >> 2; r < 4; ++r) {
+                const double2 d = diag[buf][j][l4 + 4 * r];
+                re[r] -= yx * d.x - yy * d.y;
+                im[r] -= yx * d.y + yy * d.x;
+            }
+        }
+        if (row < n) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (l4 + 4 * r < nb) qrow[(size_t)(c0 + l4 + 4 * r) * ldq] = double2{re[r], im[r]};
+        }
+    }
+}
+
 // The verdicts of k_potrf_upper (out[0:2]) on another factorisation: its info, and ok = 1 when info is 0
 // and every pivot keeps at least 1e-7 of its column's norm (the diagonal of G from its copy gcopy, R in
 // r, both k x k with leading dimension k).  One workgroup.
@@ -845,6 +945,16 @@ struct Solver {
         DZ_HIP(hipGetLastError());
     }
 
+    // Q[:, 0:k] <- Q R^{-1}, R the upper triangle of G (leading dimension k).
+    void trsm(double2* Q, int k) {
+        const unsigned tiles = (unsigned)((n + 15) / 16);
+        if (tiles < 1024)
+            hipLaunchKernelGGL(k_trsm_right<1>, dim3(tiles), dim3(64), 0, s, Q, n, (int)n, k, w.G.as<double2>(), k);
+        else
+            hipLaunchKernelGGL(k_trsm_right<4>, dim3((tiles + 3) / 4), dim3(256), 0, s, Q, n, (int)n, k, w.G.as<double2>(), k);
+        DZ_HIP(hipGetLastError());
+    }
+
     // Orthonormalise Q[:, 0:k] in place: Cholesky QR, or, when the Gram matrix is not
     // numerically positive definite, its eigen-decomposition G = U L U^H with the directions of
     // L < 1e-12 max(L) dropped and Q <- Q U L^{-1/2} (compacted to the front).  Returns the
@@ -858,8 +968,7 @@ struct Solver {
         DZ_HIP(hipStreamSynchronize(s));
         const zc one(1.0, 0.0), zero(0.0, 0.0);
         if (w.host_info[1]) {
-            DZ_BLAS(rocblas_ztrsm(w.blas, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
-                                  rocblas_diagonal_non_unit, ldn, k, &one, w.G.as<zc>(), k, reinterpret_cast<zc*>(Q), ldn));
+            trsm(Q, k);
             return k;
         }
         st.ortho_fallbacks++;
@@ -891,14 +1000,11 @@ struct Solver {
 
     // Q <- Q R^{-1} with G = Q^H Q = R^H R.  Throws if G is not positive definite.
     void cholqr(double2* Q, int k) {
-        const int ldn = (int)n;
         gram(Q, k, Q, k, w.S.as<double2>(), k);
         potrf_upper(k);
         DZ_HIP(hipStreamSynchronize(s));
         DZ_REQUIRE(w.host_info[0] == 0, DZHIP_ERR_HIP, "Cholesky QR: Gram matrix not positive definite");
-        const zc one(1.0, 0.0);
-        DZ_BLAS(rocblas_ztrsm(w.blas, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
-                              rocblas_diagonal_non_unit, ldn, k, &one, w.G.as<zc>(), k, reinterpret_cast<zc*>(Q), ldn));
+        trsm(Q, k);
     }
 
     // T[0:m+a, m:m+a] = V[:, 0:m+a]^H W[:, m:m+a], mirrored into the rows.

@@ -174,3 +174,22 @@ def test_eig_cholesky_blocks(dz, ctx, k):
     print(f"k={k} n={w.npw} it={st['iterations']} dv={np.max(np.abs(vals - ref)):.2e} orth={err:.1e}", flush=True)
     assert st["converged"] == 1 and st["ortho_fallbacks"] == 0
     assert np.max(np.abs(vals - ref)) < 2e-8 and err < 1e-12
+
+
+@pytest.mark.parametrize("nbands", [5, 29])
+def test_eig_large_basis(dz, ctx, nbands):
+    """A basis of more than 16,368 plane waves (four wavefronts a workgroup in the triangular solve):
+    orthonormal vectors (1e-12) with residuals below the solve's tolerance (twice it: recomputed)."""
+    from dzhip import workloads
+
+    w = workloads.bench(nbands=4)
+    assert w.npw > 16368
+    ham = dz.Hamiltonian.from_workload(ctx, w)
+    vals, vecs, st = ham.eig_solve(nbands, tol=1e-3, max_iter=200)
+    v = vecs.reshape(nbands, -1)
+    hv = ham.apply(v).reshape(nbands, -1)
+    ham.close()
+    err = np.max(np.abs(v.conj() @ v.T - np.eye(nbands)))
+    res = np.max(np.linalg.norm(hv - vals[:, None] * v, axis=1))
+    print(f"nbands={nbands} n={w.npw} it={st['iterations']} orth={err:.1e} res={res:.1e}", flush=True)
+    assert st["converged"] == 1 and err < 1e-12 and res < 2e-3
