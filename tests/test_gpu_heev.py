@@ -59,6 +59,15 @@ def test_heev_reflector_blocks(ctx, m):
     check(ctx, 0.5 * (g + g.conj().T), min(m, 20))
 
 
+@pytest.mark.parametrize("m,nev", [(5, 3), (15, 15), (16, 16), (17, 17), (65, 33), (79, 64), (80, 65), (200, 161)])
+def test_heev_orthonormalisation_tiles(ctx, m, nev):
+    """Sizes at the edges of the Newton-Schulz products' 16 x 16 tiles and of the chunks that their four
+    wavefronts share; bars as above."""
+    rng = np.random.default_rng(4000 + m)
+    g = rng.standard_normal((m, m)) + 1j * rng.standard_normal((m, m))
+    check(ctx, 0.5 * (g + g.conj().T), nev)
+
+
 def test_heev_degenerate_and_clustered(ctx):
     """Exactly degenerate triplets and pairs (symmetry-degenerate bands), a cluster split by
     1e-13, and a zero off-diagonal block (a reducible tridiagonal)."""
