@@ -242,10 +242,11 @@ struct HamSet {
         size_t nc;
         int prec, code, pkind;
         hipStream_t s;
-        void *tbuf, *partial, *qbuf;
+        void *tbuf, *partial, *qbuf, *chunks, *kseg, *tiles;  // every buffer that may be reallocated
         bool operator==(const GraphKey& o) const {
             return x == o.x && y == o.y && nc == o.nc && prec == o.prec && code == o.code && pkind == o.pkind &&
-                   s == o.s && tbuf == o.tbuf && partial == o.partial && qbuf == o.qbuf;
+                   s == o.s && tbuf == o.tbuf && partial == o.partial && qbuf == o.qbuf && chunks == o.chunks &&
+                   kseg == o.kseg && tiles == o.tiles;
         }
     };
     hipGraphExec_t graph_exec = nullptr;

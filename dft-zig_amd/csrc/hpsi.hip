@@ -2901,7 +2901,8 @@ void hamset_apply_dev(HamSet& hs, const void* x, void* y, size_t nc, bool use_gr
         hamset_launch<T>(hs, x, y, nc, code, pkind, s);
         return;
     }
-    const HamSet::GraphKey key{x, y, nc, (int)sizeof(T), code, pkind, s, hs.tbuf.ptr, hs.partial.ptr, hs.qbuf.ptr};
+    const HamSet::GraphKey key{x, y, nc, (int)sizeof(T), code, pkind, s, hs.tbuf.ptr, hs.partial.ptr, hs.qbuf.ptr,
+                               hs.chunks.ptr, hs.kseg.ptr, hs.tiles.ptr};
     if (!(hs.graph_exec && hs.graph_key == key)) {
         if (hs.graph_exec) {
             DZ_HIP(hipGraphExecDestroy(hs.graph_exec));

@@ -127,3 +127,76 @@ def test_hamset_timing_vs_per_k_loop(dz, ctx, al35):
             h.set_stream(None)
         hs.set_stream(None)
         hs.close()
+
+
+@pytest.fixture(scope="module")
+def wide_set(dz, ctx):
+    """Two k-points of a 13 bohr cell with 128 projectors and about 6,100 plane waves: K-chunks of the
+    nonlocal products differ between 12 and 128 bands (in FP64)."""
+    from dzhip import tables, workloads
+
+    cell = 13.0 * np.eye(3)
+    recip = tables.reciprocal(cell)
+    grid = tables.auto_grid(30.0, recip)
+    rng = np.random.default_rng(17)
+    pos = rng.uniform(0.0, 13.0, size=(32, 3))
+    sp = workloads.SpeciesDesc([0, 1], [0.9, 1.1], np.diag([1.6, 0.7]))
+    local_r = rng.uniform(-1.0, 0.5, size=int(np.prod(grid)))
+    hams, blocks = [], []
+    for k in ((0.25, 0.25, 0.25), (0.0, 0.5, 0.1)):
+        basis = tables.generate_basis(recip, 30.0, np.asarray(k) @ recip)
+        phi = tables.build_phi(basis.kpg, sp.l_list, sp.radial_fns())
+        hams.append(dz.Hamiltonian(ctx, grid, tables.fft_indices(basis, grid), basis.kinetic, basis.cart, local_r,
+                                   1.0 / 13.0 ** 3, [{"l_list": sp.l_list, "dij": sp.dij, "phi": phi}], pos,
+                                   np.zeros(32, dtype=np.int32)))
+        blocks.append(rng.standard_normal((128, basis.n)) + 1j * rng.standard_normal((128, basis.n)))
+    yield hams, blocks
+    for h in hams:
+        h.close()
+
+
+def _set_reference(dz, hams, x, bands, prec):
+    """y of one eager apply of the first `bands` bands on a set of its own."""
+    import torch
+
+    hs = dz.HamSet(hams)
+    y = torch.zeros_like(x)
+    torch.cuda.synchronize()
+    hs.apply_dev(x.data_ptr(), y.data_ptr(), bands, prec)
+    torch.cuda.synchronize()
+    hs.close()
+    return y
+
+
+def _packed(hams, dz, blocks, prec):
+    import torch
+
+    hs = dz.HamSet(hams)
+    cdt, rdt = (np.complex128, np.float64) if prec == 0 else (np.complex64, np.float32)
+    x = torch.from_numpy(hs.pack([b.astype(cdt) for b in blocks]).view(rdt).copy()).cuda()
+    hs.close()
+    return x
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_hamset_graph_after_other_band_count(dz, ctx, wide_set, prec):
+    """A graph of 128 bands replayed after an apply of 12 (whose chunk tables are larger in FP64, so
+    the captured ones may have moved) gives what an eager apply gives, bit for bit."""
+    import torch
+
+    hams, blocks = wide_set
+    x = _packed(hams, dz, blocks, prec)
+    ref = _set_reference(dz, hams, x, 128, prec)
+    hs = dz.HamSet(hams)
+    try:
+        y, y12 = torch.zeros_like(x), torch.zeros_like(x)
+        for _ in range(3):
+            y.zero_()
+            torch.cuda.synchronize()
+            hs.apply_dev(x.data_ptr(), y.data_ptr(), 128, prec, use_graph=True)
+            torch.cuda.synchronize()
+            assert torch.equal(y, ref)
+            hs.apply_dev(x.data_ptr(), y12.data_ptr(), 12, prec)
+            torch.cuda.synchronize()
+    finally:
+        hs.close()
