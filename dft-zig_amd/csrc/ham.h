@@ -1,6 +1,8 @@
 // Per-k Hamiltonian context held on the device (host-side struct).
 #pragma once
 
+#include <map>
+
 #include "dzhip_internal.h"
 
 namespace dzhip {
@@ -230,10 +232,16 @@ struct HamSet {
     // Active z-row tables of the z-register plane kernels over the concatenated planes.
     int zrow_max = 0;
     DevBuf plane_pw0, plane_posr, plane_zstart, plane_zrows;
-    // Nonlocal segment tables for seg_cols columns in precision seg_prec (element size).
-    size_t seg_cols = 0;
-    int seg_prec = 0, nks_total = 0, ntiles = 0;
-    DevBuf chunks, kseg, tiles;
+    // Tables of the nonlocal products over the concatenated G axis: the G tiles, and per K-split asked
+    // for (a few values over all bands and precisions) the K-chunks and each k-point's range of them.
+    // Written once and kept: applies in flight and captured graphs go on reading them.
+    struct Chunks {
+        DevBuf chunks, kseg;
+        int nks_total = 0;
+    };
+    std::map<int, Chunks> splits;
+    DevBuf tiles;
+    int ntiles = 0;
     DevBuf tbuf, partial, qbuf;
     // Captured launch sequence and what it was captured for.
     struct GraphKey {
@@ -242,11 +250,10 @@ struct HamSet {
         size_t nc;
         int prec, code, pkind;
         hipStream_t s;
-        void *tbuf, *partial, *qbuf, *chunks, *kseg, *tiles;  // every buffer that may be reallocated
+        void *tbuf, *partial, *qbuf;  // every buffer that may be reallocated
         bool operator==(const GraphKey& o) const {
             return x == o.x && y == o.y && nc == o.nc && prec == o.prec && code == o.code && pkind == o.pkind &&
-                   s == o.s && tbuf == o.tbuf && partial == o.partial && qbuf == o.qbuf && chunks == o.chunks &&
-                   kseg == o.kseg && tiles == o.tiles;
+                   s == o.s && tbuf == o.tbuf && partial == o.partial && qbuf == o.qbuf;
         }
     };
     hipGraphExec_t graph_exec = nullptr;

@@ -1429,8 +1429,14 @@ constexpr int kNlG = 16 * kNlGWaves;
 // them in four subsets: rounding there is 1e-7, and the order of the sums is kept so that FP32 results
 // are the same bits for every tile shape.
 struct NlShape {
-    int blocks, btiles, wx, ptiles, nks, kchunk;
+    int blocks, btiles, wx, ptiles, split, nks, kchunk;  // split: K-chunks asked for
 };
+// K-chunks of npw plane waves where `split` are asked for: their number and length.
+static void nl_split(int npw, int split, int* nks, int* kchunk) {
+    const int n = std::max(1, std::min((npw + 2 * kNlK - 1) / (2 * kNlK), split));
+    *kchunk = (int)round_up((npw + n - 1) / n, 2 * kNlK);
+    *nks = (npw + *kchunk - 1) / *kchunk;
+}
 template <typename T>
 static NlShape nl_shape(int P, int npw, int ncols) {
     constexpr bool fp32 = std::is_same<T, float>::value;
@@ -1446,10 +1452,9 @@ static NlShape nl_shape(int P, int npw, int ncols) {
     s.wx = P <= 32 ? 2 : 4;
     s.ptiles = std::max(1, (P + 16 * s.wx - 1) / (16 * s.wx));
     const int tiles = fp32 ? std::max(1, (P + 63) / 64) * s.btiles : s.ptiles * s.btiles;
-    const int want = fp32 || s.blocks > 5 ? 256 : 512, ktiles = (npw + 2 * kNlK - 1) / (2 * kNlK);
-    s.nks = std::max(1, std::min(ktiles, (want + tiles - 1) / tiles));
-    s.kchunk = (int)round_up((npw + s.nks - 1) / s.nks, 2 * kNlK);
-    s.nks = (npw + s.kchunk - 1) / s.kchunk;
+    const int want = fp32 || s.blocks > 5 ? 256 : 512;
+    s.split = (want + tiles - 1) / tiles;
+    nl_split(npw, s.split, &s.nks, &s.kchunk);
     return s;
 }
 
@@ -2752,41 +2757,43 @@ void hamset_build(HamSet& hs) {
                                h.npw * sizeof(float2), h.npw * sizeof(float2), hs.nproj, hipMemcpyDeviceToDevice));
         }
     }
-    hs.seg_cols = 0;
 }
 
-// Nonlocal segment tables for ncols bands: per k-point the K-chunks a single context's apply of
-// that many columns would use, their ranges in the concatenated G axis, and the G tiles.
-template <typename T>
-static void hamset_segments(HamSet& hs, size_t nc) {
-    if (hs.seg_cols == nc && hs.seg_prec == (int)sizeof(T)) return;
-    std::vector<int> chunks, kseg;
-    std::vector<int> tiles;
-    for (size_t k = 0; k < hs.ks.size(); ++k) {
-        const int npw = (int)hs.ks[k]->npw;
-        const int off = (int)hs.npw_off[k];
-        // The same split as ham_apply_dev for this k-point alone.
-        const NlShape sh = nl_shape<T>(hs.nproj, npw, (int)nc);
-        kseg.push_back((int)chunks.size() / 2);
-        for (int c = 0; c < sh.nks; ++c) {
-            chunks.push_back(off + c * sh.kchunk);
-            chunks.push_back(off + std::min(npw, (c + 1) * sh.kchunk));
+// Tables of the nonlocal products for a K-split (NlShape::split): per k-point the K-chunks a single
+// context's apply would use and their range in the concatenated G axis; with the first, the G tiles.
+static const HamSet::Chunks& hamset_chunks(HamSet& hs, int split) {
+    if (!hs.tiles.ptr) {
+        std::vector<int> tiles;
+        for (size_t k = 0; k < hs.ks.size(); ++k) {
+            const int npw = (int)hs.ks[k]->npw, off = (int)hs.npw_off[k];
+            for (int g = 0; g < npw; g += kNlG) {
+                tiles.push_back(off + g);
+                tiles.push_back(off + npw);
+                tiles.push_back((int)k);
+                tiles.push_back(0);
+            }
         }
-        kseg.push_back((int)chunks.size() / 2);
-        for (int g = 0; g < npw; g += kNlG) {
-            tiles.push_back(off + g);
-            tiles.push_back(off + npw);
-            tiles.push_back((int)k);
-            tiles.push_back(0);
-        }
+        upload(hs.tiles, tiles);
+        hs.ntiles = (int)tiles.size() / 4;
     }
-    upload(hs.chunks, chunks);
-    upload(hs.kseg, kseg);
-    upload(hs.tiles, tiles);
-    hs.nks_total = (int)chunks.size() / 2;
-    hs.ntiles = (int)tiles.size() / 4;
-    hs.seg_cols = nc;
-    hs.seg_prec = (int)sizeof(T);
+    HamSet::Chunks& t = hs.splits[split];
+    if (t.nks_total > 0) return t;
+    std::vector<int> chunks, kseg;
+    for (size_t k = 0; k < hs.ks.size(); ++k) {
+        const int npw = (int)hs.ks[k]->npw, off = (int)hs.npw_off[k];
+        int nks = 0, kchunk = 0;
+        nl_split(npw, split, &nks, &kchunk);
+        kseg.push_back((int)chunks.size() / 2);
+        for (int c = 0; c < nks; ++c) {
+            chunks.push_back(off + c * kchunk);
+            chunks.push_back(off + std::min(npw, (c + 1) * kchunk));
+        }
+        kseg.push_back((int)chunks.size() / 2);
+    }
+    upload(t.chunks, chunks);
+    upload(t.kseg, kseg);
+    t.nks_total = (int)chunks.size() / 2;
+    return t;
 }
 
 // x-line kernel of the set: the register variant member 0 runs for this precision (tuned on its
@@ -2857,12 +2864,13 @@ static void hamset_launch(HamSet& hs, const void* xv, void* yv, size_t nc, int c
     if (do_nl) {
         // Tiles as one k-point's; its K-chunks come from the table.
         const NlShape sh = nl_shape<T>(hs.nproj, (int)h0.npw, (int)nc);
-        launch_nl_proj<T>(sh, hs.nks_total, a, x, ld, hs.partial.as<C>(), hs.nproj, (int)ld, (int)nc, hs.chunks.as<int2>(),
+        const HamSet::Chunks& t = hamset_chunks(hs, sh.split);
+        launch_nl_proj<T>(sh, t.nks_total, a, x, ld, hs.partial.as<C>(), hs.nproj, (int)ld, (int)nc, t.chunks.as<int2>(),
                           (int)ld, s);
         hipLaunchKernelGGL(k_nl_dij<T>, dim3((unsigned)nc, (unsigned)nk), dim3(kDijThreads),
-                           dij_lds_bytes(hs.nproj, sizeof(C)), s, hs.partial.as<C>(), hs.nks_total, hs.qbuf.as<C>(),
+                           dij_lds_bytes(hs.nproj, sizeof(C)), s, hs.partial.as<C>(), t.nks_total, hs.qbuf.as<C>(),
                            h0.meta.as<ProjMeta>(), Sel<T>::dm(h0), hs.nproj, (int)nc, (T)h0.inv_volume,
-                           dij_split(hs.nproj, sizeof(C)), hs.kseg.as<int2>());
+                           dij_split(hs.nproj, sizeof(C)), t.kseg.as<int2>());
         DZ_HIP(hipGetLastError());
         launch_nl_back<T>(sh, hs.ntiles, a, hs.qbuf.as<C>(), y, ld, hs.nproj, (int)ld, (int)nc, hs.tiles.as<int4>(), (int)ld, s);
     }
@@ -2886,12 +2894,12 @@ void hamset_apply_dev(HamSet& hs, const void* x, void* y, size_t nc, bool use_gr
     // Everything that allocates, synchronises or sets kernel attributes happens here, before
     // the launch sequence (which a graph may capture).
     const int code = hamset_xline_code<T>(hs, nc, s);
-    hamset_segments<T>(hs, nc);
     hs.tbuf.ensure(nc * (size_t)hs.np_total * hs.ny * hs.nz * sizeof(C));
     if (hs.nproj > 0) {
-        hs.partial.ensure((size_t)hs.nks_total * nc * hs.nproj * sizeof(C));
+        const NlShape sh = nl_shape<T>(hs.nproj, (int)h0.npw, (int)nc);
+        hs.partial.ensure((size_t)hamset_chunks(hs, sh.split).nks_total * nc * hs.nproj * sizeof(C));
         hs.qbuf.ensure(hs.ks.size() * nc * hs.nproj * sizeof(C));
-        nl_prepare<T>(nl_shape<T>(hs.nproj, (int)h0.npw, (int)nc));
+        nl_prepare<T>(sh);
         set_max_dynamic_lds((const void*)k_nl_dij<T>, dij_lds_bytes(hs.nproj, sizeof(C)));
     }
     const int pkind = hamset_plane_kind<T>(hs);
@@ -2901,8 +2909,7 @@ void hamset_apply_dev(HamSet& hs, const void* x, void* y, size_t nc, bool use_gr
         hamset_launch<T>(hs, x, y, nc, code, pkind, s);
         return;
     }
-    const HamSet::GraphKey key{x, y, nc, (int)sizeof(T), code, pkind, s, hs.tbuf.ptr, hs.partial.ptr, hs.qbuf.ptr,
-                               hs.chunks.ptr, hs.kseg.ptr, hs.tiles.ptr};
+    const HamSet::GraphKey key{x, y, nc, (int)sizeof(T), code, pkind, s, hs.tbuf.ptr, hs.partial.ptr, hs.qbuf.ptr};
     if (!(hs.graph_exec && hs.graph_key == key)) {
         if (hs.graph_exec) {
             DZ_HIP(hipGraphExecDestroy(hs.graph_exec));
@@ -2934,9 +2941,13 @@ void hamset_release(HamSet& hs) {
     }
     DevBuf* bufs[] = {&hs.plane_start, &hs.plane_pw, &hs.plane_pos, &hs.plane_ystart, &hs.plane_ycols, &hs.kpl,
                       &hs.plane_pw0, &hs.plane_posr, &hs.plane_zstart, &hs.plane_zrows,
-                      &hs.kinetic64, &hs.kinetic32, &hs.a64, &hs.a32, &hs.chunks, &hs.kseg, &hs.tiles, &hs.tbuf,
-                      &hs.partial, &hs.qbuf};
+                      &hs.kinetic64, &hs.kinetic32, &hs.a64, &hs.a32, &hs.tiles, &hs.tbuf, &hs.partial, &hs.qbuf};
     for (DevBuf* b : bufs) b->release();
+    for (auto& e : hs.splits) {
+        e.second.chunks.release();
+        e.second.kseg.release();
+    }
+    hs.splits.clear();
 }
 
 template void hamset_apply_dev<double>(HamSet&, const void*, void*, size_t, bool);

@@ -200,3 +200,33 @@ def test_hamset_graph_after_other_band_count(dz, ctx, wide_set, prec):
             torch.cuda.synchronize()
     finally:
         hs.close()
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_hamset_band_counts_back_to_back(dz, ctx, wide_set, prec):
+    """Applies of 128 and 12 bands queued one after another without a wait in between, whose K-chunks
+    differ in FP64: each gives what it gives alone, bit for bit."""
+    import torch
+
+    hams, blocks = wide_set
+    x = _packed(hams, dz, blocks, prec)
+    ref = {bands: _set_reference(dz, hams, x, bands, prec) for bands in (128, 12)}
+    hs = dz.HamSet(hams)
+    stream = torch.cuda.Stream()
+    hs.set_stream(stream.cuda_stream)
+    try:
+        y = [torch.zeros_like(x) for _ in range(6)]
+        for bands in (128, 12):  # buffers and tables at their largest
+            hs.apply_dev(x.data_ptr(), y[0].data_ptr(), bands, prec)
+        stream.synchronize()
+        for t in y:
+            t.zero_()
+        torch.cuda.synchronize()
+        for i, t in enumerate(y):
+            hs.apply_dev(x.data_ptr(), t.data_ptr(), (128, 12)[i % 2], prec)
+        stream.synchronize()
+        for i, t in enumerate(y):
+            assert torch.equal(t, ref[(128, 12)[i % 2]]), i
+        hs.set_stream(None)
+    finally:
+        hs.close()
