@@ -1457,6 +1457,16 @@ static NlShape nl_shape(int P, int npw, int ncols) {
     nl_split(npw, s.split, &s.nks, &s.kchunk);
     return s;
 }
+// Partial sums (elements) of a call of ncols bands or of any fewer.  The split falls beyond five and ten
+// 16-band blocks, so the widest calls below may write more of them; a narrower call under a stream
+// capture cannot allocate.  chunks(shape): the K-chunks of a shape.
+template <typename T, typename F>
+static size_t nl_partials(int P, int npw, int ncols, F chunks) {
+    size_t most = 0;
+    for (int n : {ncols, std::min(ncols, 16 * 5), std::min(ncols, 16 * kNlMaxBlocks)})
+        most = std::max(most, (size_t)chunks(nl_shape<T>(P, npw, n)) * n * P);
+    return most;
+}
 
 template <typename T>
 __host__ __device__ constexpr size_t nl_proj_lds_bytes(int blocks, int wx) {
@@ -2548,7 +2558,7 @@ void ham_apply_dev(Ham& h, const void* xv, void* yv, size_t ncols, bool local, b
         // Launch shapes and buffers first: nothing may reallocate once two streams run.
         const NlShape sh = nl_shape<T>(h.nproj, (int)h.npw, (int)nc);
         if (do_nl) {
-            h.partial.ensure((size_t)sh.nks * nc * h.nproj * sizeof(C));
+            h.partial.ensure(nl_partials<T>(h.nproj, (int)h.npw, (int)nc, [](const NlShape& n) { return n.nks; }) * sizeof(C));
             h.qbuf.ensure(nc * h.nproj * sizeof(C));
         }
         C* tb = nullptr;
@@ -2896,10 +2906,11 @@ void hamset_apply_dev(HamSet& hs, const void* x, void* y, size_t nc, bool use_gr
     const int code = hamset_xline_code<T>(hs, nc, s);
     hs.tbuf.ensure(nc * (size_t)hs.np_total * hs.ny * hs.nz * sizeof(C));
     if (hs.nproj > 0) {
-        const NlShape sh = nl_shape<T>(hs.nproj, (int)h0.npw, (int)nc);
-        hs.partial.ensure((size_t)hamset_chunks(hs, sh.split).nks_total * nc * hs.nproj * sizeof(C));
+        hs.partial.ensure(nl_partials<T>(hs.nproj, (int)h0.npw, (int)nc, [&](const NlShape& n) {
+                              return hamset_chunks(hs, n.split).nks_total;
+                          }) * sizeof(C));
         hs.qbuf.ensure(hs.ks.size() * nc * hs.nproj * sizeof(C));
-        nl_prepare<T>(sh);
+        nl_prepare<T>(nl_shape<T>(hs.nproj, (int)h0.npw, (int)nc));
         set_max_dynamic_lds((const void*)k_nl_dij<T>, dij_lds_bytes(hs.nproj, sizeof(C)));
     }
     const int pkind = hamset_plane_kind<T>(hs);

@@ -513,3 +513,43 @@ def test_hpsi_nonlocal_band_tiles(dz, ctx, prec, natoms):
         print(f"natoms={natoms} prec={prec} nb={nb} err={err:.2e}", flush=True)
         assert err < (TOL64 if prec == 0 else TOL32)
     ham.close()
+
+
+@pytest.mark.parametrize("wide,narrow", [(96, 80), (256, 160), (160, 33)])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_hpsi_capture_after_wider_apply(dz, ctx, prec, wide, narrow):
+    """An apply of fewer bands than an eager one before it allocates nothing, so a caller can capture
+    it (128 projectors, 6,100 plane waves: the split of the nonlocal sums is finer for fewer bands);
+    three replays equal the eager result bit for bit."""
+    import torch
+
+    cell = 13.0 * np.eye(3)
+    recip = tables.reciprocal(cell)
+    grid = tables.auto_grid(30.0, recip)
+    rng = np.random.default_rng(17)
+    sp = workloads.SpeciesDesc([0, 1], [0.9, 1.1], np.diag([1.6, 0.7]))
+    basis = tables.generate_basis(recip, 30.0, np.zeros(3))
+    species = [{"l_list": sp.l_list, "dij": sp.dij, "phi": tables.build_phi(basis.kpg, sp.l_list, sp.radial_fns())}]
+    ham = dz.Hamiltonian(ctx, grid, tables.fft_indices(basis, grid), basis.kinetic, basis.cart,
+                         rng.uniform(-1.0, 0.5, size=int(np.prod(grid))), 1.0 / 13.0 ** 3, species,
+                         rng.uniform(0.0, 13.0, size=(32, 3)), np.zeros(32, dtype=np.int32))
+    x = torch.randn((wide, basis.n), dtype=torch.complex128 if prec == 0 else torch.complex64, device="cuda",
+                    generator=torch.Generator(device="cuda").manual_seed(5))
+    y, ref = torch.zeros_like(x), torch.zeros_like(x)
+    stream = torch.cuda.Stream()
+    ham.set_stream(stream.cuda_stream)
+    torch.cuda.synchronize()
+    ham.apply_dev(x.data_ptr(), y.data_ptr(), wide, prec)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream):
+        ham.apply_dev(x.data_ptr(), y.data_ptr(), narrow, prec)
+    ham.apply_dev(x.data_ptr(), ref.data_ptr(), narrow, prec)
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref)
+    ham.set_stream(None)
+    ham.close()
