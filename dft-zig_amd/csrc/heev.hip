@@ -196,7 +196,7 @@ struct Trd {
         const double xn2 = sums[0];
         double beta;
         double2 scale;
-        if (xn2 == 0.0 && alpha.y == 0.0) {
+        if (fma(alpha.y, alpha.y, xn2) == 0.0) {  // reduced already, or but for entries below 1e-162
             tau = make_double2(0.0, 0.0);
             beta = alpha.x;
             scale = make_double2(0.0, 0.0);
@@ -205,10 +205,11 @@ struct Trd {
             const double ir = rsqrt3(n2), nrm = n2 * ir;
             const double ib = alpha.x >= 0.0 ? -ir : ir;
             beta = alpha.x >= 0.0 ? -nrm : nrm;
-            tau = make_double2((beta - alpha.x) * ib, -alpha.y * ib);
-            const double2 den = make_double2(alpha.x - beta, alpha.y);
-            const double id = recip3(den.x * den.x + den.y * den.y);
-            scale = make_double2(den.x * id, -den.y * id);
+            // tau = 1 - alpha / beta and 1 / (alpha - beta) = -1 / (beta tau): |tau|^2 is between 1 and 4, where
+            // |alpha - beta|^2 has no reciprocal below a norm of 1e-154 (and comes an operation later).
+            tau = make_double2(fma(fabs(alpha.x), ir, 1.0), -alpha.y * ib);
+            const double id = recip3(tau.x * tau.x + tau.y * tau.y);
+            scale = make_double2(-(tau.x * ib) * id, tau.y * ib * id);
         }
 #pragma unroll
         for (int c = 0; c < CW; ++c) {

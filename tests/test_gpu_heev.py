@@ -172,3 +172,34 @@ def test_heev_shared_launch_falls_back_to_cooperative():
     assert out.returncode == 0, out.stderr[-2000:]
     dval, orth = map(float, out.stdout.split()[-2:])
     assert dval < 1e-12 * 30.0 and orth < 1e-12
+
+
+@pytest.mark.parametrize("tiny,bar", [(1e-150, 1e-12), (3e-155, 1e-12), (1e-158, 1e-6), (1e-170, 1e-12), (1e-310, 1e-12)])
+@pytest.mark.parametrize("m", [3, 70])
+def test_heev_tiny_columns(ctx, m, tiny, bar):
+    """One row coupled to the rest by a tiny fraction of its size.  Bars as above, but for 1e-158, whose
+    squares are subnormal numbers of about 1e-317: a norm from them, and with it the reflector, is good to
+    5e-324 / 1e-317 = 5e-7.  Below 1e-162 they are zero and the row is taken as decoupled."""
+    rng = np.random.default_rng(5000 + m)
+    g = rng.standard_normal((m, m)) + 1j * rng.standard_normal((m, m))
+    a = 0.5 * (g + g.conj().T)
+    a[0, 1:] *= tiny
+    a[1:, 0] *= tiny
+
+    def bars(b):
+        w, z = ctx.heev(b, m)
+        err = (np.max(np.abs(w - np.linalg.eigvalsh(b))), np.max(np.abs(z.conj().T @ z - np.eye(m))),
+               np.max(np.linalg.norm(b @ z - z * w, axis=0)))
+        scale = max(1.0, float(np.linalg.norm(b, 2)))
+        print(f"m={m} {tiny}: values {err[0]:.1e} orthonormality {err[1]:.1e} residual {err[2]:.1e}", flush=True)
+        assert err[0] <= bar * scale and err[1] <= bar and err[2] <= 10 * bar * scale
+
+    bars(a)
+    # The same in the last columns, and real (alpha has no imaginary part).
+    bars(np.ascontiguousarray(a[::-1, ::-1]))
+    bars(a.real.astype(complex))
+    # Tiny below an ordinary complex or real coupling of the first two rows.
+    a[1, 0] = 0.7 + 0.2j
+    a[0, 1] = a[1, 0].conj()
+    bars(a)
+    bars(a.real.astype(complex))
