@@ -16,10 +16,10 @@ struct ScfGrid {
     AxisTables tab;
     DevBuf g2, work, rho_in, rho_out, v_in, v_out, v_ion, local, part, hv, hr, slots, coef;
     // Exchange-correlation functional (DZHIP_XC_LDA_PZ or DZHIP_XC_PBE), reciprocal rows, the Hartree
-    // kernel [N] and PBE's second complex grid.
+    // kernel [N] and PBE's other complex grids.
     int xc = DZHIP_XC_LDA_PZ;
     double3 recip_rows[3] = {};
-    DevBuf work2, hartree;
+    DevBuf work2, work3, hartree;
     int hist_cap = 0;
     double diemac = 1.0, dielng = 1.0;  // model dielectric preconditioner of the Pulay residual
     std::vector<int> order;              // Pulay ring slots, oldest first

@@ -153,13 +153,13 @@ __device__ inline void pbe(double n, double g2, double* f, double* fn, double* f
 // are many workgroups, and the functional is what costs there).  Real fields share complex transforms
 // in pairs: with i G_c taken as zero at an even axis' Nyquist frequency (whose term is imaginary in r
 // space, where the real part is kept) the derivative of a real field is real, so
-//   d_x n + i d_y n = IFFT[(-G_y + i G_x) n(G)],   d_z n + i s V_H = IFFT[i (G_z + s K) n(G)],
+//   d_x n + i d_y n = IFFT[(-G_y + i G_x) n(G)],   d_z n = IFFT[i G_z n(G)],   V_H = IFFT[K n(G)],
 //   div b = Re IFFT[(G_y + i G_x) FFT(b_x + i b_y) + i G_z FFT(b_z)],
-// K the Hartree kernel 8 pi / G^2 (the mean over +G and -G, which is what the real part sees) and s a
-// power of two that keeps the two halves of a pair of like size.  PBE: five launches and six
-// transforms where there were some forty and ten, which launches bounded: 249 -> 100 us at 20 x 20 x
-// 20 (the xy-passes 16 each, on 20 CUs; barriers of their short lines bound them, k_xc_z 10, k_rho_z
-// 7, k_div_z 4, the rest launch gaps and the copies around them).  LDA: three launches.
+// K the Hartree kernel 8 pi / G^2 (the mean over +G and -G, which is what the real part sees).  V_H is no
+// field's partner: a transform rounds by the larger of a pair, and V_H would take d_z n's rounding times
+// 8 pi / G_min^2 (1e-13 Ry at 60 bohr, 4e-15 alone).  PBE: five launches and seven transforms where there
+// were some forty and ten, which launches bounded: 248 -> 103 us at 30 x 30 x 30 (101 with V_H as d_z n's
+// partner).  LDA: three launches.
 struct GridAxes {
     FftAxis ax, ay, az;
     const double2* tw;
@@ -177,16 +177,16 @@ __device__ __forceinline__ double3 deriv_g(int x, int y, int z, const GridAxes& 
                         fx * g.b1.z + fy * g.b2.z + fz * g.b3.z);
 }
 
-// xy-pass, out and back.  HARTREE: w1 = K w1.  GRADIENT: w1 = (-G_y + i G_x) w1 and w2 = i (G_z + s K)
-// w1.  DIVERGENCE: w1 = (G_y + i G_x) w1 + i G_z w2.  All times 1/N.  KP: points per thread.  DUAL
-// (planes whose two tiles fit LDS): where two fields go the same way, their planes lie side by side,
-// rows interleaved, in one transform (half the barriers).
+// xy-pass, out and back.  HARTREE: w1 = K w1.  GRADIENT: w1 = (-G_y + i G_x) w1, w2 = i G_z w1 and w3 =
+// K w1.  DIVERGENCE: w1 = (G_y + i G_x) w1 + i G_z w2.  All times 1/N.  KP: points per thread.  F: planes
+// in LDS; the fields that go the same way lie side by side there, rows interleaved, and share a
+// transform's barriers (F = 3 and 2), or take turns where so many planes do not fit (1).
 enum { kHartree = 0, kGradient = 1, kDivergence = 2 };
-template <int KIND, int KP, bool DUAL>
-__global__ __launch_bounds__(512) void k_gridxy(double2* __restrict__ w1, double2* __restrict__ w2,
-                                                const double* __restrict__ kern, double s, double scale, GridAxes g) {
+constexpr int gridxy_fields(int kind) { return kind == kGradient ? 3 : kind == kDivergence ? 2 : 1; }
+template <int KIND, int KP, int F>
+__global__ __launch_bounds__(512) void k_gridxy(double2* __restrict__ w1, double2* __restrict__ w2, double2* __restrict__ w3,
+                                                const double* __restrict__ kern, double scale, GridAxes g) {
     extern __shared__ double2 lds[];
-    constexpr int F = DUAL ? 2 : 1;
     const int nx = g.ax.n, ny = g.ay.n, half = nx + 1, pitch = F * half, tid = threadIdx.x, nthr = blockDim.x, np = nx * ny;
     double2 *twx = lds + pitch * ny, *twy = twx + nx;
     load_twiddles(twx, g.tw + g.ax.tw_off, nx, tid, nthr);
@@ -194,12 +194,12 @@ __global__ __launch_bounds__(512) void k_gridxy(double2* __restrict__ w1, double
     const size_t off = (size_t)blockIdx.x * np;
     const int *px = g.perm + g.ax.perm_off, *py = g.perm + g.ay.perm_off;
     const unsigned mx = div_magic(nx);
-    // Natural order in, digit-reversed out; fields: tiles in use.
+    // Natural order in, digit-reversed out; fields: planes in use (one or F).
     auto lines = [&](auto sign, int fields) {
         constexpr int S = decltype(sign)::value;
         lds_fft_lines<double, double2, false, S>(lds, g.ax, twx, LineSet{fields == F ? F * ny : ny, 1, fields == F ? half : pitch, nullptr},
                                                  tid, nthr);
-        lds_fft_lines<double, double2, false, S>(lds, g.ay, twy, LineSet{fields == 2 ? pitch : nx, pitch, 1, nullptr}, tid, nthr);
+        lds_fft_lines<double, double2, false, S>(lds, g.ay, twy, LineSet{fields > 1 ? pitch : nx, pitch, 1, nullptr}, tid, nthr);
     };
     const std::integral_constant<int, -1> fwd;
     const std::integral_constant<int, 1> inv;
@@ -215,70 +215,88 @@ __global__ __launch_bounds__(512) void k_gridxy(double2* __restrict__ w1, double
             dst[off + i] = lds[px[i - y * nx] + pitch * py[y] + shift];
         }
     };
-    double2 a[KP], b[KP];
+    double2 v[KP];  // this thread's points: spectrum of w1 (divergence: the sum's)
     load(w1, 0);
-    if constexpr (KIND == kDivergence && DUAL) load(w2, half);
+    if constexpr (KIND == kDivergence && F == 2) load(w2, half);
     __syncthreads();
-    lines(fwd, KIND == kDivergence && DUAL ? 2 : 1);
-    if constexpr (KIND == kDivergence && !DUAL) {
+    lines(fwd, KIND == kDivergence ? F : 1);
+    auto take = [&]() {
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
             const int i = tid + k * nthr, y = fdiv(i, nx, mx);
-            if (i < np) a[k] = lds[px[i - y * nx] + pitch * py[y]];
+            if (i < np) v[k] = lds[px[i - y * nx] + pitch * py[y]];
         }
         __syncthreads();
-        load(w2, 0);
-        __syncthreads();
-        lines(fwd, 1);
-    }
-#pragma unroll
-    for (int k = 0; k < KP; ++k) {
-        const int i = tid + k * nthr;
-        if (i >= np) continue;
-        const int y = fdiv(i, nx, mx), x = i - y * nx;
-        const double2* l = lds + px[x] + pitch * py[y];
-        const double3 q = deriv_g(x, y, blockIdx.x, g);
-        if constexpr (KIND == kHartree) {
-            const double f = kern[off + i] * scale;
-            a[k] = make_double2(f * l->x, f * l->y);
-        } else if constexpr (KIND == kGradient) {
-            const double f = q.z + s * kern[off + i];
-            const double2 v = make_double2(l->x * scale, l->y * scale);
-            a[k] = make_double2(-q.y * v.x - q.x * v.y, q.x * v.x - q.y * v.y);
-            b[k] = make_double2(-f * v.y, f * v.x);
-        } else {
-            const double2 p = DUAL ? l[0] : a[k], r = DUAL ? l[half] : l[0];
-            const double2 v = make_double2(p.x * scale, p.y * scale), u = make_double2(r.x * scale, r.y * scale);
-            a[k] = make_double2(q.y * v.x - q.x * v.y - q.z * u.y, q.x * v.x + q.y * v.y + q.z * u.x);
+    };
+    if constexpr (KIND != kDivergence || F == 1) take();
+    if constexpr (KIND == kDivergence) {
+        if constexpr (F == 1) {
+            load(w2, 0);
+            __syncthreads();
+            lines(fwd, 1);
         }
-    }
-    __syncthreads();
-    auto put = [&](const double2 (&v)[KP], int shift) {
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
-            const int i = tid + k * nthr, y = fdiv(i, nx, mx);
-            if (i < np) lds[i - y * nx + pitch * y + shift] = v[k];
+            const int i = tid + k * nthr;
+            if (i >= np) continue;
+            const int y = fdiv(i, nx, mx), x = i - y * nx;
+            const double2* l = lds + px[x] + pitch * py[y];
+            const double3 q = deriv_g(x, y, blockIdx.x, g);
+            const double2 p = F == 2 ? l[0] : v[k], r = F == 2 ? l[half] : l[0];
+            const double2 a = make_double2(p.x * scale, p.y * scale), b = make_double2(r.x * scale, r.y * scale);
+            v[k] = make_double2(q.y * a.x - q.x * a.y - q.z * b.y, q.x * a.x + q.y * a.y + q.z * b.x);
+        }
+        __syncthreads();
+    }
+    // Field f of the point's spectrum at its place in plane t.
+    auto put = [&](int f, int t) {
+#pragma unroll
+        for (int k = 0; k < KP; ++k) {
+            const int i = tid + k * nthr;
+            if (i >= np) continue;
+            const int y = fdiv(i, nx, mx), x = i - y * nx;
+            double2 u = v[k];
+            if (KIND == kHartree || (KIND == kGradient && f == 2)) {
+                const double h = kern[off + i] * scale;
+                u = make_double2(h * u.x, h * u.y);
+            } else if constexpr (KIND == kGradient) {
+                const double3 q = deriv_g(x, y, blockIdx.x, g);
+                u = make_double2(u.x * scale, u.y * scale);
+                u = f == 0 ? make_double2(-q.y * u.x - q.x * u.y, q.x * u.x - q.y * u.y) : make_double2(-q.z * u.y, q.z * u.x);
+            }
+            lds[x + pitch * y + half * t] = u;
         }
     };
-    put(a, 0);
-    if constexpr (KIND == kGradient && DUAL) put(b, half);
-    __syncthreads();
-    lines(inv, KIND == kGradient && DUAL ? 2 : 1);
-    store(w1, 0);
     if constexpr (KIND == kGradient) {
-        if constexpr (!DUAL) {
+        double2* const dst[3] = {w1, w2, w3};
+        if constexpr (F == 3) {
+#pragma unroll
+            for (int f = 0; f < 3; ++f) put(f, f);
             __syncthreads();
-            put(b, 0);
-            __syncthreads();
-            lines(inv, 1);
+            lines(inv, 3);
+#pragma unroll
+            for (int f = 0; f < 3; ++f) store(dst[f], f * half);
+        } else {
+#pragma unroll
+            for (int f = 0; f < 3; ++f) {
+                put(f, 0);
+                __syncthreads();
+                lines(inv, 1);
+                store(dst[f], 0);
+                __syncthreads();
+            }
         }
-        store(w2, DUAL ? half : 0);
+    } else {
+        put(0, 0);
+        __syncthreads();
+        lines(inv, 1);
+        store(w1, 0);
     }
 }
 
-// Columns of one z-pass workgroup (one y): kZCols of the first field, then as many of the second.  At the
-// longest axis (256) the tile is 72 KiB.
-constexpr int kZCols = 8, kZThreads = 256, kZPitch = 2 * kZCols + 1;
+// Columns of one z-pass workgroup (one y): kZCols of each field, side by side.  At the longest axis (256)
+// the tile of the GGA's three fields is 104 KiB.
+constexpr int kZCols = 8, kZThreads = 256, kZPitch = 2 * kZCols + 1, kZPitchGga = 3 * kZCols + 1;
 struct ZCols {
     int nx, y, x0, cols, cnt, ny;
     __device__ __forceinline__ ZCols(const GridAxes& g)
@@ -306,42 +324,47 @@ __global__ __launch_bounds__(kZThreads) void k_rho_z(const double* __restrict__ 
         if (c.in(i)) w[c.at(i)] = lds[i % kZCols + kZPitch * pz[i / kZCols]];
 }
 
-// z-pass in r space: V_H (and the gradient), the functional at every point, the workgroup's sums
-// [V_H rho, f_xc, v_in rho, (rho - rho_in)^2], and, GGA, b's z-transforms back into w1 and w2.
-// vout = V_H + df/dn (LDA: V_H + v_xc).
+// z-pass in r space: V_H (GGA: in w3, the gradient in w1 and w2), the functional at every point, the
+// workgroup's sums [V_H rho, f_xc, v_in rho, (rho - rho_in)^2], and, GGA, b's z-transforms back into w1
+// and w2.  vout = V_H + df/dn (LDA: V_H + v_xc).
 template <bool GGA>
 __global__ __launch_bounds__(kZThreads) void k_xc_z(double2* __restrict__ w1, double2* __restrict__ w2,
+                                                    const double2* __restrict__ w3,
                                                     const double* __restrict__ rho, const double* __restrict__ rho_in,
                                                     const double* __restrict__ vin, double* __restrict__ vout,
-                                                    double* __restrict__ part, double inv_s, GridAxes g) {
+                                                    double* __restrict__ part, GridAxes g) {
     extern __shared__ double2 lds[];
     __shared__ double red[4][kZThreads / 64];
+    constexpr int P = GGA ? kZPitchGga : kZPitch;
     const ZCols c(g);
     const int nz = g.az.n, tid = threadIdx.x;
     const int* pz = g.perm + g.az.perm_off;
-    double2* tw = lds + kZPitch * nz;
+    double2* tw = lds + P * nz;
     load_twiddles(tw, g.tw + g.az.tw_off, nz, tid, kZThreads);
     for (int i = tid; i < c.cnt; i += kZThreads) {
-        double2* l = lds + i % kZCols + kZPitch * pz[i / kZCols];
+        double2* l = lds + i % kZCols + P * pz[i / kZCols];
         const bool in = c.in(i);
         l[0] = in ? w1[c.at(i)] : make_double2(0.0, 0.0);
-        if constexpr (GGA) l[kZCols] = in ? w2[c.at(i)] : make_double2(0.0, 0.0);
+        if constexpr (GGA) {
+            l[kZCols] = in ? w2[c.at(i)] : make_double2(0.0, 0.0);
+            l[2 * kZCols] = in ? w3[c.at(i)] : make_double2(0.0, 0.0);
+        }
     }
     __syncthreads();
-    lds_fft_lines<double, double2, true, 1>(lds, g.az, tw, LineSet{GGA ? 2 * kZCols : kZCols, kZPitch, 1, nullptr}, tid,
+    lds_fft_lines<double, double2, true, 1>(lds, g.az, tw, LineSet{GGA ? 3 * kZCols : kZCols, P, 1, nullptr}, tid,
                                             kZThreads);
     double sums[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll 1
     for (int i = tid; i < c.cnt; i += kZThreads) {
         if (!c.in(i)) continue;
-        double2* l = lds + i % kZCols + kZPitch * (i / kZCols);
+        double2* l = lds + i % kZCols + P * (i / kZCols);
         const size_t at = c.at(i);
         const double r = rho[at];
         double f, v, h;
         if constexpr (GGA) {
             const double gx = l[0].x, gy = l[0].y, gz = l[kZCols].x;
             double fg;
-            h = l[kZCols].y * inv_s;
+            h = l[2 * kZCols].x;
             pbe(r, gx * gx + gy * gy + gz * gz, &f, &v, &fg);
             l[0] = make_double2(fg * gx, fg * gy);
             l[kZCols] = make_double2(fg * gz, 0.0);
@@ -369,10 +392,10 @@ __global__ __launch_bounds__(kZThreads) void k_xc_z(double2* __restrict__ w1, do
         part[4 * (blockIdx.x + gridDim.x * blockIdx.y) + tid] = s;
     }
     if constexpr (GGA) {
-        lds_fft_lines<double, double2, false, -1>(lds, g.az, tw, LineSet{2 * kZCols, kZPitch, 1, nullptr}, tid, kZThreads);
+        lds_fft_lines<double, double2, false, -1>(lds, g.az, tw, LineSet{2 * kZCols, P, 1, nullptr}, tid, kZThreads);
         for (int i = tid; i < c.cnt; i += kZThreads) {
             if (!c.in(i)) continue;
-            const double2* l = lds + i % kZCols + kZPitch * pz[i / kZCols];
+            const double2* l = lds + i % kZCols + P * pz[i / kZCols];
             w1[c.at(i)] = l[0];
             w2[c.at(i)] = l[kZCols];
         }
@@ -481,22 +504,23 @@ double ScfGrid::dot(const double* a, const double* c) {
 }
 
 namespace {
-// Threads and points per thread of an xy-pass by the plane's points (its tile fits LDS: at most 10,240).
+// Threads and points per thread of an xy-pass by the plane's points (one tile in LDS: at most 10,240; two:
+// 5,120; three: 3,413, and always up to 1,024).
 template <int KIND>
-void launch_gridxy(int nx, int ny, int nz, hipStream_t s, double2* w1, double2* w2, const double* kern, double sc,
+void launch_gridxy(int nx, int ny, int nz, hipStream_t s, double2* w1, double2* w2, double2* w3, const double* kern,
                    double scale, const GridAxes& g) {
+    constexpr int F = gridxy_fields(KIND);
     const int np = nx * ny;
     size_t lds = fft_xy_lds_bytes(nx, ny, sizeof(double2));
-    const size_t lds2 = lds + (size_t)(nx + 1) * ny * sizeof(double2);
-    const bool dual = KIND != kHartree && lds2 <= kMaxLdsBytes;
-    if (dual) lds = lds2;
-    constexpr bool D = KIND != kHartree;
-    auto* fn = dual ? (np <= 1024 ? k_gridxy<KIND, 4, D> : k_gridxy<KIND, 12, D>)
-                    : (np <= 1024   ? k_gridxy<KIND, 4, false>
-                       : np <= 6144 ? k_gridxy<KIND, 12, false>
-                                    : k_gridxy<KIND, 20, false>);
+    const size_t all = lds + (size_t)(F - 1) * (nx + 1) * ny * sizeof(double2);
+    const bool together = F > 1 && all <= kMaxLdsBytes;
+    if (together) lds = all;
+    auto* fn = np <= 1024   ? k_gridxy<KIND, 4, F>
+               : together   ? k_gridxy<KIND, F == 3 ? 8 : 12, F>
+               : np <= 6144 ? k_gridxy<KIND, 12, 1>
+                            : k_gridxy<KIND, 20, 1>;
     set_max_dynamic_lds((const void*)fn, lds);
-    hipLaunchKernelGGL(fn, dim3((unsigned)nz), dim3(np <= 1024 ? 256 : 512), lds, s, w1, w2, kern, sc, scale, g);
+    hipLaunchKernelGGL(fn, dim3((unsigned)nz), dim3(np <= 1024 ? 256 : 512), lds, s, w1, w2, w3, kern, scale, g);
     DZ_HIP(hipGetLastError());
 }
 }  // namespace
@@ -509,12 +533,8 @@ void ScfGrid::hxc(const double* rho, const double* rho_ref, const double* vin, d
     DZ_REQUIRE(fft_xy_lds_bytes(nx, ny, sizeof(double2)) <= kMaxLdsBytes &&
                    fft_z_lds_bytes(nx, nz, sizeof(double2)) <= kMaxLdsBytes,
                DZHIP_ERR_HIP, "SCF grid: plane too large for the FFT kernels' LDS");
-    double2 *w1 = work.as<double2>(), *w2 = work2.as<double2>();
+    double2 *w1 = work.as<double2>(), *w2 = work2.as<double2>(), *w3 = work3.as<double2>();
     double *kern = hartree.as<double>(), *sums = part.as<double>();
-    // s V_H is at most about n, as the gradient of a valence density (a bohr's scale) is.
-    double g2min = 1e300;
-    for (const double3& b : recip_rows) g2min = std::min(g2min, b.x * b.x + b.y * b.y + b.z * b.z);
-    const double sc = std::exp2(std::rint(std::log2(g2min / (8.0 * M_PI))));
     const double scale = 1.0 / (double)n;
     const dim3 gz((unsigned)((nx + kZCols - 1) / kZCols), (unsigned)ny);
     const size_t ldsz = (size_t)(kZPitch + 1) * nz * sizeof(double2);
@@ -522,18 +542,19 @@ void ScfGrid::hxc(const double* rho, const double* rho_ref, const double* vin, d
     hipLaunchKernelGGL(k_rho_z, gz, dim3(kZThreads), ldsz, s, rho, w1, g);
     DZ_HIP(hipGetLastError());
     if (gga) {
-        launch_gridxy<kGradient>(nx, ny, nz, s, w1, w2, kern, sc, scale, g);
-        set_max_dynamic_lds((const void*)k_xc_z<true>, ldsz);
-        hipLaunchKernelGGL(k_xc_z<true>, gz, dim3(kZThreads), ldsz, s, w1, w2, rho, rho_ref, vin, vout, sums, 1.0 / sc, g);
+        launch_gridxy<kGradient>(nx, ny, nz, s, w1, w2, w3, kern, scale, g);
+        const size_t ldsg = (size_t)(kZPitchGga + 1) * nz * sizeof(double2);
+        set_max_dynamic_lds((const void*)k_xc_z<true>, ldsg);
+        hipLaunchKernelGGL(k_xc_z<true>, gz, dim3(kZThreads), ldsg, s, w1, w2, w3, rho, rho_ref, vin, vout, sums, g);
         DZ_HIP(hipGetLastError());
-        launch_gridxy<kDivergence>(nx, ny, nz, s, w1, w2, kern, sc, scale, g);
+        launch_gridxy<kDivergence>(nx, ny, nz, s, w1, w2, w3, kern, scale, g);
         set_max_dynamic_lds((const void*)k_div_z, ldsz);
         hipLaunchKernelGGL(k_div_z, gz, dim3(kZThreads), ldsz, s, w1, vout, g);
         DZ_HIP(hipGetLastError());
     } else {
-        launch_gridxy<kHartree>(nx, ny, nz, s, w1, w2, kern, sc, scale, g);
+        launch_gridxy<kHartree>(nx, ny, nz, s, w1, w2, w3, kern, scale, g);
         set_max_dynamic_lds((const void*)k_xc_z<false>, ldsz);
-        hipLaunchKernelGGL(k_xc_z<false>, gz, dim3(kZThreads), ldsz, s, w1, w2, rho, rho_ref, vin, vout, sums, 1.0, g);
+        hipLaunchKernelGGL(k_xc_z<false>, gz, dim3(kZThreads), ldsz, s, w1, w2, w3, rho, rho_ref, vin, vout, sums, g);
         DZ_HIP(hipGetLastError());
     }
     if (!out) return;
@@ -595,7 +616,7 @@ ScfGrid* scf_grid_create(Context* ctx, int nx, int ny, int nz, const double* rec
 void scf_grid_destroy(ScfGrid* g) {
     if (!g) return;
     DevBuf* bufs[] = {&g->g2, &g->work, &g->rho_in, &g->rho_out, &g->v_in, &g->v_out, &g->v_ion, &g->local,
-                      &g->part, &g->hv, &g->hr, &g->slots, &g->coef, &g->work2, &g->hartree};
+                      &g->part, &g->hv, &g->hr, &g->slots, &g->coef, &g->work2, &g->work3, &g->hartree};
     for (DevBuf* b : bufs) b->release();
     g->tab.release();
     delete g;
@@ -746,6 +767,7 @@ void scf_grid_mix(ScfGrid& g, double beta, int pulay) {
 void scf_grid_set_xc(ScfGrid& g, int functional) {
     if (functional == DZHIP_XC_PBE) {
         g.work2.ensure(g.n * sizeof(double2));
+        g.work3.ensure(g.n * sizeof(double2));
     }
     g.xc = functional;
 }

@@ -319,3 +319,41 @@ def test_scf_pbe_al(dz, ctx, concurrent):
     assert np.max(np.abs(e[:m] - gold["energies"][:m])) < 1e-8
     assert np.max(np.abs(np.array(run.eigenvalues) - gold["eigenvalues"])) < EV_TOL
     assert float(np.sum(np.abs(run.rho - gold["rho"]))) * s.volume / run.rho.size < RHO_L1
+
+
+@pytest.mark.parametrize("shape,lengths", [((60, 64, 54), (60.0, 60.0, 60.0)), ((96, 90, 40), (55.0, 60.0, 20.0)),
+                                           ((32, 30, 180), (20.0, 20.0, 120.0)), ((45, 48, 50), (30.0, 30.0, 30.0))])
+@pytest.mark.parametrize("xc", ["lda_pz", "pbe"])
+def test_scf_grid_hartree_large_cells(dz, ctx, shape, lengths, xc):
+    """V_H of a few atoms in large cells against 80-bit transforms.  The density is below 1e-12, where both
+    functionals are zero, so V_in is V_H.  eps log2(N) / 2 of max |V_H|: a transform's error is about
+    0.6 u sqrt(log2 N) of the rms value, u = eps / 2, here twice and at five times its rms at most."""
+    import scipy.fft
+
+    n = int(np.prod(shape))
+    recip = 2.0 * np.pi * np.linalg.inv(np.diag(lengths)).T
+    rng = np.random.default_rng(1)
+    rho = np.full(shape, 0.02)
+    for _ in range(4):
+        c = rng.random(3) * lengths
+        r2 = [np.minimum(np.abs(np.arange(m) / m * l - ci), l - np.abs(np.arange(m) / m * l - ci)) ** 2
+              for m, l, ci in zip(shape, lengths, c)]
+        rho += 0.3 * np.exp(-(r2[0][:, None, None] + r2[1][None, :, None] + r2[2][None, None, :]) / (2 * 1.2 ** 2))
+    rho *= 1e-13
+    g = [np.fft.fftfreq(m, 1.0 / m).astype(np.longdouble) * np.longdouble(recip[i, i]) for i, m in enumerate(shape)]
+    g2 = g[0][:, None, None] ** 2 + g[1][None, :, None] ** 2 + g[2][None, None, :] ** 2
+    g2[0, 0, 0] = 1.0
+    k = 8.0 * np.longdouble(np.pi) / g2
+    k[0, 0, 0] = 0.0
+    ref = scipy.fft.ifftn(k * scipy.fft.fftn(rho.astype(np.clongdouble))).real
+    grid = dz.ScfGrid(ctx, shape, recip, float(np.prod(lengths)))
+    try:
+        grid.set_xc(xc)
+        grid.init_rho(np.ascontiguousarray(rho.transpose(2, 1, 0)).reshape(-1))
+        got = grid.read(dz.GRID_VIN).reshape(shape[::-1]).transpose(2, 1, 0)
+    finally:
+        grid.close()
+    err = float(np.max(np.abs(got - ref)) / np.max(np.abs(ref)))
+    tol = np.finfo(np.float64).eps * np.log2(n) / 2
+    print(f"{shape} {xc} error {err:.2e} of max |V_H|, bar {tol:.2e}", flush=True)
+    assert err < tol
