@@ -10,11 +10,12 @@
 #include <cstdlib>
 #include <mutex>
 
+#include "trd_shape.h"
+
 namespace dzhip {
 
 namespace {
 
-constexpr int kTrdWaves = 4;  // wavefronts per workgroup of the tridiagonalisation, one per SIMD
 constexpr unsigned kSpinLimit = 1u << 22;  // polls of one exchange (under a microsecond each) before giving up
 // The same for a tridiagonalisation admitted by the gate: its grid may find the device short
 // of CUs for a long time while other streams' kernels keep taking them, and it is then repeated as
@@ -1100,10 +1101,9 @@ struct TrdKernel {
     const void* fn;
     size_t lds() const { return (size_t)4 * 64 * nq * sizeof(double2); }
 };
-#define DZ_TRD(NQ) {NQ, 1, (const void*)k_hetrd<NQ, 1>}, {NQ, 2, (const void*)k_hetrd<NQ, 2>}
-const TrdKernel kTrdKernels[] = {DZ_TRD(1), DZ_TRD(2), DZ_TRD(3), DZ_TRD(4), DZ_TRD(6),
-                                 DZ_TRD(8), DZ_TRD(11), DZ_TRD(13), DZ_TRD(16)};
-#undef DZ_TRD
+#define DZ_TRD_ENTRY(NQ, CW) {NQ, CW, (const void*)k_hetrd<NQ, CW>},
+const TrdKernel kTrdKernels[] = {DZ_TRD_INSTANCES(DZ_TRD_ENTRY)};
+#undef DZ_TRD_ENTRY
 
 // Co-resident workgroups per device for the tridiagonalisation (one per CU at its LDS size),
 // queried once per device.
@@ -1125,37 +1125,32 @@ CoopInfo coop_info(int dev) {
         DZ_REQUIRE(coop != 0, DZHIP_ERR_HIP, "device does not support cooperative launches");
         for (const TrdKernel& k : kTrdKernels) set_max_dynamic_lds(k.fn, k.lds());
         set_max_dynamic_lds((const void*)k_stein, stein_lds_bytes(kHeevMaxM));
-        // Launch-shape override for sweeps: trailing columns per workgroup (4 or 8).
+        // Launch-shape override: at least so many trailing columns per workgroup (4, 8 or 16).
         if (const char* env = std::getenv("DZHIP_HEEV_COLS")) c.cols_per_group = std::max(0, std::atoi(env));
         c.groups = cus;
     }
     return c;
 }
 
-// Launch shape of the tridiagonalisation: the instance and its G workgroups.  One column per
-// wavefront while the workgroups fit the device (m <= 1024 on 256 CUs): a step's chain is latency
-// and the redundant vector work of each wavefront, so a second column only lengthens it (m = 164 /
-// 328 / 648, whole eigensolver call, us: 821 / 1786 / 4013 with one, 856 / 1891 / 4560 with two).
-// This kernel alone: 1,024 -> 400 us at m = 164 and 4,887 -> 2,150 us at m = 648 (6.2 -> 2.4 and
-// 7.5 -> 3.3 us a reflector) against columns in LDS shared by four wavefronts with block sums and a
-// grid barrier.
+// Launch shape of the tridiagonalisation: the instance and its G workgroups (trd_pick).  On 256 CUs every
+// size takes one column per wavefront; whole eigensolver calls with one / two of them, us: m = 164
+// 577 / 626, 328 1,420 / 1,547, 648 (300 vectors) 3,152 / 3,718.  This kernel alone at one: 1,024 -> 400 us
+// at m = 164 and 4,887 -> 2,150 us at m = 648 (6.2 -> 2.4 and 7.5 -> 3.3 us a reflector) against columns in
+// LDS shared by four wavefronts with block sums and a grid barrier.
 TrdKernel trd_shape(int m, int* G_out) {
     int dev = 0;
     DZ_HIP(hipGetDevice(&dev));
     const CoopInfo ci = coop_info(dev);
+    const TrdPick p = trd_pick(m, ci.groups, ci.cols_per_group);
     const TrdKernel* k = nullptr;
-    int cw = ci.cols_per_group >= 2 * kTrdWaves ? 2 : 1;
-    if ((m + kTrdWaves * cw - 1) / (kTrdWaves * cw) > ci.groups) cw = 2;
     for (const TrdKernel& c : kTrdKernels)
-        if (!k && c.cw == cw && m <= 64 * c.nq) k = &c;
-    const int G = (m + kTrdWaves * cw - 1) / (kTrdWaves * cw);
+        if (c.nq == p.nq && c.cw == p.cw) k = &c;
     DZ_REQUIRE(k, DZHIP_ERR_ARG, "Hermitian eigensolver: matrix too large for the tridiagonalisation");
     // Every workgroup must be co-resident.
     int per_cu = 0;
     DZ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k->fn, 64 * kTrdWaves, k->lds()));
-    DZ_REQUIRE(per_cu >= 1 && G <= per_cu * ci.groups, DZHIP_ERR_HIP,
-               "Hermitian eigensolver: grid does not fit on the device");
-    *G_out = G;
+    DZ_REQUIRE(per_cu >= 1, DZHIP_ERR_HIP, "Hermitian eigensolver: grid does not fit on the device");
+    *G_out = p.groups;
     return *k;
 }
 

@@ -203,3 +203,37 @@ def test_heev_tiny_columns(ctx, m, tiny, bar):
     a[0, 1] = a[1, 0].conj()
     bars(a)
     bars(a.real.astype(complex))
+
+
+@pytest.mark.parametrize("cols,sizes", [(8, (1, 8, 9, 129, 193, 257, 385, 513, 705, 833, 1024)),
+                                        (16, (1, 16, 17, 257, 384, 385, 513, 704))])
+def test_heev_columns_per_workgroup(cols, sizes):
+    """The tridiagonalisation's instances of two and four columns a wavefront, which a device of fewer CUs
+    takes, selected from the host in a child process (DZHIP_HEEV_COLS), at the edges of their sizes;
+    bars as above, against LAPACK's eigenvalues."""
+    import os
+    import subprocess
+    import sys
+    from pathlib import Path
+
+    root = Path(__file__).resolve().parents[1]
+    script = (
+        "import sys, numpy as np; sys.path.insert(0, %r); import dzhip\n"
+        "ctx = dzhip.Context(0)\n"
+        "for m in %r:\n"
+        "    rng = np.random.default_rng(6000 + m); g = rng.standard_normal((m, m)) + 1j * rng.standard_normal((m, m))\n"
+        "    a = 0.5 * (g + g.conj().T); nev = min(m, 24); print('m', m, file=sys.stderr, flush=True)\n"
+        "    w, z = ctx.heev(a, nev); s = max(1.0, float(np.linalg.norm(a, 2)))\n"
+        "    print(m, np.max(np.abs(w - np.linalg.eigvalsh(a)[:nev])) / s, np.max(np.abs(z.conj().T @ z - np.eye(nev))),\n"
+        "          np.max(np.linalg.norm(a @ z - z * w, axis=0)) / s, flush=True)\n"
+    ) % (str(root / "dft-zig_amd"), sizes)
+    print(f"child: heev of {sizes} with DZHIP_HEEV_COLS={cols}", flush=True)
+    out = subprocess.run([sys.executable, "-c", script], env=dict(os.environ, DZHIP_HEEV_COLS=str(cols)),
+                         capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr[-2000:]
+    lines = [l.split() for l in out.stdout.splitlines()]
+    assert [int(l[0]) for l in lines] == list(sizes)
+    for l in lines:
+        print(*l, flush=True)
+        dval, orth, res = map(float, l[1:])
+        assert dval <= 1e-12 and orth <= 1e-12 and res <= 1e-11
