@@ -148,7 +148,7 @@ struct Trd {
     const TrdArgs& a;
     double2* lds;  // two steps' [p | column j], M64 rows each
     double2* s_x;  // two steps' [NW * CW own columns' next row | v's next row]
-    int* s_bad;
+    int* s_bad;    // two steps' flag: the exchange gave up
     int m, t, lane, wv, last_col;
     bool scribe;  // the wavefront that owns the last column writes T and the reflectors
     int ic[CW];
@@ -286,7 +286,7 @@ struct Trd {
             if (spins > a.spin_limit || __any(stop)) {
                 if (lane == 0) {
                     __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    *s_bad = 1;
+                    s_bad[j & 1] = 1;
                 }
                 break;
             }
@@ -300,7 +300,7 @@ struct Trd {
             }
         }
         __syncthreads();
-        if (*s_bad) return false;
+        if (s_bad[j & 1]) return false;  // by step parity: a faster wavefront may already give up in the next one
         // Rows below j of sp and sn are an earlier step's (finite) and meet v = 0 there; rows from m
         // on are zero.
         const double2* sx = s_x + ((j - 1) & 1) * (NW * CW + 1);
@@ -379,15 +379,15 @@ template <int NQ, int CW>
 __global__ __launch_bounds__(64 * kTrdWaves, 1) void k_hetrd(TrdArgs a) {
     extern __shared__ double2 lds[];
     __shared__ double2 s_x[2 * (kTrdWaves * CW + 1)];
-    __shared__ int s_bad;
+    __shared__ int s_bad[2];
     using K = Trd<NQ, CW>;
     const int t = (int)threadIdx.x, g = (int)blockIdx.x, m = a.m;
-    K k{a, lds, s_x, &s_bad, m, t, t & 63, __builtin_amdgcn_readfirstlane(t >> 6)};
+    K k{a, lds, s_x, s_bad, m, t, t & 63, __builtin_amdgcn_readfirstlane(t >> 6)};
     k.last_col = min(m, (g + 1) * K::NW * CW) - 1;
     k.scribe = false;
     for (int i = t; i < 4 * K::M64; i += K::NT) lds[i] = make_double2(0.0, 0.0);
     if (t < 2 * (K::NW * CW + 1)) s_x[t] = make_double2(0.0, 0.0);
-    if (t == 0) s_bad = 0;
+    if (t < 2) s_bad[t] = 0;
 #pragma unroll
     for (int c = 0; c < CW; ++c) {
         const int i = k.ic[c] = (g * K::NW + k.wv) * CW + c;

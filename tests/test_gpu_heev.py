@@ -237,3 +237,35 @@ def test_heev_columns_per_workgroup(cols, sizes):
         print(*l, flush=True)
         dval, orth, res = map(float, l[1:])
         assert dval <= 1e-12 and orth <= 1e-12 and res <= 1e-11
+
+
+def test_heev_shared_launch_repeats_are_counted():
+    """With the admitted launch's spin limit at one poll the exchange gives up (every workgroup exits
+    normally, whichever of its wavefronts gives up first) and the call is repeated cooperatively: sizes of
+    two to 162 workgroups, each call counted as a repeat and its spectrum LAPACK's (1e-12 of the largest
+    eigenvalue)."""
+    import os
+    import subprocess
+    import sys
+    from pathlib import Path
+
+    root = Path(__file__).resolve().parents[1]
+    sizes = (40, 164, 328, 648)
+    script = (
+        "import sys, numpy as np; sys.path.insert(0, %r); import dzhip\n"
+        "ctx = dzhip.Context(0)\n"
+        "for m in %r:\n"
+        "    rng = np.random.default_rng(7000 + m); g = rng.standard_normal((m, m)) + 1j * rng.standard_normal((m, m))\n"
+        "    a = 0.5 * (g + g.conj().T); ref = np.linalg.eigvalsh(a)[:20]; before = dzhip.heev_retries()\n"
+        "    w, _ = ctx.heev(a, 20)\n"
+        "    print(m, np.max(np.abs(w - ref)) / np.max(np.abs(ref)), dzhip.heev_retries() - before, flush=True)\n"
+    ) % (str(root / "dft-zig_amd"), sizes)
+    print(f"child: heev of {sizes} with DZHIP_HEEV_SHARED_SPIN=1", flush=True)
+    out = subprocess.run([sys.executable, "-c", script], env=dict(os.environ, DZHIP_HEEV_SHARED_SPIN="1"),
+                         capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr[-2000:]
+    lines = [l.split() for l in out.stdout.splitlines()]
+    assert [int(l[0]) for l in lines] == list(sizes)
+    for l in lines:
+        print(*l, flush=True)
+        assert float(l[1]) < 1e-12 and int(l[2]) == 1
