@@ -512,10 +512,6 @@ static void section_times(EigWork& w, double* out) {
     w.ev_used = 0;
 }
 
-// Lowest nev eigenpairs of the Hermitian m x m matrix A (lower triangle, leading dimension lda)
-// into Y (leading dimension ldy) and the host vector returned (ascending).  The library's device
-// eigensolver up to m = kHeevMaxM; rocSOLVER zheevd beyond (it overwrites a copy of A in Y,
-// which must then hold m columns).
 // Upper Cholesky factorisation S = R^H R of a Hermitian k x k matrix (column-major, leading dimension
 // ld; the upper triangle of S is read, A gets R and zeros below it), k <= kPotrfMax, one workgroup,
 // right-looking in blocks of kPotrfNb rows:
@@ -780,7 +776,10 @@ __global__ __launch_bounds__(256) void k_chol_check(const double2* __restrict__ 
     }
 }
 
-// Lowest nev eigenpairs of A; the eigenvalues in w.evals and, once s is synchronised, w.host_evals.
+// Lowest nev eigenpairs of the Hermitian m x m matrix A (lower triangle, leading dimension lda): vectors into
+// Y (leading dimension ldy), values, ascending, into w.evals and, once s is synchronised, w.host_evals.  The
+// library's device eigensolver up to m = kHeevMaxM; rocSOLVER zheevd beyond (it overwrites a copy of A in Y,
+// which must then hold m columns).
 static void subspace_eigh(EigWork& w, const double2* A, int lda, int m, int nev, double2* Y, int ldy, hipStream_t s) {
     if (m <= kHeevMaxM) {
         heev_lowest_shared(w.heev, A, lda, m, nev, w.evals.as<double>(), Y, ldy, s);
@@ -861,23 +860,18 @@ struct Solver {
         DZ_HIP(hipGetLastError());
     }
 
-    void gemm(rocblas_operation ta, rocblas_operation tb, int m, int nn, int k, zc alpha, const double2* A,
-              int lda, const double2* B, int ldb, zc beta, double2* C, int ldc) {
+    // C[:, 0:nn] = alpha A[:, 0:k] B[0:k, 0:nn] + beta C (m rows): basis times coefficients.
+    void gemm(int m, int nn, int k, double alpha, const double2* A, int lda, const double2* B, int ldb, double beta,
+              double2* C, int ldc) {
         if (m <= 0 || nn <= 0) return;
-        if (ta == rocblas_operation_none && tb == rocblas_operation_none && k > 0 && alpha.imag() == 0.0 &&
-            beta.imag() == 0.0) {
-            // Basis times coefficients: the library's own MFMA kernel.
-            int jb = 1, ntiles = 1;
-            bp_tiles(nn, &jb, &ntiles);
-            const int wx = m <= 8192 ? 2 : 4;  // 32-row tiles where 64-row ones would not fill the CUs
-            hipLaunchKernelGGL((wx == 4 ? gemm_fn<4>(jb) : gemm_fn<2>(jb)),
-                               dim3((unsigned)((m + 16 * wx - 1) / (16 * wx)), (unsigned)ntiles), dim3(64u * wx), 0, s, A, lda,
-                               B, ldb, C, ldc, m, k, nn, alpha.real(), beta.real());
-            DZ_HIP(hipGetLastError());
-            return;
-        }
-        DZ_BLAS(rocblas_zgemm(w.blas, ta, tb, m, nn, k, &alpha, reinterpret_cast<const zc*>(A), lda,
-                              reinterpret_cast<const zc*>(B), ldb, &beta, reinterpret_cast<zc*>(C), ldc));
+        DZ_REQUIRE(k > 0, DZHIP_ERR_STATE, "basis product over no columns");
+        int jb = 1, ntiles = 1;
+        bp_tiles(nn, &jb, &ntiles);
+        const int wx = m <= 8192 ? 2 : 4;  // 32-row tiles where 64-row ones would not fill the CUs
+        hipLaunchKernelGGL((wx == 4 ? gemm_fn<4>(jb) : gemm_fn<2>(jb)),
+                           dim3((unsigned)((m + 16 * wx - 1) / (16 * wx)), (unsigned)ntiles), dim3(64u * wx), 0, s, A, lda, B,
+                           ldb, C, ldc, m, k, nn, alpha, beta);
+        DZ_HIP(hipGetLastError());
     }
 
     // Squared column norms into out (device or pinned memory).
@@ -899,8 +893,7 @@ struct Solver {
         for (int pass = 0; pass < 2 && m > 0; ++pass) {
             // S = V^H Q ; Q -= V S
             gram(V(), m, Q, a, w.S.as<double2>(), max_sub);
-            gemm(rocblas_operation_none, rocblas_operation_none, ldn, a, m, zc(-1.0, 0.0), V(), ldn,
-                 w.S.as<double2>(), max_sub, zc(1.0, 0.0), Q, ldn);
+            gemm(ldn, a, m, -1.0, V(), ldn, w.S.as<double2>(), max_sub, 1.0, Q, ldn);
         }
         col_norms2(Q, a, w.norms.as<double>());
         hipLaunchKernelGGL(k_keep_cols, dim3(1), dim3(256), 0, s, w.norms0.as<double>(), w.norms.as<double>(), a,
@@ -966,7 +959,6 @@ struct Solver {
         gram(Q, k, Q, k, w.S.as<double2>(), k);
         potrf_upper(k);
         DZ_HIP(hipStreamSynchronize(s));
-        const zc one(1.0, 0.0), zero(0.0, 0.0);
         if (w.host_info[1]) {
             trsm(Q, k);
             return k;
@@ -981,8 +973,7 @@ struct Solver {
         while (first < k && !(lam[first] > thr)) ++first;
         const int kk = k - first;
         if (kk == 0) return 0;
-        gemm(rocblas_operation_none, rocblas_operation_none, ldn, kk, k, one, Q, ldn,
-             w.G.as<double2>() + (size_t)first * k, k, zero, w.HQ.as<double2>(), ldn);
+        gemm(ldn, kk, k, 1.0, Q, ldn, w.G.as<double2>() + (size_t)first * k, k, 0.0, w.HQ.as<double2>(), ldn);
         std::vector<int> idx(kk);
         std::vector<double> scl(kk);
         for (int j = 0; j < kk; ++j) {
@@ -1096,10 +1087,8 @@ struct Solver {
 
     void ritz(int m) {
         const int ldn = (int)n;
-        gemm(rocblas_operation_none, rocblas_operation_none, ldn, nb, m, zc(1.0, 0.0), V(), ldn, w.Tw.as<double2>(),
-             max_sub, zc(0.0, 0.0), w.X.as<double2>(), ldn);
-        gemm(rocblas_operation_none, rocblas_operation_none, ldn, nb, m, zc(1.0, 0.0), W(), ldn, w.Tw.as<double2>(),
-             max_sub, zc(0.0, 0.0), w.HX.as<double2>(), ldn);
+        gemm(ldn, nb, m, 1.0, V(), ldn, w.Tw.as<double2>(), max_sub, 0.0, w.X.as<double2>(), ldn);
+        gemm(ldn, nb, m, 1.0, W(), ldn, w.Tw.as<double2>(), max_sub, 0.0, w.HX.as<double2>(), ldn);
     }
 
     // Basis <- [X, Qnew] (already orthonormal), W <- [HX, HQnew], T rebuilt.
