@@ -19,8 +19,8 @@ namespace {
 constexpr unsigned kSpinLimit = 1u << 22;  // polls of one exchange (under a microsecond each) before giving up
 // The same for a tridiagonalisation admitted by the gate: its grid may find the device short
 // of CUs for a long time while other streams' kernels keep taking them, and it is then repeated as
-// a cooperative launch (heev_lowest_shared).  Si-64 concurrent-k SCF, mixed arm to 1e-6 Ha: 9.16 s
-// at 2^16 polls (frequent repeats), 8.60 s at 2^19, 10.21 s with cooperative launches only.
+// a cooperative launch (heev_lowest_shared).  Si-64 concurrent-k SCF, mixed arm to 1e-6 Ha: 5.7 s and no
+// repeat at 2^16 polls and at 2^19; 5.7 s with cooperative launches only.
 constexpr unsigned kSpinLimitShared = 1u << 19;
 
 // One DPP row rotation of a double (both halves moved by the same row_ror:N control).
@@ -479,9 +479,11 @@ __device__ __forceinline__ int sturm_count(const double2* de, int m, double x, d
 // Eigenvalue blockIdx.x (ascending) of T by multisection: each round the workgroup's 256 lanes count
 // at 256 interior points of [lo, hi] and keep the sub-interval that holds the eigenvalue; seven
 // rounds reach the last bits, where 64 points took nine.  The FP64 issue rate bounds it, one
-// wavefront per SIMD.  Also writes the Gershgorin scale of T to scal[0] (block 0).  nev = 160, one
-// wavefront per eigenvalue, one recurrence and divisions before: m = 164 / 648 113 -> 65 us,
-// 418 -> 228 us, the reflectors' compact form (11 and 30 us before) included.
+// wavefront per SIMD (the registers of compact_reflectors, which shares the launch).  Also writes the
+// Gershgorin scale of T to scal[0] (block 0).  nev = 160, one wavefront per eigenvalue, one recurrence and
+// divisions before: m = 164 / 648 113 -> 65 us, 418 -> 228 us, the reflectors' compact form (11 and 30 us
+// before) included.  More eigenvalues than CUs take turns; whole calls for all of them: m = 648 7,276 ->
+// 3,596 us, m = 1,000 14,219 -> 8,971 us.
 __device__ __forceinline__ void stebz(const double* __restrict__ d_in, const double* __restrict__ e_in, int m,
                                       double* __restrict__ w, double* __restrict__ scal, const int* __restrict__ err,
                                       double2* de) {
@@ -1084,7 +1086,10 @@ __global__ __launch_bounds__(64 * NW, 1) void k_apply_q(const double2* __restric
     }
 }
 
-// The instance and its wavefronts; above 768 rows eight wavefronts hold what four have no registers for.
+// The instance and its wavefronts.  Above 768 rows two blocks' V and W take all registers of eight
+// wavefronts, which spill 94 of them; four wavefronts would hold twice as much each.  Whole calls there
+// against one wavefront per eigenvector and one reflector at a time: m = 1,000, 160 vectors 11,829 -> 5,914
+// us, all 14,219 -> 8,971 us.
 const void* apply_q_kernel(int m, int* waves) {
     *waves = m <= 768 ? 4 : 8;
     if (m <= 256) return (const void*)k_apply_q<1, 4>;
