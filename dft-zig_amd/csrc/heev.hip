@@ -673,33 +673,29 @@ __device__ __forceinline__ double divergent(double v) {
     asm volatile("" : "+v"(v));
     return v;
 }
-__global__ __launch_bounds__(64) void k_stein(const double* __restrict__ d_in, const double* __restrict__ e_in, int m,
-                                              int nev, const double* __restrict__ w, const double* __restrict__ scal,
-                                              double* __restrict__ Z, int ldz) {
-    extern __shared__ double sh[];
-    const int k = (int)blockIdx.x, lane = (int)threadIdx.x;
-    if (k >= nev) return;
-    constexpr int NB = kSteinBlock;
-    const int mp = stein_rows(m), ma = mp + NB;      // rows computed; rows the loads ahead may touch
-    double2* de = reinterpret_cast<double2*>(sh);    // d, e
-    double2* lp = de + ma;                           // multiplier, 1 where rows r and r + 1 are exchanged
-    double2* uu = lp + ma;                           // 1 / U[r][r], U[r][r + 1]
-    double* u2 = reinterpret_cast<double*>(uu + ma);  // U[r][r + 2]
-    double* x = u2 + ma;
-    const double lam = w[k];
-    for (int r = lane; r < ma; r += 64) {
-        de[r] = make_double2(r < m ? d_in[r] : lam + 1.0, r + 1 < m ? e_in[r] : 0.0);
-        // Seeded start (splitmix64 of eigenvalue and row).
-        unsigned long long h = 0x9E3779B97F4A7C15ull * (unsigned long long)(k + 1) + (unsigned long long)r;
-        h = (h ^ (h >> 30)) * 0xBF58476D1CE4E5B9ull;
-        h = (h ^ (h >> 27)) * 0x94D049BB133111EBull;
-        h ^= h >> 31;
-        x[r] = r < m ? (double)(h >> 11) * (1.0 / 9007199254740992.0) - 0.5 : 0.0;
+struct Stein {
+    int m, mp;     // rows; rows computed
+    double2* de;   // d, e
+    double2* lp;   // multiplier, 1 where rows r and r + 1 are exchanged
+    double2* uu;   // 1 / U[r][r], U[r][r + 1]
+    double* u2;    // U[r][r + 2]
+    double* x;
+    int ma;        // rows the loads ahead may touch
+
+    __device__ __forceinline__ Stein(double* sh, int rows) : m(rows), mp(stein_rows(rows)) {
+        ma = mp + kSteinBlock;
+        de = reinterpret_cast<double2*>(sh);
+        lp = de + ma;
+        uu = lp + ma;
+        u2 = reinterpret_cast<double*>(uu + ma);
+        x = u2 + ma;
     }
-    __syncthreads();
-    const double bnorm = fmax(scal[0], 1e-300);
-    const double pert = 2.220446049250313e-16 * bnorm + 1e-300;
-    {
+    __device__ __forceinline__ void load(const double* __restrict__ d_in, const double* __restrict__ e_in, double lam, int r) const {
+        de[r] = make_double2(r < m ? d_in[r] : lam + 1.0, r + 1 < m ? e_in[r] : 0.0);
+    }
+    // T - lam = P L U, pivots raised to pert.
+    __device__ __forceinline__ void factor(double lam, double pert) const {
+        constexpr int NB = kSteinBlock;
         // Row r: (ca, cb); row r + 1 starts with c = e_r.
         double ca = divergent(de[0].x - lam), cb = divergent(de[0].y), c = cb;
         double2 nx[NB];
@@ -729,8 +725,9 @@ __global__ __launch_bounds__(64) void k_stein(const double* __restrict__ d_in, c
             }
         }
     }
-    __syncthreads();
-    for (int it = 0; it < 3; ++it) {
+    // x <- (T - lam)^-1 x.
+    __device__ __forceinline__ void solve() const {
+        constexpr int NB = kSteinBlock;
         // P L y = x, in place.
         double xr = divergent(x[0]);
         double2 nl[NB];
@@ -766,7 +763,7 @@ __global__ __launch_bounds__(64) void k_stein(const double* __restrict__ d_in, c
         double z0 = 0.0, z1 = 0.0;
         double2 nu[NB];
         double n2[NB];
-        auto load = [&](int top) {
+        auto ahead = [&](int top) {
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
                 nu[i] = uu[top - i];
@@ -774,7 +771,7 @@ __global__ __launch_bounds__(64) void k_stein(const double* __restrict__ d_in, c
                 nx[i] = x[top - i];
             }
         };
-        load(mp - 1);
+        ahead(mp - 1);
         for (int r0 = mp - 1; r0 >= 0; r0 -= NB) {
             double2 u[NB];
             double v2[NB], xi[NB];
@@ -784,7 +781,7 @@ __global__ __launch_bounds__(64) void k_stein(const double* __restrict__ d_in, c
                 v2[i] = n2[i];
                 xi[i] = nx[i];
             }
-            load(max(r0 - NB, NB - 1));
+            ahead(max(r0 - NB, NB - 1));
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
                 const double z = (xi[i] - v2[i] * z1 - u[i].y * z0) * u[i].x;
@@ -793,8 +790,9 @@ __global__ __launch_bounds__(64) void k_stein(const double* __restrict__ d_in, c
                 z0 = z;
             }
         }
-        __syncthreads();
-        // Scale by the largest entry (the solve amplifies by up to 1 / pert), then normalise.
+    }
+    // x / |x| (one wavefront): scaled by the largest entry first (a solve amplifies by up to 1 / pert).
+    __device__ __forceinline__ void normalise(int lane) const {
         double mx = 0.0;
         for (int r = lane; r < m; r += 64) mx = fmax(mx, fabs(x[r]));
 #pragma unroll
@@ -808,17 +806,51 @@ __global__ __launch_bounds__(64) void k_stein(const double* __restrict__ d_in, c
         s2 = wave_sum(s2);
         const double sc = inv_mx / sqrt(fmax(s2, 1e-300));
         for (int r = lane; r < m; r += 64) x[r] *= sc;
+    }
+};
+__device__ __forceinline__ double stein_pert(double bnorm) { return 2.220446049250313e-16 * fmax(bnorm, 1e-300) + 1e-300; }
+
+__global__ __launch_bounds__(64) void k_stein(const double* __restrict__ d_in, const double* __restrict__ e_in, int m,
+                                              int nev, const double* __restrict__ w, const double* __restrict__ scal,
+                                              double* __restrict__ Z, int ldz) {
+    extern __shared__ double sh[];
+    const int k = (int)blockIdx.x, lane = (int)threadIdx.x;
+    if (k >= nev) return;
+    const Stein t(sh, m);
+    const double lam = w[k];
+    for (int r = lane; r < t.ma; r += 64) {
+        t.load(d_in, e_in, lam, r);
+        // Seeded start (splitmix64 of eigenvalue and row).
+        unsigned long long h = 0x9E3779B97F4A7C15ull * (unsigned long long)(k + 1) + (unsigned long long)r;
+        h = (h ^ (h >> 30)) * 0xBF58476D1CE4E5B9ull;
+        h = (h ^ (h >> 27)) * 0x94D049BB133111EBull;
+        h ^= h >> 31;
+        t.x[r] = r < m ? (double)(h >> 11) * (1.0 / 9007199254740992.0) - 0.5 : 0.0;
+    }
+    __syncthreads();
+    t.factor(lam, stein_pert(scal[0]));
+    __syncthreads();
+    for (int it = 0; it < 3; ++it) {
+        t.solve();
+        __syncthreads();
+        t.normalise(lane);
         __syncthreads();
     }
-    for (int r = lane; r < m; r += 64) Z[(size_t)k * ldz + r] = x[r];
+    for (int r = lane; r < m; r += 64) Z[(size_t)k * ldz + r] = t.x[r];
 }
 
 // Members of each cluster (consecutive eigenvalues closer than cluster_tol), in order, made
 // orthonormal against the cluster's earlier members by two passes of classical Gram-Schmidt (one
 // workgroup per cluster; the first member leads).  Inverse iteration gives each member a vector in
-// the cluster's invariant subspace, so the orthonormal result spans the same subspace.
-__global__ __launch_bounds__(256) void k_stein_cluster(const double* __restrict__ w, const double* __restrict__ scal,
+// the cluster's invariant subspace, so the orthonormal result spans the same subspace.  Where the members
+// of a split T (equal blocks) came out nearly parallel, what a projection leaves has lost as many digits as
+// it is short; below kSteinLeft of the vector another solve (by wavefront 0) brings them back, with the
+// earlier members out of its start.
+constexpr double kSteinLeft = 0.05;
+__global__ __launch_bounds__(256) void k_stein_cluster(const double* __restrict__ d_in, const double* __restrict__ e_in,
+                                                       const double* __restrict__ w, const double* __restrict__ scal,
                                                        int nev, int m, double* __restrict__ Z, int ldz) {
+    extern __shared__ double sh[];
     __shared__ double dots[kHeevMaxM];
     __shared__ double red[4];
     const int i = (int)blockIdx.x;
@@ -828,34 +860,54 @@ __global__ __launch_bounds__(256) void k_stein_cluster(const double* __restrict_
     int last = i;
     while (last + 1 < nev && w[last + 1] - w[last] <= tau_c) ++last;
     if (last == i) return;
+    const Stein s(sh, m);
     const int t = (int)threadIdx.x, wv = t >> 6, lane = t & 63;
     for (int k = i + 1; k <= last; ++k) {
         double* x = Z + (size_t)k * ldz;
-        for (int pass = 0; pass < 2; ++pass) {
-            for (int p = i + wv; p < k; p += 4) {
-                const double* zp = Z + (size_t)p * ldz;
-                double sdot = 0.0;
-                for (int r = lane; r < m; r += 64) sdot += zp[r] * x[r];
-                sdot = wave_sum(sdot);
-                if (lane == 0) dots[p - i] = sdot;
+        for (int attempt = 0;; ++attempt) {
+            for (int pass = 0; pass < 2; ++pass) {
+                for (int p = i + wv; p < k; p += 4) {
+                    const double* zp = Z + (size_t)p * ldz;
+                    double sdot = 0.0;
+                    for (int r = lane; r < m; r += 64) sdot += zp[r] * x[r];
+                    sdot = wave_sum(sdot);
+                    if (lane == 0) dots[p - i] = sdot;
+                }
+                __syncthreads();
+                for (int r = t; r < m; r += 256) {
+                    double acc = x[r];
+                    for (int p = i; p < k; ++p) acc -= dots[p - i] * Z[(size_t)p * ldz + r];
+                    x[r] = acc;
+                }
+                __syncthreads();
+            }
+            double s2 = 0.0;
+            for (int r = t; r < m; r += 256) s2 += x[r] * x[r];
+            s2 = wave_sum(s2);
+            if (lane == 0) red[wv] = s2;
+            __syncthreads();
+            const double nrm = sqrt(red[0] + red[1] + red[2] + red[3]);
+            const double inv = nrm > 0.0 ? 1.0 / nrm : 0.0;
+            for (int r = t; r < m; r += 256) x[r] *= inv;
+            __syncthreads();
+            if (nrm >= kSteinLeft || attempt == 2) break;
+            const double lam = w[k];
+            for (int r = t; r < s.ma; r += 256) {
+                s.load(d_in, e_in, lam, r);
+                s.x[r] = r < m ? x[r] : 0.0;
             }
             __syncthreads();
-            for (int r = t; r < m; r += 256) {
-                double acc = x[r];
-                for (int p = i; p < k; ++p) acc -= dots[p - i] * Z[(size_t)p * ldz + r];
-                x[r] = acc;
+            if (wv == 0) {
+                s.factor(lam, stein_pert(scal[0]));
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                s.solve();
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                s.normalise(lane);
             }
+            __syncthreads();
+            for (int r = t; r < m; r += 256) x[r] = s.x[r];
             __syncthreads();
         }
-        double s2 = 0.0;
-        for (int r = t; r < m; r += 256) s2 += x[r] * x[r];
-        s2 = wave_sum(s2);
-        if (lane == 0) red[wv] = s2;
-        __syncthreads();
-        const double nrm = sqrt(red[0] + red[1] + red[2] + red[3]);
-        const double inv = nrm > 0.0 ? 1.0 / nrm : 0.0;
-        for (int r = t; r < m; r += 256) x[r] *= inv;
-        __syncthreads();
     }
 }
 
@@ -1130,6 +1182,7 @@ CoopInfo coop_info(int dev) {
         DZ_REQUIRE(coop != 0, DZHIP_ERR_HIP, "device does not support cooperative launches");
         for (const TrdKernel& k : kTrdKernels) set_max_dynamic_lds(k.fn, k.lds());
         set_max_dynamic_lds((const void*)k_stein, stein_lds_bytes(kHeevMaxM));
+        set_max_dynamic_lds((const void*)k_stein_cluster, stein_lds_bytes(kHeevMaxM));
         // Launch-shape override: at least so many trailing columns per workgroup (4, 8 or 16).
         if (const char* env = std::getenv("DZHIP_HEEV_COLS")) c.cols_per_group = std::max(0, std::atoi(env));
         c.groups = cus;
@@ -1249,7 +1302,8 @@ void run_eig(const HeevBufs& b, int m, int nev, double* w_dev, double2* Y, int l
     hipLaunchKernelGGL(k_stein, dim3((unsigned)nev), dim3(64), stein_lds_bytes(m), s, b.d, b.e, m, nev, w_dev, scal,
                        b.z, m);
     DZ_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_stein_cluster, dim3((unsigned)nev), dim3(256), 0, s, w_dev, scal, nev, m, b.z, m);
+    hipLaunchKernelGGL(k_stein_cluster, dim3((unsigned)nev), dim3(256), stein_lds_bytes(m), s, b.d, b.e, w_dev, scal, nev, m,
+                       b.z, m);
     DZ_HIP(hipGetLastError());
     double* zc = b.z;
     double* zn = b.zt;

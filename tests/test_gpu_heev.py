@@ -269,3 +269,13 @@ def test_heev_shared_launch_repeats_are_counted():
     for l in lines:
         print(*l, flush=True)
         assert float(l[1]) < 1e-12 and int(l[2]) == 1
+
+
+@pytest.mark.parametrize("copies,h", [(2, 20), (2, 65), (2, 130), (3, 20), (3, 65), (3, 130), (3, 200)])
+def test_heev_equal_blocks(ctx, copies, h):
+    """Equal diagonal blocks: T splits, and inverse iteration gives the members of a cluster nearly
+    parallel vectors for some of the pairs; bars as above."""
+    for seed in range(6):
+        rng = np.random.default_rng(8000 + seed)
+        g = rng.standard_normal((h, h)) + 1j * rng.standard_normal((h, h))
+        check(ctx, np.kron(np.eye(copies), 0.5 * (g + g.conj().T)), 3 * copies * h // 4)
