@@ -206,11 +206,14 @@ struct Trd {
             const double ir = rsqrt3(n2), nrm = n2 * ir;
             const double ib = alpha.x >= 0.0 ? -ir : ir;
             beta = alpha.x >= 0.0 ? -nrm : nrm;
-            // tau = 1 - alpha / beta and 1 / (alpha - beta) = -1 / (beta tau): |tau|^2 is between 1 and 4, where
-            // |alpha - beta|^2 has no reciprocal below a norm of 1e-154 (and comes an operation later).
-            tau = make_double2(fma(fabs(alpha.x), ir, 1.0), -alpha.y * ib);
-            const double id = recip3(tau.x * tau.x + tau.y * tau.y);
-            scale = make_double2(-(tau.x * ib) * id, tau.y * ib * id);
+            tau = make_double2((beta - alpha.x) * ib, -alpha.y * ib);
+            const double2 den = make_double2(alpha.x - beta, alpha.y);
+            const double dd = den.x * den.x + den.y * den.y;
+            // The reciprocal of the mantissa, its exponent with the numerator: 1 / dd itself leaves the range
+            // below a norm of 1e-154.
+            const int ex = -__builtin_amdgcn_frexp_exp(dd);
+            const double id = recip3(__builtin_amdgcn_frexp_mant(dd));
+            scale = make_double2(__builtin_amdgcn_ldexp(den.x, ex) * id, -__builtin_amdgcn_ldexp(den.y, ex) * id);
         }
 #pragma unroll
         for (int c = 0; c < CW; ++c) {
