@@ -36,12 +36,11 @@ constexpr int kHeevNoAllocMaxM = 256;
 // Share of the device's tridiagonalisation gate held by one eigensolver call.  Its exchange needs
 // all of the grid's workgroups resident at once.  Workgroups are dealt to the XCDs round robin, so
 // a grid of G groups needs at most ceil(G / XCDs) CUs on any XCD (one workgroup per CU at worst).
-// The gate admits grids only while their sum stays within the CUs of one XCD: of m / 4 workgroups, four
+// The gate admits grids only while their sum stays within the CUs of one XCD: of m / 4 workgroups, five
 // of m = 164 or two of m = 328 at a time, but one of m = 648.  (Two columns a wavefront would admit two of
 // those: eight threads' calls at m = 648 2,189 us each instead of 2,838, a call alone 3,718 instead of
-// 3,152, 300 vectors.)  Every other kernel
-// the library launches runs to completion without waiting on another workgroup, so an admitted
-// grid's missing workgroups are placed as those retire.  That can take long: with many streams
+// 3,152, 300 vectors.)  Every other kernel the library launches runs to completion without waiting on
+// another workgroup, so an admitted grid's missing workgroups are placed as those retire.  That can take long: with many streams
 // issuing kernels, smaller workgroups keep refilling the CUs a tridiagonalisation workgroup (one
 // wavefront per SIMD at the larger sizes) waits for.  An admitted grid therefore gives up after 2^19
 // polls (an eighth of the cooperative launch's limit) and heev_lowest_shared repeats the call
